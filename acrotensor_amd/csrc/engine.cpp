@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <map>
 
+#include "SliceTensor.hpp"
 #include "TensorEngine.hpp"
 
 namespace acro
@@ -285,6 +286,48 @@ bool TensorEngine::MatrixOpAsKernels(const RecordedMatrixOp &op, const std::vect
     return true;
 }
 
+namespace
+{
+Tensor *parentOf(Tensor *t)
+{
+    const SliceTensor *slice = dynamic_cast<const SliceTensor *>(t);
+    return slice != nullptr ? slice->GetParent() : nullptr;
+}
+
+// Whether two tensors share memory on either side (a slice is one contiguous range of its parent).
+bool sameMemory(const Tensor *a, const Tensor *b)
+{
+    if (a == b) return true;
+    auto overlap = [](const double *pa, size_t na, const double *pb, size_t nb) {
+        return pa != nullptr && pb != nullptr && pa < pb + nb && pb < pa + na;
+    };
+    return overlap(a->GetData(), a->GetSize(), b->GetData(), b->GetSize()) ||
+           overlap(a->GetDeviceData(), a->GetSize(), b->GetDeviceData(), b->GetSize());
+}
+
+// Takes the transient mark off tensors (and off the tensors they are slices of) until the end of its life.
+class NotTransient
+{
+  public:
+    void Add(Tensor *t)
+    {
+        for (; t != nullptr; t = parentOf(t))
+        {
+            if (!t->Tensor::IsTransient()) continue;  // the mark of this view itself
+            t->SetTransient(false);
+            Marked.push_back(t);
+        }
+    }
+    ~NotTransient()
+    {
+        for (Tensor *t : Marked) t->SetTransient(true);
+    }
+
+  private:
+    std::vector<Tensor *> Marked;
+};
+}  // namespace
+
 void TensorEngine::FinishCapture(std::string *implementation)
 {
     std::vector<DimensionedKernel *> kernels;
@@ -296,30 +339,28 @@ void TensorEngine::FinishCapture(std::string *implementation)
     std::vector<RecordedMatrixOp> ops;
     ops.swap(MKLMatrixOps);
 
-    std::vector<GatheredInput> gathered;  // results of recorded scatters that the kernels read through the maps
-    auto flush = [&]() {
-        if (MKLKernels.empty()) return;
-        KernelExecutor *executor = GetAddKernelExecutor();
-        executor->SetGatheredInputs(gathered);
-        if (implementation != nullptr)
-        {
-            *implementation += executor->GetImplementation(MKLOutputT, MKLInputT);
-        }
-        else
-        {
-            LastExecutor = executor;
-            executor->ExecuteMulti(MKLOutputT, MKLInputT);
-        }
-        ResetCapture();
+    // What the capture turns into, in program order: groups of kernels, each one launch, and operations that run on
+    // their own between them.
+    struct Part
+    {
+        std::vector<DimensionedKernel *> kernels;
+        std::vector<Tensor *> outputs;
+        std::vector<std::vector<Tensor *>> inputs;
+        std::vector<GatheredInput> gathered;   // results of recorded scatters that the kernels read through the maps
+        const RecordedMatrixOp *op = nullptr;  // set: this operation instead of kernels
     };
-    // A recorded scatter need not run when its result is transient, nothing else in the capture writes the result
-    // or the source, no kernel recorded before it reads the result, and a kernel recorded after it does.
+    std::vector<Part> parts(1);
+    std::vector<GatheredInput> gathered;
+    // A recorded scatter need not run when its result is transient, nothing else in the capture writes the memory of
+    // the result or of the source, no kernel recorded before it reads the result, and a kernel recorded after it does.
     auto readThroughMap = [&](const RecordedMatrixOp &op) {
-        if (!op.scatter_out->IsTransient() || op.scatter_out == op.scatter_in) return false;
+        if (!op.scatter_out->IsTransient()) return false;
+        Tensor *result = op.scatter_out, *source = op.scatter_in;
+        if (sameMemory(result, source)) return false;
         bool read_later = false;
         for (size_t k = 0; k < kernels.size(); ++k)
         {
-            if (outputs[k] == op.scatter_out || outputs[k] == op.scatter_in) return false;
+            if (sameMemory(outputs[k], result) || sameMemory(outputs[k], source)) return false;
             for (Tensor *t : inputs[k])
             {
                 if (t != op.scatter_out) continue;
@@ -332,43 +373,18 @@ void TensorEngine::FinishCapture(std::string *implementation)
             if (&other == &op) continue;
             for (Tensor *t : {other.inverse, other.determinant, other.matrices, other.scatter_out, other.scatter_in})
             {
-                if (t == op.scatter_out || (t == op.scatter_in && t != other.scatter_in && t != other.matrices)) return false;
+                if (t == nullptr) continue;
+                const bool reads = t == other.scatter_in || t == other.matrices;
+                if (sameMemory(t, result) || (!reads && sameMemory(t, source))) return false;
             }
         }
         return read_later;
     };
-    // A capture that a matrix operation splits into several launches keeps nothing on chip across them: for its
-    // duration no tensor counts as transient (a transient result of one launch may be an operand of the next).
-    struct KeepEverything
-    {
-        std::vector<Tensor *> marked;
-        void Add(Tensor *t)
-        {
-            if (t == nullptr || !t->IsTransient()) return;
-            t->SetTransient(false);
-            marked.push_back(t);
-        }
-        ~KeepEverything()
-        {
-            for (Tensor *t : marked) t->SetTransient(true);
-        }
-    } keep;
-    auto keepAll = [&]() {
-        for (size_t k = 0; k < kernels.size(); ++k)
-        {
-            keep.Add(outputs[k]);
-            for (Tensor *t : inputs[k]) keep.Add(t);
-        }
-        for (const auto &op : ops)
-        {
-            keep.Add(op.inverse);
-            keep.Add(op.determinant);
-            keep.Add(op.matrices);
-            keep.Add(op.scatter_in);
-            bool through_map = false;  // a result that is read through its map stays transient: it is never written
-            for (const auto &g : gathered) through_map = through_map || g.operand == op.scatter_out;
-            if (!through_map) keep.Add(op.scatter_out);
-        }
+    auto onItsOwn = [&](const RecordedMatrixOp &op) {
+        parts.back().gathered = gathered;
+        if (!parts.back().kernels.empty()) parts.emplace_back();
+        parts.back().op = &op;
+        parts.emplace_back();
     };
     size_t next_op = 0;
     for (size_t k = 0; k <= kernels.size(); ++k)
@@ -377,67 +393,117 @@ void TensorEngine::FinishCapture(std::string *implementation)
         {
             const RecordedMatrixOp &op = ops[next_op];
             if (op.sum_gather)
-            {
-                // never part of a fused launch (its rows cross workgroups): runs on its own, at its place
-                keepAll();
-                flush();
-                if (implementation != nullptr)
-                {
-                    *implementation += "// sum-gather: runs on its own\n";
-                    continue;
-                }
-                SwitchToComputeLocation(*op.scatter_out);
-                MoveToComputeLocation(*op.scatter_in);
-                MoveToComputeLocation(*op.map);
-                Ops->FlatIndexedSumGather(*op.scatter_out, *op.scatter_in, *op.map);
-                continue;
-            }
-            if (op.scatter_out != nullptr)
-            {
-                if (readThroughMap(op))
-                {
-                    gathered.push_back({op.scatter_out, op.scatter_in, op.map});
-                    continue;
-                }
-                keepAll();
-                flush();
-                if (implementation != nullptr)
-                {
-                    *implementation += "// scatter whose result is not transient, or not only read by the kernels after it: runs on its own\n";
-                    continue;
-                }
-                SwitchToComputeLocation(*op.scatter_out);
-                MoveToComputeLocation(*op.scatter_in);
-                MoveToComputeLocation(*op.map);
-                Ops->FlatIndexedScatter(*op.scatter_out, *op.scatter_in, *op.map);
-                continue;
-            }
-            if (MatrixOpAsKernels(op, kernels, outputs, inputs, MKLKernels, MKLOutputT, MKLInputT)) continue;
-            keepAll();
-            flush();
-            if (implementation != nullptr)
-            {
-                *implementation += "// batched matrix operation whose result no later kernel of the capture reads: runs on its own\n";
-                continue;
-            }
-            if (op.inverse != nullptr) SwitchToComputeLocation(*op.inverse);
-            if (op.determinant != nullptr) SwitchToComputeLocation(*op.determinant);
-            MoveToComputeLocation(*op.matrices);
-            if (op.inverse != nullptr && op.determinant != nullptr)
-                Ops->BatchMatrixInvDet(*op.inverse, *op.determinant, *op.matrices);
-            else if (op.inverse != nullptr)
-                Ops->BatchMatrixInverse(*op.inverse, *op.matrices);
-            else
-                Ops->BatchMatrixDet(*op.determinant, *op.matrices);
+                onItsOwn(op);  // never part of a fused launch: its rows cross workgroups
+            else if (op.scatter_out != nullptr && readThroughMap(op))
+                gathered.push_back({op.scatter_out, op.scatter_in, op.map});
+            else if (op.scatter_out != nullptr ||
+                     !MatrixOpAsKernels(op, kernels, outputs, inputs, parts.back().kernels, parts.back().outputs, parts.back().inputs))
+                onItsOwn(op);
         }
         if (k < kernels.size())
         {
-            MKLKernels.push_back(kernels[k]);
-            MKLOutputT.push_back(outputs[k]);
-            MKLInputT.push_back(inputs[k]);
+            parts.back().kernels.push_back(kernels[k]);
+            parts.back().outputs.push_back(outputs[k]);
+            parts.back().inputs.push_back(inputs[k]);
         }
     }
-    flush();
+    parts.back().gathered = gathered;
+    if (parts.back().kernels.empty() && parts.back().op == nullptr) parts.pop_back();
+
+    // Nothing stays on chip from one part to the next: a tensor that several parts touch does not count as transient
+    // for the duration of the capture (a transient result of one launch may be an operand of the next).  One that a
+    // single part touches stays scratch space of that launch: with a sum-gather recorded behind the p = 3 mass apply, all
+    // six intermediates used to be stored for its sake (mesh of 61 x 64 x 67 elements: mass apply 357 us with, 87 us
+    // without those stores).  Tensors are told apart by the memory they lie in, whatever views the calls were given.
+    NotTransient across;
+    if (parts.size() > 1)
+    {
+        struct Touch
+        {
+            Tensor *tensor;
+            size_t part;
+        };
+        std::vector<Touch> touches;
+        for (size_t p = 0; p < parts.size(); ++p)
+        {
+            auto touch = [&](Tensor *t) {
+                if (t != nullptr) touches.push_back({t, p});
+            };
+            for (size_t k = 0; k < parts[p].kernels.size(); ++k)
+            {
+                touch(parts[p].outputs[k]);
+                for (Tensor *t : parts[p].inputs[k]) touch(t);
+            }
+            for (const auto &g : parts[p].gathered) touch(g.source);
+            if (parts[p].op != nullptr)
+            {
+                const RecordedMatrixOp &op = *parts[p].op;
+                for (Tensor *t : {op.inverse, op.determinant, op.matrices, op.scatter_out, op.scatter_in}) touch(t);
+            }
+        }
+        std::vector<Tensor *> kept;  // decided on the marks as the caller left them
+        for (const Touch &t : touches)
+        {
+            if (!t.tensor->IsTransient()) continue;
+            for (const Touch &o : touches)
+            {
+                if (o.part == t.part || !sameMemory(o.tensor, t.tensor)) continue;
+                kept.push_back(t.tensor);
+                break;
+            }
+        }
+        for (Tensor *t : kept) across.Add(t);
+    }
+
+    for (Part &part : parts)
+    {
+        if (part.op == nullptr)
+        {
+            MKLKernels.swap(part.kernels);
+            KernelExecutor *executor = GetAddKernelExecutor();
+            executor->SetGatheredInputs(part.gathered);
+            if (implementation != nullptr)
+            {
+                *implementation += executor->GetImplementation(part.outputs, part.inputs);
+            }
+            else
+            {
+                LastExecutor = executor;
+                executor->ExecuteMulti(part.outputs, part.inputs);
+            }
+            ResetCapture();
+            continue;
+        }
+        const RecordedMatrixOp &op = *part.op;
+        if (implementation != nullptr)
+        {
+            *implementation += op.sum_gather ? "// sum-gather: runs on its own\n"
+                               : op.scatter_out != nullptr
+                                   ? "// scatter whose result is not transient, or not only read by the kernels after it: runs on its own\n"
+                                   : "// batched matrix operation whose result no later kernel of the capture reads: runs on its own\n";
+            continue;
+        }
+        if (op.scatter_out != nullptr)
+        {
+            SwitchToComputeLocation(*op.scatter_out);
+            MoveToComputeLocation(*op.scatter_in);
+            MoveToComputeLocation(*op.map);
+            if (op.sum_gather)
+                Ops->FlatIndexedSumGather(*op.scatter_out, *op.scatter_in, *op.map);
+            else
+                Ops->FlatIndexedScatter(*op.scatter_out, *op.scatter_in, *op.map);
+            continue;
+        }
+        if (op.inverse != nullptr) SwitchToComputeLocation(*op.inverse);
+        if (op.determinant != nullptr) SwitchToComputeLocation(*op.determinant);
+        MoveToComputeLocation(*op.matrices);
+        if (op.inverse != nullptr && op.determinant != nullptr)
+            Ops->BatchMatrixInvDet(*op.inverse, *op.determinant, *op.matrices);
+        else if (op.inverse != nullptr)
+            Ops->BatchMatrixInverse(*op.inverse, *op.matrices);
+        else
+            Ops->BatchMatrixDet(*op.determinant, *op.matrices);
+    }
 }
 
 std::string TensorEngine::GetImplementation(const std::string &kernel_str, Tensor *output,

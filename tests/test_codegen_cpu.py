@@ -799,3 +799,42 @@ def test_operands_that_carry_a_contraction_index_alone_are_summed_first(TE):
     # a contraction shared by lanes is numbered as the terms lie in the streaming operand
     src = TE.GetImplementation("A_e = B_i_j C_e_j_i", at.Tensor(4096), at.Tensor(20, 8), at.Tensor(4096, 8, 20))
     assert "contraction shared by" in src and "lanes()=16" in src
+
+
+def test_scratch_tensors_of_one_launch_stay_on_chip_when_a_sum_gather_follows(TE):
+    """A recorded sum-gather splits the capture; only what both sides of the split touch has to reach device memory."""
+    dofs, nodes = workloads.hex_mesh_dof_map(3, 3, 3, 3)
+    M, L, y = at.IndexMapping(nodes, dofs.size), at.Tensor(nodes), at.Tensor(nodes)
+    M.map[:] = dofs.ravel()
+    wl = workloads.config4(E=27)
+
+    def source(prepare, after=None):
+        tensors = workloads.bind_to_engine(wl, at, transient=True)
+        prepare(tensors)
+        TE.BeginMultiKernelLaunch()
+        TE.FlatIndexedScatter(tensors["X"], L, M)
+        for k, out, ins in wl.kernels:
+            TE(k, tensors[out], *[tensors[n] for n in ins])
+        TE.FlatIndexedSumGather(y, tensors["Y"], M)
+        if after:
+            TE("W_e_q_r_s = A_e_q_r_s D_e_q_r_s", tensors["T3"], tensors[after], tensors["D"])
+        return TE.EndMultiKernelLaunchGetImplementation()
+
+    src = source(lambda t: t["X"].SetTransient(True))
+    assert "X<-gathered" in src and "T1->lds\n" in src and "U->lds\n" in src and "Y->global" in src
+    # a transient result that the sum-gather reads, and one that a kernel after it reads, are stored
+    src = source(lambda t: t["Y"].SetTransient(True))
+    assert "Y->global" in src and "T1->lds\n" in src
+    src = source(lambda t: None, "U")
+    assert "U->lds+global" in src and "T1->lds\n" in src
+
+    # ... also when the two sides see the memory through different tensors, and the mark is a parent's
+    def alias(t):
+        t["parent"] = at.Tensor(2, *t["U"].dims)
+        t["parent"].SetTransient(True)
+        t["U"], t["again"], t["other"] = at.SliceTensor(t["parent"], 1), at.SliceTensor(t["parent"], 1), at.SliceTensor(t["parent"], 0)
+
+    src = source(alias, "again")
+    assert "U->lds+global" in src and "T1->lds\n" in src
+    src = source(alias, "other")
+    assert "U->lds\n" in src

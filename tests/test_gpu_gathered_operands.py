@@ -194,3 +194,41 @@ def test_sum_gather_recorded_in_a_capture_runs_at_its_place(at, engine, checker)
         expected = np.zeros(nodes)
         np.add.at(expected, dofs.ravel(), Y.ravel())
         assert rel_err(Lout.data, expected) <= 1e-12, transient_x
+
+
+@pytest.mark.parametrize("after", [None, "U", "T2"])
+def test_mesh_operator_in_one_capture_with_the_sum_gather(at, engine, checker, after):
+    """Scatter, mass apply, sum-gather and a kernel behind it that reads an intermediate: scratch tensors of the first
+    launch stay on chip, the one the last kernel reads reaches device memory (NaN there before the call)."""
+    dofs, nodes, M = mesh(at, 4, 3)
+    wl = workloads.config4(E=dofs.shape[0])
+    tensors = workloads.bind_to_engine(wl, at, transient=True)
+    tensors["X"].SetTransient(True)
+    rng = np.random.default_rng(31)
+    nodal = rng.uniform(-1, 1, nodes)
+    L, y = to_tensor(at, nodal), at.Tensor(nodes)
+    values = {n: wl.arrays[n] for n in wl.inputs}
+    values["X"] = nodal[dofs.ravel()].reshape(dofs.shape)
+    for name in wl.transient:
+        tensors[name].Set(np.nan)
+        tensors[name].MoveToGPU()
+    out = at.Tensor(*tensors[after].dims) if after else None
+    engine.BeginMultiKernelLaunch()
+    engine.FlatIndexedScatter(tensors["X"], L, M)
+    for k, name, ins in wl.kernels:
+        engine(k, tensors[name], *[tensors[i] for i in ins])
+    engine.FlatIndexedSumGather(y, tensors["Y"], M)
+    if after:
+        engine("W_a_b_c_d = %s_a_b_c_d" % after, out, tensors[after])
+    engine.EndMultiKernelLaunch()
+    expected = {}
+    for k, name, ins in wl.kernels:
+        expected[name] = np.zeros(tensors[name].dims)
+        checker.contract(k, expected[name], *[expected[i] if i in expected else values[i] for i in ins])
+    total = np.zeros(nodes)
+    np.add.at(total, dofs.ravel(), expected["Y"].ravel())
+    y.MoveFromGPU()
+    assert rel_err(y.data, total) <= TOL
+    if after:
+        out.MoveFromGPU()
+        assert rel_err(out.data, expected[after]) <= TOL
