@@ -154,8 +154,28 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
         }
         loadsPerSlice += n;
     }
-    const bool pencil = outputsFastest && (O <= 16 || (O <= 64 && 2 * loadsPerSlice <= O)) && envInt("ACRO_HIP_RED_PENCIL") >= 0;
     const int NTr = kReductionLanes;
+    // The big operand is the contracted indices followed by all output indices ("S_i_j = A_n_i_j B_n"): one stream of
+    // Nc x O doubles in which the output entry repeats with period O.  A lane takes two neighbouring doubles, so that a
+    // wavefront's load instruction is 1 KB of whole lines, and a workgroup a window of 2 flatLanes doubles that is a whole
+    // number of slices, so that a lane keeps its two output entries.  Bound by HBM.  Against one lane per (slice, output)
+    // and, up to 16 outputs, a lane per slice (pencil), whole call, from HBM: 2 749 324 slices of 4 x 5 98.4 -> 70.0 us,
+    // 2 000 001 of 6 x 6 122 -> 89 us, 500 001 of 3 x 5
+    // 14.4 -> 13.5 us.  Up to nine outputs a pencil is as fast on operands that the memory-side cache can hold (2^20 of
+    // 3 x 3 16.1 / 16.0 us, 10^6 of 2 x 2 10.0 / 10.2) and behind beyond (1 705 447 of 2 x 4, 109 MB, 24.6 -> 23.1 us,
+    // 4 000 001 of 2 x 3 43.9 -> 40.0), hence the line at 96 MB.
+    // Four windows are requested before they are added (8: slower), 512 workgroups (256, 1 024, 2 048: slower), fewer for
+    // a stream of less than 8 windows each (4: 20 001 slices of 6 x 8 9.2 us, 8: 7.7, the partials being half as many).
+    const long period = O % 2 == 0 ? O / 2 : O;   // lanes after which the output entries repeat
+    const long flatLanes = NTr / period * period;
+    const bool pencilForm = outputsFastest && (O <= 16 || (O <= 64 && 2 * loadsPerSlice <= O)) && envInt("ACRO_HIP_RED_PENCIL") >= 0;
+    bool flat = outputsFastest && O >= 2 && flatLanes >= 192 && !big->repeated && big->size == Nc * O &&
+                big->idx.size() >= s.contr.size() && envInt("ACRO_HIP_RED_FLAT") >= 0 &&
+                (!pencilForm || O > 9 || big->size >= (12L << 20) || envInt("ACRO_HIP_RED_FLAT") > 0);
+    for (size_t d = 0; flat && d < s.contr.size(); ++d) flat = has(s.contr, big->idx[d]);
+    constexpr int kFlatWindows = 4;               // windows of a workgroup in flight
+    const long flatSlices = 2 * flatLanes / O;    // slices per window
+    const bool pencil = pencilForm && !flat;
     // The big operand streams through once, its values going into one term each, read by lanes that follow it through
     // memory in whole 128-byte lines per load instruction: requested with the non-temporal hint (64 column sums over 2^20
     // rows 75 -> 81 % of the HBM peak, 64 row sums 78 -> 84 %, 32 x 32 sums of element matrices 71 -> 74 %).  Not the
@@ -167,16 +187,16 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     // workgroup only NTr / O lanes would walk along a row (32-byte pieces of 64 different rows per load
     // instruction).  Instead a workgroup takes four outputs, 64 adjacent lanes each, and the workgroups are dealt
     // out over groups of outputs as well as over the contraction range.
-    const bool byRows = !pencil && !outputsFastest && O > 4 && NTr / O < 64 && (envInt("ACRO_HIP_ONE_PASS") <= 0 || O > NTr) &&
-                        envInt("ACRO_HIP_RED_ROWS") >= 0;
+    const bool forced = envInt("ACRO_HIP_ONE_PASS") > 0;   // (whatever the size)
+    const bool byRows = !pencil && !outputsFastest && O > 4 && NTr / O < 64 && (!forced || O > NTr) && envInt("ACRO_HIP_RED_ROWS") >= 0;
     // More than 256 outputs that are the fastest dimension of the big operand ("S_i_j = A_e_i_j" with 16 x 16 outputs
     // and more): a workgroup takes 256 neighbouring outputs, a lane each, and a share of the contraction range; the
     // lanes of a wavefront read 512 consecutive bytes per term.  The finishing kernel has a workgroup per 256 outputs.
-    const bool wide = !pencil && !byRows && O > NTr;   // (up to 256 outputs: a lane per output in every workgroup, below)
+    const bool wide = !pencil && !flat && !byRows && O > NTr;   // (up to 256 outputs: a lane per output in every workgroup, below)
     // More outputs than one workgroup's lanes, whichever way they were summed: the finishing kernel has a workgroup per
     // 256 outputs too.
     const bool wideFinish = wide || O > 1024;
-    const long Sn = pencil ? NTr : (byRows ? 64 : (wide ? 1 : NTr / O));  // contraction slices per workgroup and step
+    const long Sn = flat ? flatSlices : (pencil ? NTr : (byRows ? 64 : (wide ? 1 : NTr / O)));  // contraction slices per workgroup and step
     // (Two neighbouring outputs per lane, read as one 16-byte piece, measured slower: "S_i_j = A_e_i_j" with 32 x 32
     // outputs over 131 072 entries 70 -> 60 % of the HBM peak.)
     const long Ow = NTr / Sn, Go = (byRows || wide) ? (O + Ow - 1) / Ow : 1;  // outputs per workgroup, groups of outputs
@@ -186,8 +206,18 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     // 214 / 263 us with the loop unrolled 2 / 4 times).  One lane per (slice, output entry): 8 bytes per lane
     // and load, so up to 512 workgroups and four loads in flight per lane (also swept: 256 - 8 192 workgroups,
     // unroll 1 - 8).
-    const long G = (byRows || (wide && Go > 1)) ? std::min<long>(std::max<long>(1, 1024 / Go), std::max<long>(1, Nc / (Sn * 16)))
-                                                : std::min<long>(pencil ? envInt("ACRO_HIP_RED_GROUPS", 256) : 512, std::max<long>(1, Nc / (Sn * (pencil ? 4 : 16))));
+    long G = (byRows || (wide && Go > 1)) ? std::min<long>(std::max<long>(1, 1024 / Go), std::max<long>(1, Nc / (Sn * 16)))
+                                          : std::min<long>(pencil ? envInt("ACRO_HIP_RED_GROUPS", 256) : 512,
+                                                           std::max<long>(1, Nc / (flat && O <= 64 ? Sn * 2 * kFlatWindows : pencil ? Sn * 4 : (flat ? NTr / O : Sn) * 16)));
+    // A sum that a few workgroups read within a microsecond or two is over before a second launch is issued: the
+    // workgroup that finishes last adds the partials in the same launch (see below), and the range is shared out over
+    // at most onePassGroups workgroups for it.  Larger sums keep the second kernel: every arrival at the counter writes
+    // back the L2 of its XCD (256 workgroups: 18.4 us in one launch against 16.3 us in two).
+    // (4 096 slices of 3 x 3 7.6 -> 4.8 us per call, 37 529 of 2 x 3 7.5 -> 5.4, 7 373 of 6 x 4 7.5 -> 5.2; at most 16 or 64
+    // workgroups the same within 0.3 us.)
+    constexpr long onePassGroups = 32, onePassSteps = 4;
+    const bool onePass = !byRows && !wide && O <= 64 && (forced || (G <= onePassGroups * onePassSteps && envInt("ACRO_HIP_ONE_PASS") >= 0));
+    if (onePass && !forced) G = std::min(G, onePassGroups);
     // G counts the shares of the contraction range (rows of partials in the scratch buffer); the grid has one
     // workgroup per share and group of outputs.
     const long gridG = G * Go;
@@ -196,7 +226,7 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     // measured 16.8 instead of 17.2 us for the pair of launches at n = 2^20), at most 1024.  The one-pass
     // variant finishes with the lanes of the partial kernel.
     int NTf = NTr;
-    const bool twoKernels = envInt("ACRO_HIP_ONE_PASS") <= 0 || wideFinish || O > NTr;
+    const bool twoKernels = !onePass;
     if (twoKernels && !wideFinish)
     {
         NTf = kReductionLanes;
@@ -211,15 +241,16 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     std::snprintf(hex, sizeof(hex), "%016llx",
                   static_cast<unsigned long long>(hashString(dimName + "/reduction/" + (opt.noalias ? "n" : "a") +
                                                              (Positional() ? "p" : "u") +
-                                                             (twoKernels ? "2" : (envInt("ACRO_HIP_ONE_PASS") >= 2 ? "1l" : "1")) + "/" + str(envInt("ACRO_HIP_RED_PENCIL")) +
-                                                             (byRows ? "/rows" : (wide ? "/wide" : "")))));
+                                                             (twoKernels ? "2" : "1") + "/" + str(envInt("ACRO_HIP_RED_PENCIL")) +
+                                                             (byRows ? "/rows" : (wide ? "/wide" : (flat ? "/flat" : ""))))));
     plan.module_name = std::string("acro_red_") + hex;
     const std::string fPartial = plan.module_name + "_partial", fFinal = plan.module_name + "_final";
 
     std::ostringstream sched;
     sched << "reduction schedule: " << O << " output entries, contraction of " << Nc << " terms split over " << G
           << " workgroups x " << Sn << " slices ("
-          << (pencil ? "a lane owns whole slices"
+          << (flat ? "output entries on adjacent lanes, two on each, " + str(2 * flatLanes) + " entries of the operand per window"
+              : pencil ? "a lane owns whole slices"
                      : (byRows ? "four outputs per workgroup, 64 adjacent lanes along each"
                                : (wide ? "256 outputs per workgroup, a lane each"
                                        : (outputsFastest ? "output entries on adjacent lanes" : "slices on adjacent lanes"))))
@@ -252,15 +283,96 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     // ---- stage 1: per-workgroup partial sums
     out << "\nextern \"C\" __global__ __launch_bounds__(" << NTr << ") void " << fPartial << "(" << ParamList()
         << ", double *__restrict__ scratch)\n{\n";
-    out << "    __shared__ double red[" << (pencil ? NTr * O : (byRows ? NTr + Ow * 16 : NTr)) << "];\n";
+    out << "    __shared__ double red[" << (flat ? 2 * NTr : pencil ? NTr * O : (byRows ? NTr + Ow * 16 : NTr)) << "];\n";
     if (!twoKernels) out << "    __shared__ int isLast;\n";
     out << "    const int lane = threadIdx.x;\n";
+    if (flat) out << "    typedef double acro_pair __attribute__((ext_vector_type(2), aligned(8)));\n";
     // Workgroups interleave: in every step the G workgroups together read one contiguous window of the
     // operands, so the device-wide access pattern is a single moving front.  Neighbouring workgroups share the
     // cache lines at their border, so neighbours run on the same XCD (one L2): hardware deals consecutive
     // workgroup ids round-robin to the 8 XCDs.
     const std::string gExpr = (G % 8 == 0) ? "(long)(blockIdx.x % 8) * " + str(G / 8) + " + blockIdx.x / 8" : std::string("blockIdx.x");
-    if (pencil)
+    if (flat)
+    {
+        // Streams that the memory-side cache (256 MB) cannot hold until the next call are read with the non-temporal hint
+        // (440 MB: 71.9 -> 66.7 us; three sets of 84 MB in turn, which it does hold: 13.6 -> 15.4 us, hence the line).
+        // (whole lines per slice take it at any size, as before: see ntBig)
+        const bool hint = ntBig || (envInt("ACRO_HIP_RED_NT") >= 0 && big->size >= (1L << 25));
+        const long window = 2 * flatLanes, windows = big->size / window;
+        const std::string A = PtrName(big->uvar) + (uvars[big->uvar].viewOffset != 0 ? " + " + Lit(uvars[big->uvar].viewOffset) : std::string());
+        // the product of one term, the big operand's entry being `x`; slice `c`, output entry o0 or o1
+        auto term = [&](const std::string &x, int k) {
+            std::string prod;
+            for (const auto &r : s.in)
+            {
+                std::string opnd = x;
+                if (&r != big)
+                {
+                    std::string at = uvars[r.uvar].viewOffset != 0 ? Lit(uvars[r.uvar].viewOffset) : std::string("0");
+                    for (size_t d = 0; d < r.idx.size(); ++d)
+                    {
+                        const bool contracted = has(s.contr, r.idx[d]);
+                        const std::vector<int> &ids = contracted ? contrIds : outIds;
+                        long div = 1;
+                        for (size_t j = ids.size(); j-- > 0 && ids[j] != r.idx[d];) div *= extent[ids[j]];
+                        std::string n = (contracted ? "c" : "o") + str(static_cast<long>(k));
+                        if (div > 1) n = "(" + n + " / " + str(div) + ")";
+                        if (ids[0] != r.idx[d]) n = "(" + n + " % " + str(static_cast<long>(extent[r.idx[d]])) + ")";
+                        at += " + " + std::string(contracted ? "(" + std::string(OffsetType()) + ")" : "") + n + " * " + Lit(r.stride[d]);
+                    }
+                    opnd = PtrName(r.uvar) + "[" + at + "]";
+                }
+                prod = prod.empty() ? opnd : "(" + prod + " * " + opnd + ")";
+            }
+            return prod;
+        };
+        const std::string cType = Nc < (1L << 31) - 2 * flatSlices ? "int" : "long";
+        out << "    const int o0 = (2 * lane) % " << O << ", o1 = (2 * lane + 1) % " << O << ", n0 = (2 * lane) / " << O << ", n1 = (2 * lane + 1) / " << O << ";\n";
+        out << "    const long g = " << gExpr << ";\n";
+        out << "    const double *A = " << A << " + 2 * lane;\n";
+        out << "    double s0[" << kFlatWindows << "], s1[" << kFlatWindows << "];\n";
+        out << "#pragma unroll\n    for (int u = 0; u < " << kFlatWindows << "; ++u) s0[u] = s1[u] = 0.0;\n";
+        out << "    if (lane < " << flatLanes << ")\n    {\n";
+        out << "        long w = g;\n";
+        out << "        for (; w + " << (kFlatWindows - 1) * G << " < " << windows << "; w += " << kFlatWindows * G << ")\n        {\n";
+        out << "            acro_pair x[" << kFlatWindows << "];\n";
+        out << "#pragma unroll\n            for (int u = 0; u < " << kFlatWindows << "; ++u)\n            {\n";
+        out << "                const acro_pair *p = reinterpret_cast<const acro_pair *>(A + (w + u * " << G << "L) * " << window << ");\n";
+        out << "                x[u] = " << (hint ? "__builtin_nontemporal_load(p)" : "*p") << ";\n            }\n";
+        out << "#pragma unroll\n            for (int u = 0; u < " << kFlatWindows << "; ++u)\n            {\n";
+        out << "                const " << cType << " c = (" << cType << ")((w + u * " << G << "L) * " << flatSlices << "), c0 = c + n0, c1 = c + n1;\n";
+        out << "                s0[u] += " << term("x[u].x", 0) << ";\n                s1[u] += " << term("x[u].y", 1) << ";\n            }\n        }\n";
+        out << "        for (; w < " << windows << "; w += " << G << ")\n        {\n";
+        out << "            const acro_pair x = *reinterpret_cast<const acro_pair *>(A + w * " << window << ");\n";
+        out << "            const " << cType << " c = (" << cType << ")(w * " << flatSlices << "), c0 = c + n0, c1 = c + n1;\n";
+        out << "            s0[0] += " << term("x.x", 0) << ";\n            s1[0] += " << term("x.y", 1) << ";\n        }\n";
+        if (Nc % flatSlices != 0)
+        {
+            // the slices behind the last whole window
+            const long c0 = windows * flatSlices;
+            out << "        if (g == " << G - 1 << ")\n        {\n";
+            out << "            const " << cType << " c0 = " << c0 << " + n0, c1 = " << c0 << " + n1;\n";
+            out << "            if (c0 < " << Nc << ") s0[1] += " << term("A[" + str(windows * window) + "L]", 0) << ";\n";
+            out << "            if (c1 < " << Nc << ") s1[1] += " << term("A[" + str(windows * window) + "L + 1]", 1) << ";\n        }\n";
+        }
+        out << "    }\n";
+        out << "    red[2 * lane] = (s0[0] + s0[1]) + (s0[2] + s0[3]);\n    red[2 * lane + 1] = (s1[0] + s1[1]) + (s1[2] + s1[3]);\n    __syncthreads();\n";
+        // the window's slices are added by `shares` lanes per output entry, then by one: a fixed order
+        long shares = 1;
+        while (4 * shares * shares <= flatSlices && 2 * shares * O <= NTr) shares *= 2;
+        if (shares > 1)
+        {
+            const long each = (flatSlices + shares - 1) / shares;
+            out << "    double part = 0.0;\n    if (lane < " << shares * O << ")\n    {\n";
+            out << "#pragma unroll\n        for (int k = 0; k < " << each << "; ++k)\n        {\n";
+            out << "            const int n = (lane / " << O << ") * " << each << " + k;\n";
+            out << "            part += n < " << flatSlices << " ? red[n * " << O << " + lane % " << O << "] : 0.0;\n        }\n    }\n";
+            out << "    __syncthreads();\n    if (lane < " << shares * O << ") red[lane] = part;\n    __syncthreads();\n";
+        }
+        out << "    if (lane < " << O << ")\n    {\n        double t = 0.0;\n";
+        out << "        for (int k = 0; k < " << (shares > 1 ? shares : flatSlices) << "; ++k) t += red[k * " << O << " + lane];\n";
+    }
+    else if (pencil)
     {
         for (long o = 0; o < O; ++o) out << "    double acc" << o << " = 0.0;\n";
         out << "    {\n        const long g = " << gExpr << ";\n";
@@ -402,17 +514,15 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     else if (twoKernels)
         out << "        scratch[(long)blockIdx.x * " << O << " + lane] = t;\n    }\n}\n";
     else
-        out << "        __hip_atomic_store(&scratch[(long)blockIdx.x * " << O
+        out << "        __hip_atomic_store(&scratch[" << "(long)blockIdx.x * " << O
             << " + lane], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n    }\n";
 
     // ---- stage 2: add the per-workgroup partials in a fixed order and apply the assignment operator.
-    // Default: a second, single-workgroup kernel.
-    // ACRO_HIP_ONE_PASS=1: the workgroup that arrives last at a device-wide counter does it instead (partials
-    // written with device-scope atomic stores, arrival counted with a release, the last workgroup acquires; the
-    // counter lives behind the partials in the scratch buffer, which the executor zeroes when it allocates it,
-    // and the last workgroup sets it back to zero).  A release at device scope writes back the L2 of the
-    // workgroup's XCD; with 256 workgroups the single launch measured 18.4 us against 16.3 us for the two
-    // launches (55.9 us when every lane also fenced), so it is not the default.
+    // A second, single-workgroup kernel, or, where few workgroups share the range (onePass above), the workgroup that
+    // arrives last at a device-wide counter: the partials are written by the first wavefront (at most 64 outputs) with
+    // device-scope atomic stores, its first lane counts the arrival with a release, the last workgroup acquires.  The
+    // counter lies behind the partials in the scratch buffer, which the executor zeroes when it allocates it, and the
+    // last workgroup sets it back to zero.
     auto emitFinish = [&](const std::string &load) {
         out << "    const int g2 = lane / " << O << ", o2 = lane % " << O << ";\n";
         out << "    double sum2 = 0.0;\n";
@@ -475,17 +585,8 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     }
     else
     {
-        // The partials were stored by the wavefront of lane 0 with device-scope atomic stores; its release on the
-        // counter orders them before the arrival.  Only the last workgroup needs the acquire side.
-        // ACRO_HIP_ONE_PASS=2: the partials were written through to the device's point of coherence by the
-        // atomic stores; the storing wavefront only waits until they are acknowledged (a workgroup-scope release)
-        // and the arrival is counted without the device-scope release that writes back the XCD's L2.
-        const bool light = envInt("ACRO_HIP_ONE_PASS") >= 2;
-        if (light) out << "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"workgroup\");\n";
-        out << "    __syncthreads();\n";
         out << "    if (lane == 0)\n    {\n";
-        out << "        const unsigned int arrived = __hip_atomic_fetch_add(" << counter
-            << ", 1u, " << (light ? "__ATOMIC_RELAXED" : "__ATOMIC_RELEASE") << ", __HIP_MEMORY_SCOPE_AGENT);\n";
+        out << "        const unsigned int arrived = __hip_atomic_fetch_add(" << counter << ", 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);\n";
         out << "        isLast = (arrived == " << G - 1 << "u);\n    }\n";
         out << "    __syncthreads();\n";
         out << "    if (!isLast) return;\n";
@@ -498,7 +599,7 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     plan.source = out.str();
     plan.scratch_doubles = static_cast<size_t>(G * O) + (twoKernels ? 0 : 1);
     plan.nb = 1;
-    plan.lds_bytes = static_cast<int>((pencil ? NTr * O : NTr) * 8);
+    plan.lds_bytes = static_cast<int>((flat ? 2 * NTr : pencil ? NTr * O : NTr) * 8);
     FillParams(plan, false);
     const int S = static_cast<int>(stores.size());
     HipLaunch partial;

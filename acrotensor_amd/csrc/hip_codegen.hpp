@@ -130,9 +130,12 @@
 //                               no non-temporal hint on operands that are read once in whole lines (chain, reduction, Gram
 //                               and product schedules)
 //   ACRO_HIP_RED_ROWS=-1        split contractions of few long rows: all outputs in every workgroup, NT / outputs lanes along a row
-//   ACRO_HIP_ONE_PASS=1         split contractions: the workgroup that finishes last adds the per-workgroup partials
-//                               instead of a second kernel (measured 18.4 against 16.3 us: the device-scope release
-//                               writes back the XCD's L2 once per workgroup)
+//   ACRO_HIP_ONE_PASS=1|-1      split contractions of up to 64 outputs: the workgroup that finishes last adds the per-workgroup
+//                               partials whatever the size / never (default: where at most 128 workgroups would share the
+//                               range; 256 workgroups 18.4 against 16.3 us: the device-scope release writes back the XCD's
+//                               L2 once per workgroup)
+//   ACRO_HIP_RED_FLAT=-1|1      split contractions whose outputs are the fastest dimensions of the big operand: never / always
+//                               two neighbouring entries per lane (default: from ten outputs or 96 MB on)
 //   ACRO_HIP_RED_GROUPS=<n> / ACRO_HIP_RED_UNROLL=<n>
 //                               split contractions where a lane owns whole slices: number of workgroups (default 256, one per
 //                               compute unit) and slices a lane requests before it adds them (default 1)

@@ -1439,3 +1439,56 @@ def test_dense_operator_with_dimensions_in_any_order(at, engine, checker, kernel
     if "-=" in kernel:
         expected = 2.0 * out0 - expected
     assert rel_err(got, expected) <= TOL
+
+
+@pytest.mark.parametrize("kernel,terms,outs,others", [
+    # slices per window are 2 * 252 / 9 = 56: below one window, one exactly, one more, several steps of the unrolled loop
+    ("S_i_j = A_n_i_j B_n", (2049,), (3, 3), ("n",)), ("S_i_j += A_n_i_j B_n", (56 * 40,), (3, 3), ("n",)),
+    ("S_i_j -= A_n_i_j B_n", (56 * 41 + 1,), (3, 3), ("n",)), ("S_i_j = A_n_i_j B_n", (56 * 8 * 130 + 55,), (3, 3), ("n",)),
+    ("S_i_j = A_n_i_j B_n", (30011,), (4, 5), ("n",)), ("S_i_j = A_n_i_j B_n", (5003,), (6, 6), ("n",)), ("S_i = A_n_i", (9001,), (2,), ()),
+    ("S_i = A_n_i B_n", (12007,), (40,), ("n",)), ("S_i = A_n_i B_n C_i", (9007,), (64,), ("n", "i")), ("S_i = A_n_i B_n", (8009,), (127,), ("n",)),
+    ("S_j_i = A_n_m_i_j B_m C_j_n", (97, 101), (5, 7), ("m", "jn")), ("S_i = B_m_n A_m_n_i C_n_i B_m_n", (61, 67), (11,), ("mn", "ni")),
+])
+def test_split_contraction_with_two_entries_per_lane(at, engine, checker, monkeypatch, kernel, terms, outs, others):
+    """The stream of (terms, outputs) in windows: remainders of windows, odd and even numbers of outputs, both finishes,
+    a first entry that is not 16-byte aligned, NaN that must stay where it is put.  Integer values: exact."""
+    monkeypatch.setenv("ACRO_HIP_RED_FLAT", "1")
+    te = at.TensorEngine("HIP")
+    rng = np.random.default_rng(len(kernel) + terms[0])
+    ext = {}
+    lhs, rhs = kernel.replace("+=", "=").replace("-=", "=").split("=")
+    tokens = rhs.split()
+    big = [t for t in tokens if t.startswith("A_")][0].split("_")[1:]
+    ext.update(zip(big, terms + outs))
+    shape = {t.split("_")[0]: tuple(ext[x] for x in t.split("_")[1:]) for t in [lhs.strip()] + tokens}
+    values = {n: rng.integers(-4, 5, s).astype(np.float64) for n, s in shape.items()}
+    parent = at.Tensor(int(np.prod(shape["A"])) + 1)       # the operand starts at an odd double of its parent
+    parent.data[...] = np.concatenate([[np.nan], values["A"].ravel()])
+    parent.MoveToGPU()
+    at.synchronize()
+    A = at.Tensor(*shape["A"], hdata=np.empty(shape["A"]), ddata=parent.GetDeviceData() + 8, ongpu=True)
+    tensors = {n: (A if n == "A" else to_tensor(at, v)) for n, v in values.items()}
+    src = te.GetImplementation(kernel, tensors["S"], *[tensors[t.split("_")[0]] for t in tokens])
+    assert "two on each" in src
+    for _ in range(3):
+        te(kernel, tensors["S"], *[tensors[t.split("_")[0]] for t in tokens])
+    S = tensors["S"]
+    S.MoveFromGPU()
+    expected = values["S"].copy()
+    for _ in range(3):
+        term = np.einsum(",".join("".join(t.split("_")[1:]) for t in tokens) + "->" + "".join(lhs.strip().split("_")[1:]),
+                         *[values[t.split("_")[0]] for t in tokens])
+        expected = expected + term if "+=" in kernel else expected - term if "-=" in kernel else term
+    assert np.array_equal(S.data, expected)
+    # one NaN: only its output entry sees it
+    where = tuple(d - 1 for d in shape["A"])
+    values["A"][where] = np.nan
+    if "=" in kernel and "+=" not in kernel and "-=" not in kernel:
+        parent.MoveFromGPU()
+        parent.data[1:] = values["A"].ravel()
+        parent.MoveToGPU()
+        at.synchronize()
+        te(kernel, S, *[tensors[t.split("_")[0]] for t in tokens])
+        S.MoveFromGPU()
+        out = tuple(where[big.index(x)] for x in lhs.strip().split("_")[1:])
+        assert np.isnan(S.data[out]) and np.isnan(S.data).sum() == 1

@@ -96,3 +96,25 @@ def test_work_that_needs_the_host_is_refused_while_recording(at, engine):
     assert np.array_equal(A.data, B.data)
     with pytest.raises(at.AcroError):
         at.recorded_launches().launch()                   # nothing recorded
+
+
+@pytest.mark.parametrize("n", [4096, 33000])              # one launch, the last workgroup adds; two launches
+def test_replays_of_a_split_contraction_match_eager_launches(at, engine, n):
+    rng = np.random.default_rng(n)
+    A, B, S = to_tensor(at, rng.uniform(0, 1, (n, 4, 5))), to_tensor(at, rng.uniform(0.5, 1.5, n)), at.Tensor(4, 5)
+    engine("S_i_j = A_n_i_j B_n", S, A, B)
+    assert ("finishes last" in engine.GetLastImplementation()) == (n == 4096)
+    with at.recorded_launches() as seq:
+        engine("S_i_j = A_n_i_j B_n", S, A, B)
+    for rep in range(4):
+        A.Mult(1.25)
+        at.synchronize()
+        seq.launch()
+        S.MoveFromGPU()
+        replayed = S.data.copy()
+        S.MoveToGPU()
+        S.Set(0.0)
+        engine("S_i_j = A_n_i_j B_n", S, A, B)
+        S.MoveFromGPU()
+        assert np.array_equal(replayed, S.data) and replayed.min() > 0.0, rep
+        S.MoveToGPU()
