@@ -785,7 +785,14 @@ auto Generator::ChooseCopyOutTile() -> void
             if (uvars[r.uvar].storage == u.storage) return;
         }
     }
-    if (st.tileSize > envInt("ACRO_HIP_COPY_OUT_MAX", 2048)) return;
+    // Results in planes ("D_e_m_n_k1_k2_k3" with the lanes along k and the tile (m, n)) whose length is no multiple of 64
+    // bytes: a wavefront's stores start anywhere in a line, and a streaming store of part of a 64-byte piece costs as much as
+    // two.  An entry's planes are one contiguous range, so they leave through a tile too, of up to 64 KB.  Geometric factors
+    // from the Jacobians, planes of 343 doubles: 207 -> 173 us (ordinary stores 180), 125: 43.4 -> 40.7, 729: 264 -> 236;
+    // lengths that are such multiples keep their stores: 1 000 441 (through the tile 464), 512 254 (259), 216 166 (171).
+    bool oddPlanes = s.laneCount % 8 != 0 && s.laneCount >= 64 && s.out.idx.size() > s.lane.size() && envInt("ACRO_HIP_COPY_OUT_PLANES") >= 0;
+    for (size_t d = 0; oddPlanes && d < s.lane.size(); ++d) oddPlanes = has(s.lane, s.out.idx[s.out.idx.size() - 1 - d]);
+    if (st.tileSize > envInt("ACRO_HIP_COPY_OUT_MAX", oddPlanes ? 8192 : 2048)) return;
     // the run of consecutive outputs of one work item: the trailing output dimensions that are tile indices
     long run = 1;
     for (size_t d = s.out.idx.size(); d-- > 0;)
@@ -809,8 +816,8 @@ auto Generator::ChooseCopyOutTile() -> void
     {
         const int entries = static_cast<int>(std::max<long>(1, 64 / std::max<long>(1, s.laneCount)));
         const double coverage = WaveStoreLineCoverage(k, entries);
-        scattered = s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", 30) ||
-                                         (coverage < 0.95 && envInt("ACRO_HIP_COPY_OUT_WRITERS") >= 0 && WritesDominate()));
+        scattered = oddPlanes || (s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", 30) ||
+                                         (coverage < 0.95 && envInt("ACRO_HIP_COPY_OUT_WRITERS") >= 0 && WritesDominate())));
     }
     if (subs.size() != 1 && !scattered) return;
     if (run < longRun && !scattered) return;
