@@ -4,10 +4,13 @@ The library is built in-tree by ``acrotensor_amd.build.build_library`` (hipcc, g
 it is missing: there is no host fallback for any operation.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libacrotensor_hip.so")
+CALL_PATH = os.path.join(_HERE, "lib", "_acro_call.so")
 
 c_int_p = ctypes.POINTER(ctypes.c_int)
 c_double_p = ctypes.POINTER(ctypes.c_double)
@@ -84,6 +87,22 @@ SIGNATURES = {
 }
 
 _lib = None
+_contract = None
+
+
+def contract_function():
+    """``contract(engine address, kernel string, output, tuple of inputs) -> status``: acro_engine_contract for tensors
+    of acrotensor_amd.api, without ctypes between (csrc/python_call.cpp)."""
+    global _contract
+    if _contract is None:
+        load()
+        if not os.path.exists(CALL_PATH):
+            raise RuntimeError("_acro_call.so is not built (%s missing): run `make -C acrotensor_amd/csrc`." % CALL_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("_acro_call", CALL_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_acro_call", loader))
+        loader.exec_module(module)
+        _contract = module.contract
+    return _contract
 
 
 def load():

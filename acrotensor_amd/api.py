@@ -70,6 +70,7 @@ class Tensor:
             _check(self._lib.acro_tensor_create(n, arr, hptr, dptr, 1 if ongpu else 0, ctypes.byref(self._h)))
         else:
             raise AcroError("A tensor needs at least one dimension.")
+        self._address = self._h.value
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None
@@ -201,7 +202,9 @@ class TensorEngine:
     def __init__(self, exec_type="HIP"):
         self._lib = _capi.load()
         self._h = ctypes.c_void_p()
+        self._contract = _capi.contract_function()
         _check(self._lib.acro_engine_create(exec_type.encode(), ctypes.byref(self._h)))
+        self._address = self._h.value
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None
@@ -217,8 +220,8 @@ class TensorEngine:
         return arr, len(tensors)
 
     def __call__(self, kernel, out, *inputs):
-        arr, n = self._handles(inputs)
-        _check(self._lib.acro_engine_contract(self._h, kernel.encode(), out._h, arr, n))
+        if self._contract(self._address, kernel, out, inputs):
+            _check(1)
 
     def contract_no_alloc(self, kernel, out, *inputs):
         """The same as calling the engine, for callers that cannot allocate: tensors must be resident on the device

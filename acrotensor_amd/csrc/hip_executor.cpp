@@ -8,6 +8,7 @@
 //  * a group that cannot be fused safely (no common outer index, a variable used with different shapes, or
 //    overlapping variables of which one is written) is executed as one launch per kernel, in stream order;
 //  * everything is enqueued on the library's stream and never synchronised here.
+#include <algorithm>
 #include <map>
 #include <memory>
 
@@ -291,13 +292,15 @@ class HipExecutor : public KernelExecutor
             // what Bind derives from a slice's parents: the tensor it is a view of, where, and that tensor's shape
             const Tensor *root = t;
             s.offset = 0;
-            while (const SliceTensor *sl = dynamic_cast<const SliceTensor *>(root))
+            while (const Tensor *parent = root->GetViewParent())
             {
-                s.offset += sl->GetOffset();
-                root = sl->GetParent();
+                s.offset += static_cast<const SliceTensor *>(root)->GetOffset();
+                root = parent;
             }
             s.root = root;
+            s.root_host = root->GetData();
             s.root_device = root->GetDeviceData();
+            s.root_size = root->GetSize();
             s.root_shape = 1469598103934665603ull;
             for (int d = 0; d < root->GetRank(); ++d) s.root_shape = (s.root_shape ^ static_cast<unsigned>(root->GetDim(d))) * 1099511628211ull;
             ThisCall.push_back(s);
@@ -307,7 +310,7 @@ class HipExecutor : public KernelExecutor
             note(outputs[ki]);
             for (const Tensor *t : inputs[ki]) note(t);
         }
-        const bool repeated = gathered.empty() && LastCallVariant != nullptr && ThisCall == LastCall;
+        const bool repeated = gathered.empty() && LastCallVariant != nullptr && (ThisCall == LastCall || SameBinding());
         HipCodegenOptions options;
         if (!repeated)
         {
@@ -334,6 +337,7 @@ class HipExecutor : public KernelExecutor
         {
             LastCall.swap(ThisCall);
             LastCallVariant = &v;
+            if (!repeated) NoteBinding(options);
         }
         MaterialiseGathered(gathered, v.plan.gathers_applied ? &options.gathered : nullptr);
         std::vector<const int *> gatherMap(gathered.size(), nullptr);
@@ -403,8 +407,8 @@ class HipExecutor : public KernelExecutor
     struct Seen
     {
         const Tensor *tensor, *root;
-        const double *host, *device, *root_device;
-        size_t size, offset;
+        const double *host, *device, *root_host, *root_device;
+        size_t size, offset, root_size;
         unsigned long long root_shape;
         bool transient;
         bool operator==(const Seen &o) const
@@ -415,6 +419,79 @@ class HipExecutor : public KernelExecutor
     };
     std::vector<Seen> ThisCall, LastCall;
     Variant *LastCallVariant = nullptr;
+    // How the previous call's tensors relate to each other, per occurrence: the first occurrence of the same tensor, of the
+    // same root, of the same host range.  A call on other tensors that relate in the same way, with the same shapes,
+    // offsets and marks, binds to the same operands (a program that goes through several sets of tensors).
+    struct Relation
+    {
+        int tensor, root, range;
+        bool operator==(const Relation &o) const { return tensor == o.tensor && root == o.root && range == o.range; }
+    };
+    std::vector<Relation> LastRelations;
+    std::vector<int> LastRoots;       // the first occurrence of every root
+    std::vector<char> WrittenRoots;   // ... and whether a kernel of the group writes it
+    bool LastCallAliased = true;
+
+    static Relation Relate(const std::vector<Seen> &call, size_t i)
+    {
+        Relation r{-1, -1, -1};
+        for (size_t j = 0; j <= i && (r.tensor < 0 || r.root < 0 || r.range < 0); ++j)
+        {
+            const int first = static_cast<int>(j);
+            if (r.tensor < 0 && call[j].tensor == call[i].tensor) r.tensor = first;
+            if (r.root < 0 && call[j].root == call[i].root) r.root = first;
+            if (r.range < 0 && call[j].host == call[i].host && call[j].size == call[i].size) r.range = first;
+        }
+        return r;
+    }
+
+    // After the analysis of a call (now in LastCall): what SameBinding compares the next one with.
+    void NoteBinding(const HipCodegenOptions &options)
+    {
+        LastCallAliased = !options.noalias;
+        LastRelations.clear();
+        LastRoots.clear();
+        WrittenRoots.clear();
+        for (size_t i = 0; i < LastCall.size(); ++i)
+        {
+            LastRelations.push_back(Relate(LastCall, i));
+            if (LastRelations.back().root == static_cast<int>(i)) LastRoots.push_back(static_cast<int>(i));
+        }
+        WrittenRoots.assign(LastRoots.size(), 0);
+        size_t i = 0;
+        for (int ki = 0; ki < MultiKernel->GetNumKernels(); i += 1 + MultiKernel->Kernels[ki]->GetNumInputVars(), ++ki)
+        {
+            const int root = LastRelations[i].root;   // occurrence i is the output of kernel ki
+            WrittenRoots[std::find(LastRoots.begin(), LastRoots.end(), root) - LastRoots.begin()] = 1;
+        }
+    }
+
+    // Whether this call's tensors lead to the previous call's variant without the analysis.
+    bool SameBinding() const
+    {
+        if (LastCallAliased || ThisCall.size() != LastRelations.size()) return false;
+        for (size_t i = 0; i < ThisCall.size(); ++i)
+        {
+            const Seen &a = ThisCall[i], &b = LastCall[i];
+            if (a.size != b.size || a.offset != b.offset || a.transient != b.transient || a.root_shape != b.root_shape) return false;
+            if (!(Relate(ThisCall, i) == LastRelations[i])) return false;
+        }
+        // no written root overlaps another
+        for (size_t x = 0; x < LastRoots.size(); ++x)
+        {
+            const Seen &a = ThisCall[LastRoots[x]];
+            for (size_t y = x + 1; y < LastRoots.size(); ++y)
+            {
+                if (!WrittenRoots[x] && !WrittenRoots[y]) continue;
+                const Seen &b = ThisCall[LastRoots[y]];
+                if (a.root_host < b.root_host + b.root_size && b.root_host < a.root_host + a.root_size) return false;
+                if (a.root_device != nullptr && b.root_device != nullptr && a.root_device < b.root_device + b.root_size &&
+                    b.root_device < a.root_device + a.root_size)
+                    return false;
+            }
+        }
+        return true;
+    }
 };
 
 KernelExecutor *CreateHipExecutor(DimensionedMultiKernel *multi_kernel)

@@ -43,6 +43,7 @@ class SliceTensor : public Tensor
     bool IsMappedToGPU() const override;
     bool IsOnGPU() const override;
     bool IsTransient() const override;
+    const Tensor *GetViewParent() const override { return FullT; }
 
     Tensor *GetParent() const { return FullT; }
     size_t GetOffset() const { return Offset; }

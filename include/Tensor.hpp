@@ -138,6 +138,8 @@ class Tensor
     // on-chip memory only, so its contents in device memory are unspecified afterwards.
     void SetTransient(bool transient) { Transient = transient; }
     virtual bool IsTransient() const { return Transient; }
+    // The tensor this one is a view of; null for all but SliceTensor.
+    virtual const Tensor *GetViewParent() const { return nullptr; }
 
     // Extension (no counterpart in the reference, which allocates with new[], tensor/Tensor.cpp:196): host buffers
     // that tensors allocate from now on are page-locked, so MoveToGPU / MoveFromGPU run as direct transfers at
