@@ -546,8 +546,10 @@ auto Generator::EmitUnrolledBody(int k, ForwardMap &forwarded, std::vector<std::
 
     std::vector<int> value(nidx, 0);
     const long tc = s.tileCount;
+    std::vector<size_t> firstLine;   // of every tile entry's arithmetic
     for (long t = 0; t < tc; ++t)
     {
+        firstLine.push_back(body.compute.size());
         long rem = t;
         for (int j = static_cast<int>(s.tile.size()) - 1; j >= 0; --j)
         {
@@ -592,6 +594,7 @@ auto Generator::EmitUnrolledBody(int k, ForwardMap &forwarded, std::vector<std::
         forwarded[std::make_pair(s.out.uvar, goff)] = name;
     }
 
+    InterleaveTile(k, firstLine, body.compute);
     // The scope of a kernel applied after a matrix kernel is nested in that kernel's: back to the default there.
     for (int q = k; q > 0 && subs[q].fusedWithPrev; --q)
     {
@@ -605,6 +608,38 @@ auto Generator::EmitUnrolledBody(int k, ForwardMap &forwarded, std::vector<std::
     for (const auto &l : body.compute) lines.push_back(l);
     for (const auto &l : body.stores) lines.push_back(l);
     if (globalLoads != nullptr) *globalLoads = body.globalLoads;
+}
+
+// A transposed stage ("V1_e_i_r_s = B_q_i U_e_q_r_s", tile i, contraction q) reads its scalar operand down the columns when
+// the outputs of the tile are summed one after the other: all rows, 2 registers per entry, would have to be in scalar
+// registers at once (spilled from 81 entries on: mass apply at p = 8, 9^3 points 208 -> 175 us, diffusion apply 125 -> 112,
+// 10^3 133 -> 115; below 64 entries the compiler finds the order, 7 x 7 83 against 93).  Its sums are
+// written term by term instead, a row of the operand at a time (every output's own order of terms, and so its value, is the
+// same).
+auto Generator::InterleaveTile(int k, const std::vector<size_t> &firstLine, std::vector<std::string> &compute) const -> void
+{
+    const Sub &s = subs[k];
+    const int mode = envInt("ACRO_HIP_INTERLEAVE_TILE");
+    if (s.contr.size() != 1 || s.tile.size() != 1 || firstLine.size() < 2 || mode < 0) return;
+    bool downColumns = false;
+    for (size_t v = 0; v < s.in.size(); ++v)
+    {
+        const VarRef &r = s.in[v];
+        if (SourceOf(k, static_cast<int>(v)) != kFromConstant || r.idx.size() != 2 || r.size < (mode > 0 ? mode : 64)) continue;
+        downColumns = downColumns || (r.idx[0] == s.contr[0] && r.idx[1] == s.tile[0]);
+    }
+    const size_t lines = firstLine[1] - firstLine[0];
+    if (!downColumns || compute.size() - firstLine[0] != lines * firstLine.size()) return;
+    for (size_t t = 1; t < firstLine.size(); ++t)
+    {
+        if (firstLine[t] - firstLine[t - 1] != lines) return;
+    }
+    std::vector<std::string> turned(compute.begin(), compute.begin() + firstLine[0]);
+    for (size_t j = 0; j < lines; ++j)
+    {
+        for (size_t first : firstLine) turned.push_back(compute[first + j]);
+    }
+    compute.swap(turned);
 }
 
 // One work item of a matrix kernel: the entries of the operand's matrix are loaded like any operand, the

@@ -55,6 +55,9 @@
 //   ACRO_HIP_LDS_PAD=1|2        pad LDS tile strides against bank conflicts (2: even if a resident workgroup is lost)
 //   ACRO_HIP_PACK=1|-1          1: pick batch / workgroup size for wavefront utilisation also when one batch entry per
 //                               workgroup would do; -1: never (default: only for groups that batch several entries)
+//   ACRO_HIP_PACK_CHAINS=-1     groups of parallel chains choose batch and workgroup size like other groups
+//   ACRO_HIP_INTERLEAVE_TILE=-1|<n>  transposed stages sum the outputs of a tile one after the other / term by term from operators
+//                               of n entries on (default 64)
 //   ACRO_HIP_PERSIST=<n>        persistent grid of n workgroups per CU looping over the batch
 //   ACRO_HIP_PIPELINE=1         with ACRO_HIP_PERSIST: streaming inputs stay in registers across iterations and are
 //                               requested one iteration ahead

@@ -353,6 +353,7 @@ class Generator
     std::string GlobalStore(int k, const std::string &gaddr, const std::string &value) const;
     bool NeedsLdsCopy(int k) const;
     bool CopiesOutFromLds(int k) const;
+    void InterleaveTile(int k, const std::vector<size_t> &firstLine, std::vector<std::string> &compute) const;
     void EmitUnrolledBody(int k, ForwardMap &forwarded, std::vector<std::string> &lines, const std::map<std::string, std::string> *preloaded = nullptr, std::vector<std::pair<std::string, std::string>> *globalLoads = nullptr);
     void EmitMatrixBody(int k, Body &body, ForwardMap &forwarded);
     void EmitSplitLanesBody(int k, std::vector<std::string> &lines);

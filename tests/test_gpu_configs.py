@@ -97,6 +97,19 @@ def test_config5_diffusion_apply(at, engine, checker, E, Q, P, transient):
             assert rel_err(fetch(tensors, name), expected[name]) <= TOL, name
 
 
+@pytest.mark.parametrize("E,Q,P", [(3, 6, 5), (2, 7, 6), (5, 6, 6), (3, 7, 7), (3, 9, 9), (2, 10, 9), (7, 9, 9)])
+@pytest.mark.parametrize("transient", [False, True])
+def test_diffusion_apply_with_three_wavefronts_or_two_entries_per_workgroup(at, engine, checker, E, Q, P, transient):
+    # chains that fill about half of their wavefronts (two entries), three wavefronts per phase, phases of six wavefronts in
+    # two passes, operators of more than 64 entries applied transposed a row at a time
+    test_config5_diffusion_apply(at, engine, checker, E, Q, P, transient)
+
+
+@pytest.mark.parametrize("E,Q,P,transient", [(11, 9, 9, True), (10, 10, 9, False), (9, 8, 8, True)])
+def test_mass_apply_with_operators_read_a_row_at_a_time(at, engine, checker, E, Q, P, transient):
+    test_mass_apply_at_other_degrees(at, engine, checker, E, Q, P, transient)
+
+
 def golden_workloads():
     return sorted(f for f in os.listdir(GOLDEN) if f.startswith("workload_")) if os.path.isdir(GOLDEN) else []
 
