@@ -1110,7 +1110,45 @@ auto Generator::ChooseBatching() -> void
         // wavefronts (p=2 mass assembly).  Groups that batch anyway take the better packing (p=1 mass apply:
         // 8 -> 14 entries per workgroup, 62.9 -> 74.9 % of the HBM peak; p=4: 2 -> 5 entries in 256 lanes,
         // 67.5 -> 72.0 %), and so do groups whose wavefronts would be mostly idle.
-        const bool wanted = envInt("ACRO_HIP_PACK") > 0 || (envInt("ACRO_HIP_PACK") == 0 && (NB > 1 || idle < 0.5));
+        // So do groups of parallel chains (phases of several kernels, "chains") whose kernels fill about half of their
+        // wavefronts, whatever the pointwise kernels between them do: diffusion apply at p = 4, 6^3 points, two entries in
+        // 256 lanes 86.8 -> 69.0 us.  Chains that fill more keep one entry, and where a phase is then three wavefronts, the
+        // workgroup is three wavefronts too (the fourth had nothing but its share of the pointwise kernel, and kept its
+        // registers): p = 5, 6^3 / 7^3 points 90.9 -> 81.6 / 92.2 -> 70.4 us, p = 6, 7^3 / 8^3 93.3 -> 83.2 / 88.0 -> 83.8.
+        // Full wavefronts keep four (p = 7, 8^3 points 66.5 against 69.5 us).  Phases of six wavefronts run in two passes
+        // of three where no phase is narrower than two and LDS lets four workgroups live on a compute unit (p = 8, 9^3
+        // points 112 -> 83.5 us; a single wavefront in the first and last phase, p = 7, 9^3: 66.9 against 69.1; three
+        // workgroups, p = 7 and 10^3: 940 against 1 110).
+        double chainItems = 0.0, chainLanes = 0.0;
+        long mostWaves = 0, leastWaves = 64;
+        for (int ph = 0; ph <= subs.back().phase; ++ph)
+        {
+            long kernelsHere = 0, waves = 0;
+            double items = 0.0, lanes = 0.0;
+            for (const auto &s : subs)
+            {
+                if (s.phase != ph || s.fusedWithPrev) continue;
+                const double weight = static_cast<double>(std::max<long>(1, s.tileCount * s.contrCount));
+                ++kernelsHere;
+                waves += (s.laneCount + 63) / 64;
+                items += weight * s.laneCount;
+                lanes += weight * 64.0 * ((s.laneCount + 63) / 64);
+            }
+            if (kernelsHere > 0) leastWaves = std::min(leastWaves, waves);
+            if (kernelsHere < 3) continue;
+            chainItems += items;
+            chainLanes += lanes;
+            mostWaves = std::max(mostWaves, waves);
+        }
+        const bool chains = chainLanes > 0.0 && envInt("ACRO_HIP_PACK_CHAINS") >= 0;
+        const double chainFill = chains ? chainItems / chainLanes : 1.0;
+        auto ldsOfOneEntry = [&] {
+            const int firstFit = PlaceLds(1), bothEnds = PlaceLdsFromBothEnds(1);
+            return bothEnds > 0 ? std::min(firstFit, bothEnds) : firstFit;
+        };
+        const bool threeWide = mostWaves == 3 || (mostWaves == 6 && leastWaves >= 2 && ldsOfOneEntry() <= 160 * 1024 / 8 / 4);
+        if (chains && NB == 1 && NT == 256 && threeWide && chainFill >= 0.54 && chainFill < 0.9) NT = bestNT = 192;
+        const bool wanted = envInt("ACRO_HIP_PACK") > 0 || (envInt("ACRO_HIP_PACK") == 0 && NT != 192 && (NB > 1 || idle < 0.5 || chainFill < 0.54));
         if (wanted && best >= 1.1 * base)
         {
             NB = bestNB;
