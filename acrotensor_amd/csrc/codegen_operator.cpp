@@ -762,6 +762,10 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
         const long C = sh.comp;
         // (a block of rows: the entries' results lie `stride` apart and start at row `off`)
         const long stride = sh.allRows > 0 ? sh.allRows : rows, off = sh.rowOffset;
+        // Runs of 128 bytes that start anywhere in a 64-byte piece: ordinary stores, which L2 merges; with streaming stores
+        // a piece that two of them share reaches memory twice.  125 x 64 on 131 072 entries and its transpose behind it
+        // 110.0 -> 102.2 us, 115 x 64 108.2 -> 98.8, 110 x 60 109.2 -> 103.2; never slower from 75 x 40 on.
+        const bool streamsHere = streams && (stride % 8 == 0 || envInt("ACRO_HIP_OPERATOR_ODD_ROWS") < 0);
         if (viaStage)
         {
             const int perRound = 4 / stageRounds;   // result registers (entries g + 4 r) per round
@@ -844,7 +848,7 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
             out << "                " << guard << "mid[(4 * r + g) * " << midStride << " + 16 * t + c] = " << value << ";\n";
         else if (C > 1)
             out << "                " << guard << "a[" << 16 * C << " * t]" << (ks.op == '=' ? " = " : (ks.op == '+' ? " += " : " -= ")) << value << ";\n";
-        else if (streams)
+        else if (streamsHere)
             out << "                " << guard << "__builtin_nontemporal_store(" << value << ", a + 4 * r * " << stride << " + 16 * t);\n";
         else
             out << "                " << guard << "a[4 * r * " << stride << " + 16 * t]" << (ks.op == '=' ? " = " : (ks.op == '+' ? " += " : " -= ")) << value << ";\n";
