@@ -502,7 +502,15 @@ auto Generator::TiledProductPattern(const Sub &s, TiledProductShape &p) const ->
     split(blocks, std::min<long>(3, mostJ), mostJ, envInt("ACRO_HIP_TILED_PRODUCT_PREFER", 4), p.panels, p.TJ);
     // (strips: up to 12 of them, four per workgroup rather than more: 128^3 per entry 57 -> 59 %, 125^3 45 -> 48 %, 192^3
     // 30.5 -> 38 %; from 13 on, as many as possible: 256^3 31.5 against 30.4 %, and the large products without a batch index)
-    split(strips, std::min<long>(4, mostW), mostW, strips <= 12 ? 4 : 8, p.tilesM, p.W);
+    // One panel and many strips (the transposed operator of an interpolation, "Y_e_i = B_q_i U_e_q"): every workgroup has all
+    // columns, so halving its rows costs no second read of the other factor but of the small one, and twice as many
+    // workgroups overlap loads with products (131 072 entries, 125 terms by 64 columns with the product before it 102.2 ->
+    // STRIPS us).
+    const bool skinny = !p.batched && p.panels == 1 && strips > 1024;
+    if (skinny)
+        split(strips, std::min<long>(4, mostW), std::min<long>(4, mostW), 4, p.tilesM, p.W);
+    else
+        split(strips, std::min<long>(4, mostW), mostW, strips <= 12 ? 4 : 8, p.tilesM, p.W);
     // (few workgroups, a product without a batch index of moderate size: tiles of half the height fill the device better;
     // 1 024 x 1 024 x 1 024: 14.5 -> 31.6 TFLOP/s)
     if (p.E * p.tilesM * p.panels < 512 && p.W > 4 && mostW > 4 && envInt("ACRO_HIP_TILED_PRODUCT_HALF") >= 0) split(strips, 4, 4, 4, p.tilesM, p.W);

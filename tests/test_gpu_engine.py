@@ -1513,3 +1513,15 @@ def test_operator_in_blocks_of_rows_whose_rows_are_no_whole_pieces(at, engine, c
         assert np.array_equal(parent.data[1:-1], sign * (X @ B.T).ravel()) and parent.data[0] == parent.data[-1] == -7.0
         parent.MoveToGPU()
         at.synchronize()
+
+
+@pytest.mark.parametrize("rows", [16 * 1024, 16 * 1024 + 1, 16 * 1025 - 3, 16 * 1028 + 5])
+def test_product_of_many_rows_by_one_panel_of_columns(at, engine, rows):
+    # either side of the 1 024 strips from which a workgroup takes four of them; integer values: exact
+    rng = np.random.default_rng(rows)
+    B, U = rng.integers(-3, 4, (125, 64)).astype(np.float64), rng.integers(-3, 4, (rows, 125)).astype(np.float64)
+    Y = at.Tensor(rows, 64)
+    engine("Y_e_i = B_q_i U_e_q", Y, to_tensor(at, B), to_tensor(at, U))
+    assert ("tiles of %d rows x 64 columns" % (64 if rows > 16 * 1024 else 128)) in engine.GetLastImplementation()
+    Y.MoveFromGPU()
+    assert np.array_equal(Y.data, U @ B)
