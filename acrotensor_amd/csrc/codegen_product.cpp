@@ -504,9 +504,9 @@ auto Generator::TiledProductPattern(const Sub &s, TiledProductShape &p) const ->
     // 30.5 -> 38 %; from 13 on, as many as possible: 256^3 31.5 against 30.4 %, and the large products without a batch index)
     // One panel and many strips (the transposed operator of an interpolation, "Y_e_i = B_q_i U_e_q"): every workgroup has all
     // columns, so halving its rows costs no second read of the other factor but of the small one, and twice as many
-    // workgroups overlap loads with products (131 072 entries, 125 terms by 64 columns with the product before it 102.2 ->
-    // STRIPS us).
-    const bool skinny = !p.batched && p.panels == 1 && strips > 1024;
+    // workgroups overlap loads with products (with the product before it, on 131 072 vectors 125 by 64 101.9 -> 101.3 us,
+    // on 130 000 110 by 60 103.2 -> 96.9, 128 by 50 85.2 -> 81.9).
+    const bool skinny = !p.batched && p.panels == 1 && strips > 12;
     if (skinny)
         split(strips, std::min<long>(4, mostW), std::min<long>(4, mostW), 4, p.tilesM, p.W);
     else

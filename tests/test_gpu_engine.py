@@ -1515,13 +1515,13 @@ def test_operator_in_blocks_of_rows_whose_rows_are_no_whole_pieces(at, engine, c
         at.synchronize()
 
 
-@pytest.mark.parametrize("rows", [16 * 1024, 16 * 1024 + 1, 16 * 1025 - 3, 16 * 1028 + 5])
+@pytest.mark.parametrize("rows", [16 * 4096, 16 * 4096 + 1, 16 * 4100 - 3, 70001])
 def test_product_of_many_rows_by_one_panel_of_columns(at, engine, rows):
-    # either side of the 1 024 strips from which a workgroup takes four of them; integer values: exact
+    # strips of 16 rows, four per workgroup: whole workgroups and remainders; integer values: exact
     rng = np.random.default_rng(rows)
     B, U = rng.integers(-3, 4, (125, 64)).astype(np.float64), rng.integers(-3, 4, (rows, 125)).astype(np.float64)
     Y = at.Tensor(rows, 64)
     engine("Y_e_i = B_q_i U_e_q", Y, to_tensor(at, B), to_tensor(at, U))
-    assert ("tiles of %d rows x 64 columns" % (64 if rows > 16 * 1024 else 128)) in engine.GetLastImplementation()
+    assert "tiles of 64 rows x 64 columns" in engine.GetLastImplementation()
     Y.MoveFromGPU()
     assert np.array_equal(Y.data, U @ B)
