@@ -169,7 +169,8 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     const long period = O % 2 == 0 ? O / 2 : O;   // lanes after which the output entries repeat
     const long flatLanes = NTr / period * period;
     const bool pencilForm = outputsFastest && (O <= 16 || (O <= 64 && 2 * loadsPerSlice <= O)) && envInt("ACRO_HIP_RED_PENCIL") >= 0;
-    bool flat = outputsFastest && O >= 2 && flatLanes >= 192 && !big->repeated && big->size == Nc * O &&
+    // (a lane adds the workgroup's partials of one output entry, so no more entries than lanes; more: "wide" below)
+    bool flat = outputsFastest && O >= 2 && O <= NTr && flatLanes >= 192 && !big->repeated && big->size == Nc * O &&
                 big->idx.size() >= s.contr.size() && envInt("ACRO_HIP_RED_FLAT") >= 0 &&
                 (!pencilForm || O > 9 || big->size >= (12L << 20) || envInt("ACRO_HIP_RED_FLAT") > 0);
     for (size_t d = 0; flat && d < s.contr.size(); ++d) flat = has(s.contr, big->idx[d]);

@@ -838,3 +838,18 @@ def test_scratch_tensors_of_one_launch_stay_on_chip_when_a_sum_gather_follows(TE
     assert "U->lds+global" in src and "T1->lds\n" in src
     src = source(alias, "other")
     assert "U->lds\n" in src
+
+
+def test_sums_of_a_stream_take_two_entries_per_lane_only_up_to_one_output_per_lane(TE):
+    """256 lanes add the partials: above 256 outputs every number of them, odd or even, goes to the form with a lane per
+    output and several workgroups side by side (384 to 512 even ones used to divide by zero)."""
+    for outputs in (10, 11, 128, 129, 190, 191, 192, 193, 254, 255, 256, 257, 258, 382, 383, 384, 385, 386, 400, 448, 510, 511, 512, 514, 600):
+        src = TE.GetImplementation("S_i = A_n_i", at.Tensor(outputs), at.Tensor(5000, outputs))
+        even = outputs if outputs % 2 else outputs // 2     # lanes after which a pair's output entries repeat
+        two = outputs <= 256 and 256 // even * even >= 192
+        assert "%d output entries" % outputs in src
+        assert ("two on each" in src) == two and ("256 outputs per workgroup" in src) == (outputs > 256), outputs
+    for kernel, dims, others in (("S_i_j -= A_n_i_j B_n", (20, 20), [(5000,)]), ("S_j_i = A_m_n_i_j", (16, 24), []), ("S_i_j += A_n_i_j", (22, 22), [])):
+        big = (50, 100) + dims if "m" in kernel else (5000,) + dims
+        out = dims[::-1] if kernel.startswith("S_j") else dims
+        assert "256 outputs per workgroup" in TE.GetImplementation(kernel, at.Tensor(*out), at.Tensor(*big), *[at.Tensor(*d) for d in others])

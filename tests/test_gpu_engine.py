@@ -1525,3 +1525,16 @@ def test_product_of_many_rows_by_one_panel_of_columns(at, engine, rows):
     assert "tiles of 64 rows x 64 columns" in engine.GetLastImplementation()
     Y.MoveFromGPU()
     assert np.array_equal(Y.data, U @ B)
+
+
+@pytest.mark.parametrize("outputs", [191, 192, 254, 255, 256, 257, 382, 384, 400, 512, 514])
+def test_sums_of_a_stream_around_the_lanes_of_a_workgroup(at, engine, outputs):
+    # two entries per lane up to 256 outputs, a lane per output above; integer values: exact
+    rng = np.random.default_rng(outputs)
+    A, B = rng.integers(-4, 5, (5001, outputs)).astype(np.float64), rng.integers(-4, 5, 5001).astype(np.float64)
+    S = at.Tensor(outputs)
+    for kernel, expected, inputs in (("S_i = A_n_i", A.sum(axis=0), (A,)), ("S_i -= A_n_i B_n", A.sum(axis=0) - B @ A, (A, B))):
+        engine(kernel, S, *[to_tensor(at, x) for x in inputs])
+        S.MoveFromGPU()
+        assert np.array_equal(S.data, expected), kernel
+        S.MoveToGPU()
