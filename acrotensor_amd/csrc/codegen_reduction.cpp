@@ -207,18 +207,23 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     // 214 / 263 us with the loop unrolled 2 / 4 times).  One lane per (slice, output entry): 8 bytes per lane
     // and load, so up to 512 workgroups and four loads in flight per lane (also swept: 256 - 8 192 workgroups,
     // unroll 1 - 8).
-    long G = (byRows || (wide && Go > 1)) ? std::min<long>(std::max<long>(1, 1024 / Go), std::max<long>(1, Nc / (Sn * 16)))
+    const long G = (byRows || (wide && Go > 1)) ? std::min<long>(std::max<long>(1, 1024 / Go), std::max<long>(1, Nc / (Sn * 16)))
                                           : std::min<long>(pencil ? envInt("ACRO_HIP_RED_GROUPS", 256) : 512,
                                                            std::max<long>(1, Nc / (flat && O <= 64 ? Sn * 2 * kFlatWindows : pencil ? Sn * 4 : (flat ? NTr / O : Sn) * 16)));
     // A sum that a few workgroups read within a microsecond or two is over before a second launch is issued: the
-    // workgroup that finishes last adds the partials in the same launch (see below), and the range is shared out over
-    // at most onePassGroups workgroups for it.  Larger sums keep the second kernel: every arrival at the counter writes
-    // back the L2 of its XCD (256 workgroups: 18.4 us in one launch against 16.3 us in two).
-    // (4 096 slices of 3 x 3 7.6 -> 4.8 us per call, 37 529 of 2 x 3 7.5 -> 5.4, 7 373 of 6 x 4 7.5 -> 5.2; at most 16 or 64
-    // workgroups the same within 0.3 us.)
-    constexpr long onePassGroups = 32, onePassSteps = 4;
-    const bool onePass = !byRows && !wide && O <= 64 && (forced || (G <= onePassGroups * onePassSteps && envInt("ACRO_HIP_ONE_PASS") >= 0));
-    if (onePass && !forced) G = std::min(G, onePassGroups);
+    // workgroup that finishes last adds the partials in the same launch (see below).  Every arrival at the counter writes
+    // back the L2 of its XCD, so the line is a number of shares.  us per call, one launch / two (which take 5.1 to 6.1 from
+    // run to run), on inputs that the caches hold | on others:
+    //   flat     6 x 4 outputs, 16 shares 4.8 / 6.0 | 4.9 / 6.0   32: 5.0 / 6.0 | 5.2 / 6.0   64: 5.3 / 5.9 | 5.7 / 5.9
+    //            95: 6.4 / 5.9 | 6.8 / 5.9   8 x 8, 32: 4.6 / 5.9 | 5.3 / 6.0   64: 5.8 / 6.1 | 6.3 / 6.0   78: 7.1 / 6.1 | 7.8 / 6.1
+    //   others   3 x 3, 4: 4.8 / 6.0 | 5.1 / 6.1   16: 5.4 / 5.9 | 6.0 / 6.0   44: 6.0 / 6.0 | 6.7 / 6.5   127: 7.3 / 6.0 | 9.0 / 8.1
+    //            four rows times a vector, 15: 5.5 / 6.1 | 6.2 / 6.3   8 x 8 outputs of two vectors (a lane adds 64 sums), 7:
+    //            18.8 / 17.8 | 19.3 / 18.4
+    // What is saved is the host's part of a launch: replays of a recorded sequence, which have none, take 0.1 to 0.6 us longer
+    // in one launch (3 x 3, 16 shares 5.2 / 4.8).
+    const long onePassShares = flat ? 32 : 16;
+    const bool onePass = !byRows && !wide && O <= 64 &&
+                         (forced || (G <= onePassShares && (flat || O <= 16) && envInt("ACRO_HIP_ONE_PASS") >= 0));
     // G counts the shares of the contraction range (rows of partials in the scratch buffer); the grid has one
     // workgroup per share and group of outputs.
     const long gridG = G * Go;

@@ -135,9 +135,9 @@
 //                               and product schedules)
 //   ACRO_HIP_RED_ROWS=-1        split contractions of few long rows: all outputs in every workgroup, NT / outputs lanes along a row
 //   ACRO_HIP_ONE_PASS=1|-1      split contractions of up to 64 outputs: the workgroup that finishes last adds the per-workgroup
-//                               partials whatever the size / never (default: where at most 128 workgroups would share the
-//                               range; 256 workgroups 18.4 against 16.3 us: the device-scope release writes back the XCD's
-//                               L2 once per workgroup)
+//                               partials whatever the size / never (default: where few workgroups share the range, see
+//                               EmitReduction; 256 workgroups 18.4 against 16.3 us: the device-scope release writes back the
+//                               XCD's L2 once per workgroup)
 //   ACRO_HIP_RED_FLAT=-1|1      split contractions whose outputs are the fastest dimensions of the big operand: never / always
 //                               two neighbouring entries per lane (default: from ten outputs or 96 MB on)
 //   ACRO_HIP_RED_GROUPS=<n> / ACRO_HIP_RED_UNROLL=<n>

@@ -1,5 +1,7 @@
 """The code generator and the hipRTC compile step run without a device: generate, compile for gfx950 and inspect
 the source of kernels for the five baseline configurations and for the schedule's corner cases."""
+import re
+
 import numpy as np
 import pytest
 
@@ -853,3 +855,25 @@ def test_sums_of_a_stream_take_two_entries_per_lane_only_up_to_one_output_per_la
         big = (50, 100) + dims if "m" in kernel else (5000,) + dims
         out = dims[::-1] if kernel.startswith("S_j") else dims
         assert "256 outputs per workgroup" in TE.GetImplementation(kernel, at.Tensor(*out), at.Tensor(*big), *[at.Tensor(*d) for d in others])
+
+
+def test_small_sums_finish_in_one_launch_without_fewer_workgroups_than_two_launches_have(TE):
+    """One launch only where as many workgroups as the two launches would have are few (sums that 33 to 128 of them share
+    used to run on 32, in up to four times as many steps)."""
+    def schedule(kernel, *dims):
+        src = TE.GetImplementation(kernel, *[at.Tensor(*d) for d in dims])
+        return src.count("__global__"), int(re.search(r"terms split over (\d+) workgroups", src).group(1))
+
+    def stream(i, j, n):
+        return schedule("S_i_j = A_n_i_j B_n", (i, j), (n, i, j), (n,))
+
+    assert stream(3, 3, 4096) == (1, 4) and stream(3, 3, 16 * 1024 + 1023) == (1, 16)
+    assert stream(3, 3, 17 * 1024) == (2, 17) and stream(3, 3, 131000) == (2, 127)
+    assert stream(6, 4, 32 * 168 + 167) == (1, 32) and stream(6, 4, 33 * 168) == (2, 33)      # windows of 21 slices
+    assert stream(8, 8, 32 * 64 + 63) == (1, 32) and stream(8, 8, 33 * 64) == (2, 33)
+    assert schedule("S_i = A_n_i B_n", (1,), (16384, 1), (16384,)) == (1, 16)
+    assert schedule("S_i = A_n_i B_n", (1,), (100000, 1), (100000,)) == (2, 97)
+    assert schedule("S_i = A_i_n B_n", (4,), (4, 16384 + 1000), (17384,)) == (1, 16)
+    assert schedule("S_i = A_i_n B_n", (4,), (4, 17408), (17408,)) == (2, 17)
+    assert schedule("A_i_j = B_e_i C_e_j", (8, 8), (8000, 8), (8000, 8)) == (2, 7)
+    assert schedule("A_i_j = B_e_i C_e_j", (8, 8), (131071, 8), (131071, 8)) == (2, 127)
