@@ -525,8 +525,10 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
 
     // ---- stage 2: add the per-workgroup partials in a fixed order and apply the assignment operator.
     // A second, single-workgroup kernel, or, where few workgroups share the range (onePass above), the workgroup that
-    // arrives last at a device-wide counter: the partials are written by the first wavefront (at most 64 outputs) with
-    // device-scope atomic stores, its first lane counts the arrival with a release, the last workgroup acquires.  The
+    // arrives last at a device-wide counter: the partials are written with device-scope atomic stores, a barrier orders
+    // those of all lanes before lane 0, which counts the arrival with a release; the last workgroup acquires.  (One
+    // wavefront writes them all, at most 64 outputs, and its release would wait for all of them, but nothing in the
+    // language says so: 4 096 slices of 3 x 3 4.77 us per call with the barrier, 4.70 without, other sums the same.)  The
     // counter lies behind the partials in the scratch buffer, which the executor zeroes when it allocates it, and the
     // last workgroup sets it back to zero.
     auto emitFinish = [&](const std::string &load) {
@@ -591,7 +593,7 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     }
     else
     {
-        out << "    if (lane == 0)\n    {\n";
+        out << "    __syncthreads();\n    if (lane == 0)\n    {\n";
         out << "        const unsigned int arrived = __hip_atomic_fetch_add(" << counter << ", 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);\n";
         out << "        isLast = (arrived == " << G - 1 << "u);\n    }\n";
         out << "    __syncthreads();\n";

@@ -877,3 +877,14 @@ def test_small_sums_finish_in_one_launch_without_fewer_workgroups_than_two_launc
     assert schedule("S_i = A_i_n B_n", (4,), (4, 17408), (17408,)) == (2, 17)
     assert schedule("A_i_j = B_e_i C_e_j", (8, 8), (8000, 8), (8000, 8)) == (2, 7)
     assert schedule("A_i_j = B_e_i C_e_j", (8, 8), (131071, 8), (131071, 8)) == (2, 127)
+
+
+@pytest.mark.parametrize("kernel,dims", [("S_i_j = A_n_i_j B_n", ((3, 3), (4096, 3, 3), (4096,))),          # a lane per slice
+                                         ("S_i_j += A_n_i_j B_n", ((6, 4), (4096, 6, 4), (4096,))),         # two entries per lane
+                                         ("S_i = A_i_n B_n", ((4,), (4, 16384), (16384,)))])                # lanes along the rows
+def test_partial_sums_of_all_lanes_are_ordered_before_the_arrival_of_their_workgroup(TE, kernel, dims):
+    src = TE.GetImplementation(kernel, *[at.Tensor(*d) for d in dims])
+    stored, counted = src.index("__hip_atomic_store(&scratch["), src.index("__hip_atomic_fetch_add")
+    assert "__syncthreads();" in src[stored:counted] and "__ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT" in src[counted:counted + 300]
+    last = src.index("if (!isLast) return;")
+    assert "__syncthreads();" in src[counted:last] and src.index("__threadfence();", last) < src.index("__hip_atomic_load(&scratch[")
