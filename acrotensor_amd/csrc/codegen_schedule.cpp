@@ -1111,24 +1111,31 @@ auto Generator::ChooseBatching() -> void
         // 8 -> 14 entries per workgroup, 62.9 -> 74.9 % of the HBM peak; p=4: 2 -> 5 entries in 256 lanes,
         // 67.5 -> 72.0 %), and so do groups whose wavefronts would be mostly idle.
         // So do groups of parallel chains (phases of several kernels, "chains") whose kernels fill about half of their
-        // wavefronts, whatever the pointwise kernels between them do: diffusion apply at p = 4, 6^3 points, two entries in
-        // 256 lanes 86.8 -> 69.0 us.  Chains that fill more keep one entry, and where a phase is then three wavefronts, the
-        // workgroup is three wavefronts too (the fourth had nothing but its share of the pointwise kernel, and kept its
-        // registers): p = 5, 6^3 / 7^3 points 90.9 -> 81.6 / 92.2 -> 70.4 us, p = 6, 7^3 / 8^3 93.3 -> 83.2 / 88.0 -> 83.8.
-        // Full wavefronts keep four (p = 7, 8^3 points 66.5 against 69.5 us).  Phases of six wavefronts run in two passes
-        // of three where no phase is narrower than two and LDS lets four workgroups live on a compute unit (p = 8, 9^3
-        // points 112 -> 83.5 us; a single wavefront in the first and last phase, p = 7, 9^3: 66.9 against 69.1; three
-        // workgroups, p = 7 and 10^3: 940 against 1 110).
+        // wavefronts, whatever the pointwise kernels between them do, from four entries per compute unit on (below, the
+        // device has too few workgroups as it is): diffusion apply at p = 4, 6^3 points, two entries in 256 lanes 83 -> 64 us
+        // with 19 418 elements, 13.3 -> 12.1 with 2 000, 8.3 -> 8.6 with 1 000, 3.8 -> 4.9 with 256.  Chains that fill more
+        // keep one entry, and where a phase is then three wavefronts, the workgroup is three wavefronts too (the fourth had
+        // nothing but its share of the pointwise kernel, and kept its registers): 2^22 points, p = 5 with 6^3 / 7^3 points
+        // 90 -> 81 / 91 -> 73 us, p = 6, 7^3 83 -> 78, p = 4, 7^3 / 8^3 74 -> 65 / 76 -> 68.  Wavefronts that are nearly full keep
+        // four (fill 0.875: p = 5, 8^3 73.6 against 75.7, p = 8, 7^3 and 3 000 elements 36.5 against 39.9), and so do
+        // groups whose first or last kernel is wider than the chains between them, fewer points than coefficients (p = 8,
+        // 6^3 and 3 000 elements 31.2 against 34.3; p = 9, 7^3 42.3 against 48.1; up to a fifth wider is none the worse:
+        // p = 6, 6^3 110 -> 99).  Phases of six wavefronts run in two passes of three where no phase is narrower than two,
+        // their fill makes the second pass short and LDS lets four workgroups live on a compute unit (p = 8, 9^3 points
+        // 112 -> 83 us; fill 0.71, 8^3: 117 against 123; a single wavefront in the first and last phase, p = 7, 9^3: 66.9 against
+        // 69.1; three workgroups, p = 7 and 10^3: 940 against 1 110).
         double chainItems = 0.0, chainLanes = 0.0;
-        long mostWaves = 0, leastWaves = 64;
+        long mostWaves = 0, leastWaves = 64, chainWidth = 1, endWidth = 1;   // (widths: lanes of the widest kernel)
         for (int ph = 0; ph <= subs.back().phase; ++ph)
         {
-            long kernelsHere = 0, waves = 0;
+            long kernelsHere = 0, waves = 0, widest = 0;
             double items = 0.0, lanes = 0.0;
             for (const auto &s : subs)
             {
                 if (s.phase != ph || s.fusedWithPrev) continue;
                 const double weight = static_cast<double>(std::max<long>(1, s.tileCount * s.contrCount));
+                if (ph == 0 || ph == subs.back().phase) endWidth = std::max<long>(endWidth, s.laneCount);
+                widest = std::max<long>(widest, s.laneCount);
                 ++kernelsHere;
                 waves += (s.laneCount + 63) / 64;
                 items += weight * s.laneCount;
@@ -1139,6 +1146,7 @@ auto Generator::ChooseBatching() -> void
             chainItems += items;
             chainLanes += lanes;
             mostWaves = std::max(mostWaves, waves);
+            chainWidth = std::max(chainWidth, widest);
         }
         const bool chains = chainLanes > 0.0 && envInt("ACRO_HIP_PACK_CHAINS") >= 0;
         const double chainFill = chains ? chainItems / chainLanes : 1.0;
@@ -1146,9 +1154,9 @@ auto Generator::ChooseBatching() -> void
             const int firstFit = PlaceLds(1), bothEnds = PlaceLdsFromBothEnds(1);
             return bothEnds > 0 ? std::min(firstFit, bothEnds) : firstFit;
         };
-        const bool threeWide = mostWaves == 3 || (mostWaves == 6 && leastWaves >= 2 && ldsOfOneEntry() <= 160 * 1024 / 8 / 4);
-        if (chains && NB == 1 && NT == 256 && threeWide && chainFill >= 0.54 && chainFill < 0.9) NT = bestNT = 192;
-        const bool wanted = envInt("ACRO_HIP_PACK") > 0 || (envInt("ACRO_HIP_PACK") == 0 && NT != 192 && (NB > 1 || idle < 0.5 || chainFill < 0.54));
+        const bool threeWide = mostWaves == 3 || (mostWaves == 6 && leastWaves >= 2 && chainFill < 0.68 && ldsOfOneEntry() <= 160 * 1024 / 8 / 4);
+        if (chains && NB == 1 && NT == 256 && threeWide && 5 * endWidth <= 6 * chainWidth && chainFill >= 0.54 && chainFill < 0.85) NT = bestNT = 192;
+        const bool wanted = envInt("ACRO_HIP_PACK") > 0 || (envInt("ACRO_HIP_PACK") == 0 && NT != 192 && (NB > 1 || idle < 0.5 || (chainFill < 0.54 && E >= 1024)));
         if (wanted && best >= 1.1 * base)
         {
             NB = bestNB;

@@ -888,3 +888,14 @@ def test_partial_sums_of_all_lanes_are_ordered_before_the_arrival_of_their_workg
     assert "__syncthreads();" in src[stored:counted] and "__ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT" in src[counted:counted + 300]
     last = src.index("if (!isLast) return;")
     assert "__syncthreads();" in src[counted:last] and src.index("__threadfence();", last) < src.index("__hip_atomic_load(&scratch[")
+
+
+@pytest.mark.parametrize("elements,p,q,entries,lanes", [
+    (1024, 4, 6, 2, 256), (1023, 4, 6, 1, 256), (64, 4, 6, 1, 256),                  # two entries from four per compute unit on
+    (64, 5, 6, 1, 192), (64, 5, 7, 1, 192), (64, 4, 8, 1, 192), (64, 6, 6, 1, 192),    # three wavefronts
+    (64, 5, 8, 1, 256), (64, 8, 7, 1, 256),                                          # ... but not where they are nearly full
+    (64, 8, 6, 1, 256), (64, 7, 6, 1, 256), (64, 9, 7, 1, 256),                      # ... nor behind a wider first kernel
+    (64, 8, 9, 1, 192), (64, 8, 8, 1, 256)])                                         # six in two passes, if the second is short
+def test_workgroups_of_parallel_chains(TE, elements, p, q, entries, lanes):
+    src = chain_source(TE, workloads.config5(E=elements, Q=q, P=p + 1), transient=True)
+    assert ", %d per workgroup of %d lanes," % (entries, lanes) in src.splitlines()[1]

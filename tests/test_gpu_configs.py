@@ -97,10 +97,10 @@ def test_config5_diffusion_apply(at, engine, checker, E, Q, P, transient):
             assert rel_err(fetch(tensors, name), expected[name]) <= TOL, name
 
 
-@pytest.mark.parametrize("E,Q,P", [(3, 6, 5), (2, 7, 6), (5, 6, 6), (3, 7, 7), (3, 9, 9), (2, 10, 9), (7, 9, 9)])
+@pytest.mark.parametrize("E,Q,P", [(3, 6, 5), (1025, 6, 5), (2, 7, 6), (5, 6, 6), (3, 7, 7), (3, 9, 9), (2, 10, 9), (7, 9, 9)])
 @pytest.mark.parametrize("transient", [False, True])
 def test_diffusion_apply_with_three_wavefronts_or_two_entries_per_workgroup(at, engine, checker, E, Q, P, transient):
-    # chains that fill about half of their wavefronts (two entries), three wavefronts per phase, phases of six wavefronts in
+    # chains that fill about half of their wavefronts (two entries from 1 024 on), three wavefronts per phase, phases of six wavefronts in
     # two passes, operators of more than 64 entries applied transposed a row at a time
     test_config5_diffusion_apply(at, engine, checker, E, Q, P, transient)
 
