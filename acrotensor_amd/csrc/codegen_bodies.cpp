@@ -612,15 +612,19 @@ auto Generator::EmitUnrolledBody(int k, ForwardMap &forwarded, std::vector<std::
 
 // A transposed stage ("V1_e_i_r_s = B_q_i U_e_q_r_s", tile i, contraction q) reads its scalar operand down the columns when
 // the outputs of the tile are summed one after the other: all rows, 2 registers per entry, would have to be in scalar
-// registers at once (spilled from 81 entries on: mass apply at p = 8, 9^3 points 208 -> 175 us, diffusion apply 125 -> 112,
-// 10^3 133 -> 115; below 64 entries the compiler finds the order, 7 x 7 83 against 93).  Its sums are
-// written term by term instead, a row of the operand at a time (every output's own order of terms, and so its value, is the
-// same).
+// registers at once.  Its sums are written term by term instead, a row of the operand at a time (every output's own order
+// of terms, and so its value, is the same).  Groups do so from 9 outputs per lane on: mass apply at p = 8, 9^3 / 10^3 /
+// 12^3 points 59.3 -> 48.7 / 40.7 -> 39.5 / 36.0 -> 32.8 us on 2^23 points, diffusion apply 66.3 -> 49.2 / 72.8 -> 61.0 /
+// 94.4 -> 87.0 on 2^21; with 8 the compiler finds the order as well (9^3 34.2 / 34.2, 10^3 29.0 / 28.9, diffusion apply at
+// 12^3 70.2 against 72.0), with 7 its order is the better one (7 x 7 83 against 93).  A kernel on its own from
+// 10 on: 14 x 12 applied transposed to 30 000 vectors 6.0 -> 4.6, 12 x 10 4.0 -> 3.6, but 14 x 9 3.4 against 3.8, 15 x 7
+// 3.1 against 3.4 and 14 x 8 on 500 000 18.3 against 20.1.
 auto Generator::InterleaveTile(int k, const std::vector<size_t> &firstLine, std::vector<std::string> &compute) const -> void
 {
     const Sub &s = subs[k];
     const int mode = envInt("ACRO_HIP_INTERLEAVE_TILE");
     if (s.contr.size() != 1 || s.tile.size() != 1 || firstLine.size() < 2 || mode < 0) return;
+    if (mode == 0 && firstLine.size() < (subs.size() > 1 ? 9u : 10u)) return;
     bool downColumns = false;
     for (size_t v = 0; v < s.in.size(); ++v)
     {

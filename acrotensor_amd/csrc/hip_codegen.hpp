@@ -57,7 +57,7 @@
 //                               workgroup would do; -1: never (default: only for groups that batch several entries)
 //   ACRO_HIP_PACK_CHAINS=-1     groups of parallel chains choose batch and workgroup size like other groups
 //   ACRO_HIP_INTERLEAVE_TILE=-1|<n>  transposed stages sum the outputs of a tile one after the other / term by term from operators
-//                               of n entries on (default 64)
+//                               of n entries on (default 64, from 9 outputs in the tile on, 10 for a kernel on its own)
 //   ACRO_HIP_PERSIST=<n>        persistent grid of n workgroups per CU looping over the batch
 //   ACRO_HIP_PIPELINE=1         with ACRO_HIP_PERSIST: streaming inputs stay in registers across iterations and are
 //                               requested one iteration ahead

@@ -899,3 +899,17 @@ def test_partial_sums_of_all_lanes_are_ordered_before_the_arrival_of_their_workg
 def test_workgroups_of_parallel_chains(TE, elements, p, q, entries, lanes):
     src = chain_source(TE, workloads.config5(E=elements, Q=q, P=p + 1), transient=True)
     assert ", %d per workgroup of %d lanes," % (entries, lanes) in src.splitlines()[1]
+
+
+@pytest.mark.parametrize("rows,cols,single,group", [(14, 8, False, False), (14, 9, False, True), (15, 7, False, False), (12, 10, True, True),
+                                                    (10, 8, False, False), (9, 9, False, True), (12, 12, True, True), (6, 10, False, False)])
+def test_transposed_stages_sum_term_by_term_where_it_is_the_faster_order(monkeypatch, rows, cols, single, group):
+    """From 64 entries and 10 outputs per lane on (9 in a group of kernels); otherwise the source is what it is without."""
+    def sources():
+        te = at.TensorEngine("HIP")
+        yield te.GetImplementation("Y_e_i = B_q_i U_e_q", at.Tensor(30000, cols), at.Tensor(rows, cols), at.Tensor(30000, rows))
+        yield chain_source(te, workloads.config4(E=64, Q=rows, P=cols), transient=True)
+
+    chosen = list(sources())
+    monkeypatch.setenv("ACRO_HIP_INTERLEAVE_TILE", "-1")
+    assert [a != b for a, b in zip(chosen, sources())] == [single, group]
