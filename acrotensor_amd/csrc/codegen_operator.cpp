@@ -762,10 +762,18 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
         const long C = sh.comp;
         // (a block of rows: the entries' results lie `stride` apart and start at row `off`)
         const long stride = sh.allRows > 0 ? sh.allRows : rows, off = sh.rowOffset;
-        // Runs of 128 bytes that start anywhere in a 64-byte piece: ordinary stores, which L2 merges; with streaming stores
-        // a piece that two of them share reaches memory twice.  125 x 64 on 131 072 entries and its transpose behind it
-        // 110.0 -> 102.2 us, 115 x 64 108.2 -> 98.8, 110 x 60 109.2 -> 103.2; never slower from 75 x 40 on.
-        const bool streamsHere = streams && (stride % 8 == 0 || envInt("ACRO_HIP_OPERATOR_ODD_ROWS") < 0);
+        // Rows that are no whole 64-byte pieces, results of 26 to 144 MiB: ordinary stores, whose lines the memory-side cache
+        // still holds when the next operation reads them.  The product itself takes a little longer, the two together less:
+        // us, streaming stores -> ordinary ones, inputs and outputs changing, with the transposed product behind it | alone:
+        //   110 x 60, 131 072 entries 103.6 -> 96.6 | 50.6 -> 53.8     65 x 64 69.8 -> 65.2 | 36.7 -> 37.0
+        //   90 x 64 84.4 -> 79.8 | 42.7 -> 44.3     125 x 64, 90 000 82.1 -> 77.3 | 40.1 -> 43.0 (one set of tensors:
+        //   75.5 -> 71.0 | 36.2 -> 36.8), 131 072 102.9 -> 101.5 | 51.2 -> 52.8 (94.0 -> 86.5 | 44.8 -> 45.4),
+        //   30 000 38.0 -> 35.4 | 20.8 -> 22.8
+        // Smaller results stay in the cache either way and larger ones do not: 90 x 64, 30 000 33.3 -> 35.5 | 17.0 -> 18.8;
+        // 65 x 64, 500 000 213.5 -> 219.0 | 115.4 -> 117.5 (one set 94 -> 116); 100 x 50, 300 000 185.3 -> 191.3 | 89.4 -> 92.9.
+        const long resultDoubles = E * stride;
+        const bool readAgain = stride % 8 != 0 && resultDoubles >= (13L << 18) && resultDoubles <= (18L << 20);
+        const bool streamsHere = streams && (!readAgain || envInt("ACRO_HIP_OPERATOR_ODD_ROWS") < 0);
         if (viaStage)
         {
             const int perRound = 4 / stageRounds;   // result registers (entries g + 4 r) per round

@@ -80,6 +80,8 @@
 //                               writes out in whole lines only for a kernel on its own whose lanes each hold a long run of outputs
 //                               (default: also for the last kernel of any group whose store instructions would fill less than
 //                               30 % of the lines they touch).  ACRO_HIP_COPY_OUT_MAX=<doubles per batch entry> (default 2048)
+//   ACRO_HIP_OPERATOR_ODD_ROWS=-1  operators in blocks of rows: results of 26 to 144 MiB in rows that are no multiple of 64 bytes
+//                               keep the streaming hint on their stores, too
 //   ACRO_HIP_COPY_OUT_PLANES=-1 results in planes whose length is no multiple of 64 bytes are stored by the lanes that computed them
 //   ACRO_HIP_ROW_SUMS=-1        an element matrix times an element vector with rows that are no multiple of four doubles, and
 //                               one to three short sums per entry (dot products, row sums), run as written (lanes along the

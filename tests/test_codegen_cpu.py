@@ -913,3 +913,15 @@ def test_transposed_stages_sum_term_by_term_where_it_is_the_faster_order(monkeyp
     chosen = list(sources())
     monkeypatch.setenv("ACRO_HIP_INTERLEAVE_TILE", "-1")
     assert [a != b for a, b in zip(chosen, sources())] == [single, group]
+
+
+def test_operators_in_blocks_of_rows_store_without_the_streaming_hint_only_what_is_read_from_cache_again(TE):
+    def streams(entries, rows, cols):
+        src = TE.GetImplementation("U_e_q = B_q_i X_e_i", at.Tensor(entries, rows), at.Tensor(rows, cols), at.Tensor(entries, cols))
+        assert "operator schedule" in src
+        return "nontemporal_store" in src
+
+    assert not streams(131072, 125, 64) and streams(131072, 120, 64)          # rows of whole 64-byte pieces stream out
+    assert streams(27262, 125, 64) and not streams(27263, 125, 64)            # 13 * 2^18 doubles
+    assert streams(30000, 90, 64) and streams(300000, 65, 64) and streams(200000, 100, 50)
+    assert not streams(18 * 2 ** 20 // 65, 65, 64) and streams(18 * 2 ** 20 // 65 + 1, 65, 64)
