@@ -74,6 +74,7 @@ class Tensor:
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None
+        self._address = 0             # what engine calls pass: a released tensor is refused like a null handle
         if h:
             self._lib.acro_tensor_destroy(h)
 
@@ -208,6 +209,7 @@ class TensorEngine:
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None
+        self._address = 0
         if h:
             self._lib.acro_engine_destroy(h)
 

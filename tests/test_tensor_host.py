@@ -92,3 +92,16 @@ def test_index_mapping_rows_stay_aligned_when_domain_entries_have_no_preimage():
     M.ComputeInverse()
     inv, off = M.inverse
     assert list(off) == [0, 1, 1, 2, 2, 4] and list(inv) == [1, 3, 0, 2]
+
+
+def test_engine_calls_refuse_what_has_been_released():
+    """A tensor or an engine whose handle is gone (released before its last reference) is an error, not a stale address."""
+    A, B, S, te = at.Tensor(4), at.Tensor(4), at.Tensor(4), at.TensorEngine("HIP")
+    B.__del__()
+    with pytest.raises(at.AcroError, match="null"):
+        te("S_i = A_i B_i", S, A, B)
+    with pytest.raises(at.AcroError, match="null"):
+        te("B_i = A_i", B, A)
+    te.__del__()
+    with pytest.raises(at.AcroError, match="null"):
+        te("S_i = A_i", S, A)
