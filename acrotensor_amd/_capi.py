@@ -10,7 +10,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libacrotensor_hip.so")
-CALL_PATH = os.path.join(_HERE, "lib", "_acro_call.so")
+CALL_PATH = os.path.join(_HERE, "lib", "_acro_call" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 c_int_p = ctypes.POINTER(ctypes.c_int)
 c_double_p = ctypes.POINTER(ctypes.c_double)
@@ -90,14 +90,21 @@ _lib = None
 _contract = None
 
 
+def _contract_through_ctypes(engine, kernel, out, inputs):
+    arr = (ctypes.c_void_p * max(1, len(inputs)))(*[t._address for t in inputs])
+    return load().acro_engine_contract(engine, kernel.encode(), out._address, arr, len(inputs))
+
+
 def contract_function():
     """``contract(engine address, kernel string, output, tuple of inputs) -> status``: acro_engine_contract for tensors
-    of acrotensor_amd.api, without ctypes between (csrc/python_call.cpp)."""
+    of acrotensor_amd.api, without ctypes between (csrc/python_call.cpp) where the library was built with this
+    interpreter's headers at hand."""
     global _contract
     if _contract is None:
         load()
         if not os.path.exists(CALL_PATH):
-            raise RuntimeError("_acro_call.so is not built (%s missing): run `make -C acrotensor_amd/csrc`." % CALL_PATH)
+            _contract = _contract_through_ctypes
+            return _contract
         loader = importlib.machinery.ExtensionFileLoader("_acro_call", CALL_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_acro_call", loader))
         loader.exec_module(module)

@@ -1,9 +1,14 @@
 """Host-side Tensor / SliceTensor / IndexMapping semantics through the C ABI (no device needed); expectations of
 the reference's unittest/tensor/test_Tensor.cpp:14-150 and unittest/tensor/test_SliceTensor.cpp:12-100."""
+import importlib.machinery
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
 import acrotensor_amd as at
+from acrotensor_amd import _capi
 
 
 def test_constructor_asserts():
@@ -105,3 +110,32 @@ def test_engine_calls_refuse_what_has_been_released():
     te.__del__()
     with pytest.raises(at.AcroError, match="null"):
         te("S_i = A_i", S, A)
+
+
+def test_engine_calls_do_without_the_extension_module(monkeypatch):
+    # built only where the interpreter's headers are, and only for that interpreter
+    assert _capi.CALL_PATH.endswith(importlib.machinery.EXTENSION_SUFFIXES[0])
+    monkeypatch.setattr(_capi, "CALL_PATH", _capi.CALL_PATH + ".missing")
+    monkeypatch.setattr(_capi, "_contract", None)
+    A, B, S, te = at.Tensor(4), at.Tensor(4), at.Tensor(4), at.TensorEngine("HIP")
+    with pytest.raises(at.AcroError, match="Expected ="):
+        te("S_i", S, A)
+    with pytest.raises(at.AcroError, match="Number of input tensors"):
+        te("S_i = A_i B_i", S, A)
+    te.BeginMultiKernelLaunch()
+    te("S_i = A_i B_i", S, A, B)
+    assert "S_i = A_i B_i" in te.EndMultiKernelLaunchGetImplementation()
+    B.__del__()
+    with pytest.raises(at.AcroError, match="null"):
+        te("S_i = A_i B_i", S, A, B)
+
+
+def test_the_library_builds_without_a_python_installation():
+    csrc = os.path.join(os.path.dirname(_capi.__file__), "csrc")
+
+    def plan(*args):
+        return subprocess.run(["make", "-nB", "-C", csrc, "all"] + list(args), check=True, capture_output=True, text=True).stdout
+
+    without = plan("PYTHON=/nonexistent/python3")
+    assert "libacrotensor_hip.so" in without and "python_call.cpp" not in without
+    assert "_acro_call" + importlib.machinery.EXTENSION_SUFFIXES[0] in plan()
