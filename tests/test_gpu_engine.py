@@ -1539,3 +1539,95 @@ def test_sums_of_a_stream_around_the_lanes_of_a_workgroup(at, engine, outputs):
         S.MoveFromGPU()
         assert np.array_equal(S.data, expected), kernel
         S.MoveToGPU()
+
+
+def test_other_tensors_that_relate_differently_never_take_the_previous_binding(at):
+    """A call on other tensors takes the previous call's variant only if they relate to each other as those did and nothing
+    that is written overlaps anything else.  Every call here follows one on disjoint tensors, which fills the shortcut."""
+    E, half = 1 << 16, 1 << 15
+    rng = np.random.default_rng(3)
+    values = [rng.integers(-5, 6, (E, 8)).astype(np.float64) for _ in range(4)]
+
+    def fresh(k):
+        t = to_tensor(at, values[k])
+        t.MoveToGPU()
+        return t
+
+    def over(parent, first):           # E rows of the parent's device memory behind a host buffer of its own
+        at.synchronize()
+        return at.Tensor(E, 8, hdata=np.zeros((E, 8)), ddata=parent.GetDeviceData() + 64 * first, ongpu=True)
+
+    def fetch(t):
+        t.MoveFromGPU()
+        return t.data.copy()
+
+    # a single kernel: what was compiled for disjoint operands is not what overlapping ones get
+    te = at.TensorEngine("HIP")
+
+    def single(S, A, B, expected):
+        te("S_i_j = A_i_j B_i_j", S, A, B)
+        if expected is not None:
+            assert np.array_equal(fetch(S), expected)
+        return te.GetLastImplementation()
+
+    def disjoint_single():
+        assert "__restrict__ T1" in single(at.Tensor(E, 8), fresh(0), fresh(1), values[0] * values[1])
+
+    disjoint_single()
+    disjoint_single()                  # (through the shortcut)
+    parent = at.Tensor(2 * E, 8)
+    parent.MoveToGPU()
+    A = over(parent, 0)
+    te("A_i_j = B_i_j", A, fresh(2))
+    disjoint_single()
+    assert "__restrict__" not in single(over(parent, half), A, fresh(1), None)     # device memory overlaps, host memory does not
+    disjoint_single()
+    both = to_tensor(at, np.stack([values[0], values[1]]))
+    assert single(at.SliceTensor(both, 0), at.SliceTensor(both, 1), fresh(2), values[1] * values[2])
+    disjoint_single()
+    A = fresh(3)
+    single(at.Tensor(E, 8), A, A, values[3] * values[3])                            # two inputs become one tensor
+    disjoint_single()
+    A = fresh(2)
+    single(A, A, fresh(1), values[2] * values[1])                                   # in place
+    disjoint_single()
+    te("S_i_j = A_i_j A_i_j", at.Tensor(E, 8), A, A)
+    for k, l in ((0, 1), (2, 3), (1, 1)):                                           # one name, two tensors
+        S = at.Tensor(E, 8)
+        te("S_i_j = A_i_j A_i_j", S, fresh(k), fresh(l))
+        assert np.array_equal(fetch(S), values[k] * values[l]), (k, l)
+
+    # a group: what may not be fused runs kernel by kernel, in order
+    te = at.TensorEngine("HIP")
+
+    def group(T, S, A, B, B2=None):
+        te.BeginMultiKernelLaunch()
+        te("T_i_j = A_i_j B_i_j", T, A, B)
+        te("S_i_j = T_i_j B_i_j", S, T, B2 or B)
+        te.EndMultiKernelLaunch()
+        return fetch(T), fetch(S)
+
+    def disjoint_group():
+        T, S = group(at.Tensor(E, 8), at.Tensor(E, 8), fresh(0), fresh(1))
+        assert np.array_equal(T, values[0] * values[1]) and np.array_equal(S, values[0] * values[1] * values[1])
+
+    disjoint_group()
+    disjoint_group()
+    A = over(parent, 0)
+    te("A_i_j = B_i_j", A, fresh(2))
+    disjoint_group()
+    # S lies half-way in A: entries of A that the first kernel reads must not be overwritten before (fused, they would be)
+    T, S = group(at.Tensor(E, 8), over(parent, half), A, fresh(1))
+    assert np.array_equal(T, values[2] * values[1]) and np.array_equal(S, T * values[1])
+    disjoint_group()
+    T, S = group(at.Tensor(E, 8), at.Tensor(E, 8), fresh(0), fresh(1), B2=fresh(3))                # one name, two tensors
+    assert np.array_equal(S, values[0] * values[1] * values[3])
+    disjoint_group()
+    A = fresh(2)
+    T, S = group(at.Tensor(E, 8), A, A, fresh(1))                                                  # the last result replaces the input
+    assert np.array_equal(S, values[2] * values[1] * values[1])
+    disjoint_group()
+    both = to_tensor(at, np.stack([values[0], values[1], values[2]]))
+    T, S = group(at.SliceTensor(both, 0), at.SliceTensor(both, 1), at.SliceTensor(both, 2), fresh(3))
+    assert np.array_equal(S, values[2] * values[3] * values[3])
+    disjoint_group()
