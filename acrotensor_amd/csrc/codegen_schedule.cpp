@@ -790,8 +790,10 @@ auto Generator::ChooseCopyOutTile() -> void
     // two.  An entry's planes are one contiguous range, so they leave through a tile too, of up to 64 KB.  Geometric factors
     // from the Jacobians, planes of 343 doubles: 207 -> 173 us (ordinary stores 180), 125: 43.4 -> 40.7, 729: 264 -> 236;
     // lengths that are such multiples keep their stores: 1 000 441 (through the tile 464), 512 254 (259), 216 166 (171).
-    // (groups; a kernel on its own keeps its stores)
-    bool oddPlanes = subs.size() > 1 && s.laneCount % 8 != 0 && s.laneCount >= 64 && s.out.idx.size() > s.lane.size() && envInt("ACRO_HIP_COPY_OUT_PLANES") >= 0;
+    // Groups only, and results from 6 MB on: before, few workgroups leave the tile's barrier and second pass in the open
+    // (100 elements, 343 points 2.5 against 3.2 us, 729 3.4 against 4.3; 500 elements, 125 points 2.8 against 3.0; from 6 to
+    // 20 MB slower on one set of tensors in the caches, 300 x 9 x 9 planes of 81 5.0 -> 5.4, and faster on changing ones, 6.8 -> 5.5).
+    bool oddPlanes = subs.size() > 1 && E * st.tileSize >= (3L << 18) && s.laneCount % 8 != 0 && s.laneCount >= 64 && s.out.idx.size() > s.lane.size() && envInt("ACRO_HIP_COPY_OUT_PLANES") >= 0;
     for (size_t d = 0; oddPlanes && d < s.lane.size(); ++d) oddPlanes = has(s.lane, s.out.idx[s.out.idx.size() - 1 - d]);
     if (st.tileSize > envInt("ACRO_HIP_COPY_OUT_MAX", oddPlanes ? 8192 : 2048)) return;
     // the run of consecutive outputs of one work item: the trailing output dimensions that are tile indices

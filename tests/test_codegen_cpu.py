@@ -925,3 +925,18 @@ def test_operators_in_blocks_of_rows_store_without_the_streaming_hint_only_what_
     assert streams(27262, 125, 64) and not streams(27263, 125, 64)            # 13 * 2^18 doubles
     assert streams(30000, 90, 64) and streams(300000, 65, 64) and streams(200000, 100, 50)
     assert not streams(18 * 2 ** 20 // 65, 65, 64) and streams(18 * 2 ** 20 // 65 + 1, 65, 64)
+
+
+@pytest.mark.parametrize("points", [5, 7, 9])
+def test_planes_of_odd_length_leave_through_a_tile_from_6_mb_on(TE, points):
+    n = 9 * points ** 3
+    for elements in (100, 786431 // n, 786432 // n + 1, 2000):
+        D, W, C = at.Tensor(elements, 3, 3, points, points, points), at.Tensor(points, points, points), at.Tensor(elements, points, points, points)
+        J, Jinv, Jdet = at.Tensor(elements, points, points, points, 3, 3), at.Tensor(elements, points, points, points, 3, 3), at.Tensor(elements, points, points, points)
+        Jinv.SetTransient(True)
+        Jdet.SetTransient(True)
+        TE.BeginMultiKernelLaunch()
+        TE.BatchMatrixInvDet(Jinv, Jdet, J)
+        TE("D_e_m_n_k1_k2_k3 = W_k1_k2_k3 C_e_k1_k2_k3 Jdet_e_k1_k2_k3 Jinv_e_k1_k2_k3_n_j Jinv_e_k1_k2_k3_m_j", D, W, C, Jdet, Jinv, Jinv)
+        src = TE.EndMultiKernelLaunchGetImplementation()
+        assert ("D: LDS tiles -> device memory" in src) == (elements * n >= 786432), elements

@@ -217,9 +217,10 @@ def test_geometric_factors_at_full_size(at, engine, checker):
                 assert not got[diagonal, a, b].any()
 
 
-@pytest.mark.parametrize("E,Q", [(6, 5), (9, 7), (11, 9), (13, 11)])
+@pytest.mark.parametrize("E,Q", [(6, 5), (701, 5), (9, 7), (257, 7), (121, 9), (13, 11)])
 def test_planes_of_odd_length_leave_through_a_tile(at, engine, checker, E, Q):
-    # 125, 343 and 729 doubles per plane: one contiguous range per entry (1 331: its tile would not fit; the elements are the largest extent, so the batch)
+    # 125, 343 and 729 doubles per plane: one contiguous range per entry (1 331: its tile would not fit; less than 6 MB of them
+    # keep their stores)
     J, W, C = jacobians(np.random.default_rng(E * Q), E, Q, 3)
     tJ, tW, tC = to_tensor(at, J), to_tensor(at, W), to_tensor(at, C)
     Jinv, Jdet, D = at.Tensor(*J.shape), at.Tensor(*C.shape), at.Tensor(E, 3, 3, Q, Q, Q)
@@ -231,6 +232,6 @@ def test_planes_of_odd_length_leave_through_a_tile(at, engine, checker, E, Q):
     engine.BatchMatrixInvDet(Jinv, Jdet, tJ)
     engine(GEOMETRIC_FACTORS[3], D, tW, tC, Jdet, Jinv, Jinv)
     engine.EndMultiKernelLaunch()
-    assert ("D: LDS tiles -> device memory" in engine.GetLastImplementation()) == (Q < 11)
+    assert ("D: LDS tiles -> device memory" in engine.GetLastImplementation()) == (E > 100)
     D.MoveFromGPU()
     assert rel_err(D.data, expected_factors(checker, 3, J, W, C)[2]) <= TOL
