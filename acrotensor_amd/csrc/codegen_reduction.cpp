@@ -163,7 +163,9 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     // 2 000 001 of 6 x 6 122 -> 89 us, 500 001 of 3 x 5
     // 14.4 -> 13.5 us.  Up to nine outputs a pencil is as fast on operands that the memory-side cache can hold (2^20 of
     // 3 x 3 16.1 / 16.0 us, 10^6 of 2 x 2 10.0 / 10.2) and behind beyond (1 705 447 of 2 x 4, 109 MB, 24.6 -> 23.1 us,
-    // 4 000 001 of 2 x 3 43.9 -> 40.0), hence the line at 96 MB.
+    // 4 000 001 of 2 x 3 43.9 -> 40.0), hence the line at 96 MB; with seven or nine at 256 MB (7 outputs, inputs changing:
+    // 130 MB 29.2 / 30.1, 192 MB 40.5 / 40.2, one set of tensors 24.0 / 26.6 and 32.8 / 35.5, 300 MB 60.6 -> 54.9; 9 outputs:
+    // 130 MB 26.5 / 27.8, 192 MB 36.2 / 37.4, 300 MB 53.6 -> 52.4).
     // Four windows are requested before they are added (8: slower), 512 workgroups (256, 1 024, 2 048: slower), fewer for
     // a stream of less than 8 windows each (4: 20 001 slices of 6 x 8 9.2 us, 8: 7.7, the partials being half as many).
     const long period = O % 2 == 0 ? O / 2 : O;   // lanes after which the output entries repeat
@@ -172,7 +174,7 @@ auto Generator::EmitReduction(HipKernelPlan &plan) -> void
     // (a lane adds the workgroup's partials of one output entry, so no more entries than lanes; more: "wide" below)
     bool flat = outputsFastest && O >= 2 && O <= NTr && flatLanes >= 192 && !big->repeated && big->size == Nc * O &&
                 big->idx.size() >= s.contr.size() && envInt("ACRO_HIP_RED_FLAT") >= 0 &&
-                (!pencilForm || O > 9 || big->size >= (12L << 20) || envInt("ACRO_HIP_RED_FLAT") > 0);
+                (!pencilForm || O > 9 || big->size >= (O == 7 || O == 9 ? 32L << 20 : 12L << 20) || envInt("ACRO_HIP_RED_FLAT") > 0);
     for (size_t d = 0; flat && d < s.contr.size(); ++d) flat = has(s.contr, big->idx[d]);
     constexpr int kFlatWindows = 4;               // windows of a workgroup in flight
     const long flatSlices = 2 * flatLanes / O;    // slices per window

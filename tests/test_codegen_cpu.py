@@ -940,3 +940,13 @@ def test_planes_of_odd_length_leave_through_a_tile_from_6_mb_on(TE, points):
         TE("D_e_m_n_k1_k2_k3 = W_k1_k2_k3 C_e_k1_k2_k3 Jdet_e_k1_k2_k3 Jinv_e_k1_k2_k3_n_j Jinv_e_k1_k2_k3_m_j", D, W, C, Jdet, Jinv, Jinv)
         src = TE.EndMultiKernelLaunchGetImplementation()
         assert ("D: LDS tiles -> device memory" in src) == (elements * n >= 786432), elements
+
+
+def test_sums_of_few_outputs_become_one_stream_beyond_what_the_memory_side_cache_holds(TE):
+    def stream(outputs, doubles):
+        n = doubles // outputs
+        return "two on each" in TE.GetImplementation("S_i = A_n_i B_n", at.Tensor(outputs), at.Tensor(n, outputs), at.Tensor(n))
+
+    assert [stream(o, 13 << 20) for o in (3, 5, 6, 7, 8, 9, 10)] == [True, True, True, False, True, False, True]     # 104 MB
+    assert [stream(o, (11 << 20)) for o in (3, 6, 9, 10)] == [False, False, False, True]                             # 88 MB
+    assert stream(7, (32 << 20) + 9) and stream(9, (32 << 20) + 9) and not stream(9, (32 << 20) - 9)
