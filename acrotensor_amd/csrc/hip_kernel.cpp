@@ -219,6 +219,16 @@ HipKernel::HipKernel(const std::string &module_name, const std::string &source,
     }
 }
 
+int RunTimeCompilerVersion()
+{
+    // (hiprtcVersion does not tell releases apart; the runtime of the same release sits beside the compiler)
+    static const int version = [] {
+        int v = 0;
+        return hipRuntimeGetVersion(&v) == hipSuccess ? v / 100000 : 0;
+    }();
+    return version;
+}
+
 HipKernel::~HipKernel()
 {
     if (Module != nullptr) (void)hipModuleUnload(static_cast<hipModule_t>(Module));

@@ -16,6 +16,10 @@
 namespace acro
 {
 
+// Version of the run-time compiler in this process, major * 100 + minor of its ROCm release.  It is the one whose libraries
+// were loaded first: the system's, or those that a framework of the host program brings along.
+int RunTimeCompilerVersion();
+
 class HipKernel
 {
   public:

@@ -1,5 +1,6 @@
 """The code generator and the hipRTC compile step run without a device: generate, compile for gfx950 and inspect
 the source of kernels for the five baseline configurations and for the schedule's corner cases."""
+import ctypes
 import re
 
 import numpy as np
@@ -896,8 +897,9 @@ def test_partial_sums_of_all_lanes_are_ordered_before_the_arrival_of_their_workg
     (64, 5, 8, 1, 256), (64, 8, 7, 1, 256),                                          # ... but not where they are nearly full
     (64, 8, 6, 1, 256), (64, 7, 6, 1, 256), (64, 9, 7, 1, 256),                      # ... nor behind a wider first kernel
     (64, 8, 9, 1, 192), (64, 8, 8, 1, 256)])                                         # six in two passes, if the second is short
-def test_workgroups_of_parallel_chains(TE, elements, p, q, entries, lanes):
-    src = chain_source(TE, workloads.config5(E=elements, Q=q, P=p + 1), transient=True)
+def test_workgroups_of_parallel_chains(monkeypatch, elements, p, q, entries, lanes):
+    monkeypatch.setenv("ACRO_HIP_PACK_CHAINS", "1")
+    src = chain_source(at.TensorEngine("HIP"), workloads.config5(E=elements, Q=q, P=p + 1), transient=True)
     assert ", %d per workgroup of %d lanes," % (entries, lanes) in src.splitlines()[1]
 
 
@@ -950,3 +952,15 @@ def test_sums_of_few_outputs_become_one_stream_beyond_what_the_memory_side_cache
     assert [stream(o, 13 << 20) for o in (3, 5, 6, 7, 8, 9, 10)] == [True, True, True, False, True, False, True]     # 104 MB
     assert [stream(o, (11 << 20)) for o in (3, 6, 9, 10)] == [False, False, False, True]                             # 88 MB
     assert stream(7, (32 << 20) + 9) and stream(9, (32 << 20) + 9) and not stream(9, (32 << 20) - 9)
+
+
+def test_parallel_chains_have_workgroups_of_their_own_with_older_compilers_only(monkeypatch):
+    """From ROCm 7.2 on the compiler fits one entry per workgroup in half the registers, and that is the fastest shape."""
+    runtime = ctypes.CDLL({line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line}.pop())
+    version = ctypes.c_int(0)
+    assert runtime.hipRuntimeGetVersion(ctypes.byref(version)) == 0
+    wl = workloads.config5(E=64, Q=7, P=6)
+    chosen = chain_source(at.TensorEngine("HIP"), wl, transient=True)
+    monkeypatch.setenv("ACRO_HIP_PACK_CHAINS", "1" if version.value // 100000 < 702 else "-1")
+    assert chosen == chain_source(at.TensorEngine("HIP"), wl, transient=True)
+    assert ("workgroup of 192 lanes" in chosen) == (version.value // 100000 < 702)
