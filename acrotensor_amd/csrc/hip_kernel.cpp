@@ -92,7 +92,8 @@ std::string cachePath(const std::string &name, const std::string &source)
     if (dir.empty()) return "";
     int major = 0, minor = 0;
     hiprtcVersion(&major, &minor);
-    std::string salt = std::to_string(major) + "." + std::to_string(minor);
+    // (the release as well: what another release's compiler has left in the directory may be a good deal slower)
+    std::string salt = std::to_string(major) + "." + std::to_string(minor) + "." + std::to_string(RunTimeCompilerVersion());
     for (int i = 0; i < kNumCompileOptions; ++i) salt += std::string(" ") + kCompileOptions[i];
     for (const std::string &option : extraCompileOptions()) salt += " " + option;
     uint64_t h = fnv1a(source, fnv1a(salt + name));

@@ -4,7 +4,7 @@
 //
 // Compilation needs no device, so sources can be generated, compiled and inspected on a machine without a GPU;
 // the code object is loaded into the device on the first launch.  Code objects are cached on disk keyed by a
-// hash of source and options (directory $ACRO_HIP_CACHE_DIR, default $HOME/.cache/acrotensor_hip; set
+// hash of source, options and compiler release (directory $ACRO_HIP_CACHE_DIR, default $HOME/.cache/acrotensor_hip; set
 // ACRO_HIP_CACHE_DIR=off to disable).
 #ifndef ACRO_HIP_KERNEL_HPP
 #define ACRO_HIP_KERNEL_HPP

@@ -1,7 +1,10 @@
 """The code generator and the hipRTC compile step run without a device: generate, compile for gfx950 and inspect
 the source of kernels for the five baseline configurations and for the schedule's corner cases."""
 import ctypes
+import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -964,3 +967,22 @@ def test_parallel_chains_have_workgroups_of_their_own_with_older_compilers_only(
     monkeypatch.setenv("ACRO_HIP_PACK_CHAINS", "1" if version.value // 100000 < 702 else "-1")
     assert chosen == chain_source(at.TensorEngine("HIP"), wl, transient=True)
     assert ("workgroup of 192 lanes" in chosen) == (version.value // 100000 < 702)
+
+
+def test_cached_code_objects_belong_to_one_release_of_the_compiler(tmp_path):
+    """A process that has imported PyTorch compiles with the hipRTC it brings along: another release, another entry."""
+    program = """
+import ctypes, os, sys
+if sys.argv[1]: import torch
+import acrotensor_amd as at
+at.TensorEngine("HIP").GetImplementation("A_i = B_i", at.Tensor(7), at.Tensor(7))
+runtime = ctypes.CDLL({line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line}.pop())
+version = ctypes.c_int(0)
+runtime.hipRuntimeGetVersion(ctypes.byref(version))
+print(version.value // 100000)
+"""
+    env = dict(os.environ, ACRO_HIP_CACHE_DIR=str(tmp_path))
+    root = os.path.dirname(os.path.dirname(os.path.abspath(at.__file__)))
+    releases = {subprocess.run([sys.executable, "-c", program, first], cwd=root, env=env, check=True, capture_output=True, text=True).stdout.split()[-1]
+                for first in ("", "torch", "")}
+    assert len(list(tmp_path.glob("*.hsaco"))) == len(releases)
