@@ -503,9 +503,13 @@ auto Generator::TiledProductPattern(const Sub &s, TiledProductShape &p) const ->
     // (strips: up to 12 of them, four per workgroup rather than more: 128^3 per entry 57 -> 59 %, 125^3 45 -> 48 %, 192^3
     // 30.5 -> 38 %; from 13 on, as many as possible: 256^3 31.5 against 30.4 %, and the large products without a batch index)
     // One panel and many strips (the transposed operator of an interpolation, "Y_e_i = B_q_i U_e_q"): every workgroup has all
-    // columns, so halving its rows costs no second read of the other factor but of the small one, and twice as many
-    // workgroups overlap loads with products (with the product before it, on 131 072 vectors 125 by 64 101.9 -> 101.3 us,
-    // on 130 000 110 by 60 103.2 -> 96.9, 128 by 50 85.2 -> 81.9).
+    // columns, so halving its rows costs no second read of the other factor but of the small one (a chunk at a time, from
+    // L2), and the work is dealt out to the compute units in finer pieces.  us, eight strips -> four, 125 terms by 64
+    // columns on 66 000 / 100 000 / 131 072 / 200 000 / 400 000 rows: 43.2 -> 31.4, 47.7 -> 42.1, 55.4 -> 50.0, 96.7 -> 75.6,
+    // 142 -> 141; 1 000 by 64: 273 -> 190, 286 -> 271, 322 -> 331, 610 -> 516, 933 -> 1 008; 512 by 33: 99 -> 86 on 66 000,
+    // 157 -> 139 on 131 072.  Numbers of rows that divide evenly among eight-strip workgroups lose: 85 000 rows, 128 by 50
+    // 36.9 -> 40.0, 1 000 by 56 215 -> 251; 400 000, 128 by 64 138 -> 147.  Over 442 timings of 66 000 rows and more
+    // and 110 to 2 048 terms the time is 0.94 of eight strips' (0.65 to 1.23), with many terms as with few.
     const bool skinny = !p.batched && p.panels == 1 && strips > 12;
     if (skinny)
         split(strips, std::min<long>(4, mostW), std::min<long>(4, mostW), 4, p.tilesM, p.W);

@@ -1442,7 +1442,8 @@ def test_dense_operator_with_dimensions_in_any_order(at, engine, checker, kernel
 
 
 @pytest.mark.parametrize("kernel,terms,outs,others", [
-    # slices per window are 2 * 252 / 9 = 56: below one window, one exactly, one more, several steps of the unrolled loop
+    # windows of 2 * 252 / 9 = 56 slices: 36 windows and 33 slices, 40 exactly, 41 and one slice, 1 040 (several steps of the
+    # unrolled loop) and 55 slices
     ("S_i_j = A_n_i_j B_n", (2049,), (3, 3), ("n",)), ("S_i_j += A_n_i_j B_n", (56 * 40,), (3, 3), ("n",)),
     ("S_i_j -= A_n_i_j B_n", (56 * 41 + 1,), (3, 3), ("n",)), ("S_i_j = A_n_i_j B_n", (56 * 8 * 130 + 55,), (3, 3), ("n",)),
     ("S_i_j = A_n_i_j B_n", (30011,), (4, 5), ("n",)), ("S_i_j = A_n_i_j B_n", (5003,), (6, 6), ("n",)), ("S_i = A_n_i", (9001,), (2,), ()),
