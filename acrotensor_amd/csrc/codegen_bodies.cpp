@@ -895,6 +895,11 @@ auto Generator::EmitLoopBody(int k, std::vector<std::string> &lines) -> void
         (carried || s.tile.empty() ? order : inner).push_back(c);
     }
     order.insert(order.end(), inner.begin(), inner.end());
+    // One output per lane and fewer lanes than the device holds wavefronts to hide a load behind: bound by the latency of the
+    // loads, so more of them are in flight (3 x 3 sums of a stream, us with 4 / 8 / 16 / 32 / 64: 1 024 terms 39 / 26 / 20 / 18 /
+    // 19, 2 047 terms 112 / 68 / 45 / 41 / 38).  As many as the registers hold with several operands.
+    const bool fewLanes = tc == 1 && E * s.laneCount <= 16384;
+    const std::string unroll = "#pragma unroll " + std::string(!fewLanes ? "4" : (s.in.size() <= 2 ? "32" : (s.in.size() <= 4 ? "16" : "8")));
     std::string indent;
     for (size_t j = 0; j < order.size(); ++j)
     {
@@ -902,7 +907,7 @@ auto Generator::EmitLoopBody(int k, std::vector<std::string> &lines) -> void
         // Around a register tile only the innermost loop is unrolled: with every loop unrolled the compiler requests
         // all scalar operands of all terms at once and spills them.
         if (j + 1 == order.size())
-            lines.push_back(indent + (tc > 1 && extent[order[j]] <= 8 ? "#pragma unroll" : "#pragma unroll 4"));
+            lines.push_back(indent + (tc > 1 && extent[order[j]] <= 8 ? "#pragma unroll" : unroll));
         else if (tc > 1)
             lines.push_back(indent + "#pragma unroll 1");
         lines.push_back(indent + "for (int " + c + " = 0; " + c + " < " + str(extent[order[j]]) + "; ++" + c + ")");

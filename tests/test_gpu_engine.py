@@ -1632,3 +1632,24 @@ def test_other_tensors_that_relate_differently_never_take_the_previous_binding(a
     T, S = group(at.SliceTensor(both, 0), at.SliceTensor(both, 1), at.SliceTensor(both, 2), fresh(3))
     assert np.array_equal(S, values[2] * values[3] * values[3])
     disjoint_group()
+
+
+@pytest.mark.parametrize("kernel,shapes", [
+    ("S_i_j = A_n_i_j B_n", [(1024, 3, 3), (1024,)]), ("S_i_j += A_n_i_j B_n", [(1055, 3, 3), (1055,)]), ("S_i -= A_n_i", [(2047, 100)]),
+    ("S_i = A_n_i B_n C_n_i", [(543, 5), (543,), (543, 5)]), ("S_i = A_n_i B_n C_n_i D_n F_n_i", [(519, 3), (519,), (519, 3), (519,), (519, 3)]),
+    ("S_i = A_n_m_i B_m_n", [(33, 37, 4), (37, 33)]),
+])
+def test_sums_as_counted_loops_of_few_lanes(at, engine, checker, kernel, shapes):
+    """Some hundred terms per lane and few lanes: unrolled by 32, 16 and 8, with remainders of the loop.  Integer values: exact."""
+    rng = np.random.default_rng(shapes[0][0])
+    ins = [rng.integers(-4, 5, s).astype(np.float64) for s in shapes]
+    out0 = rng.integers(-4, 5, output_shape(kernel, shapes)).astype(np.float64)
+    expected = np.zeros_like(out0)
+    checker.contract(kernel.replace("+=", "=").replace("-=", "="), expected, *ins)
+    if kernel.split()[1] != "=":
+        expected = out0 + (expected if "+=" in kernel else -expected)
+    S = to_tensor(at, out0)
+    engine(kernel, S, *[to_tensor(at, a) for a in ins])
+    S.MoveFromGPU()
+    assert "as counted loops" in engine.GetLastImplementation()
+    assert np.array_equal(S.data, expected)
