@@ -245,12 +245,13 @@ __global__ __launch_bounds__(kMatLanes) void batchMatrixKernel(const double *__r
 // 64^3-element degree-3 mesh (plain ids: 46.7 and 61.7 us).
 constexpr unsigned kXcdRun = 32;
 
+template <unsigned RUN>
 __device__ inline unsigned xcdContiguousBlock()
 {
-    constexpr unsigned blk = 8 * kXcdRun;
+    constexpr unsigned blk = 8 * RUN;
     const unsigned b = blockIdx.x;
     if (b >= gridDim.x / blk * blk) return b;
-    return b / blk * blk + (b % 8) * kXcdRun + (b / 8) % kXcdRun;
+    return b / blk * blk + (b % 8) * RUN + (b / 8) % RUN;
 }
 
 __global__ __launch_bounds__(kLanes) void scatterKernel(double *__restrict__ Aout, const double *__restrict__ Ain,
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(kLanes) void scatterKernel2(double *__restrict__ Ao
                                                          const int *__restrict__ M, int range_size)
 {
     const int pairs = range_size / 2;
-    const int base = xcdContiguousBlock() * (kLanes * kScatterPairs) + threadIdx.x;
+    const int base = xcdContiguousBlock<kXcdRun>() * (kLanes * kScatterPairs) + threadIdx.x;
     int2 m[kScatterPairs];
 #pragma unroll
     for (int u = 0; u < kScatterPairs; ++u)
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(kLanes) void scatterKernel2(double *__restrict__ Ao
 
 // Row d of the inverse map lists, in increasing range order, the entries that are added into Aout[d]; summing
 // them front to back reproduces the sequential host scatter-add bit for bit and needs no atomics.
-// A workgroup owns kGatherRows * kLanes consecutive rows.  Their entries are consecutive in the inverse map, so the workgroup
+// A workgroup owns ROWS * kLanes consecutive rows.  Their entries are consecutive in the inverse map, so the workgroup
 // walks that range in chunks: all lanes gather a chunk into LDS (unit-stride reads of the map, eight gathers in
 // flight per lane whatever the row lengths are), then the lane of each row adds the part of its row that lies in
 // the chunk, in row order.  Rows are short on average (2.3 entries for a hexahedral mesh) and uneven (1 to 8), so
@@ -311,23 +312,30 @@ __global__ __launch_bounds__(kLanes) void scatterKernel2(double *__restrict__ Ao
 // then values) behind a barrier.  Lines of mesh nodes that lie on element faces have 3.6 entries per row; with 1 024 rows
 // and chunks of 2 048 those workgroups took two chunks (64^3 hexahedra of degree 3, tensors that exceed the memory-side
 // cache: 59.5 us); 512 rows per chunk of 2 048, or 1 024 per 4 096: 55.2 us; 256 rows: 57.9 us; 2 048 rows: 64 us.
+// Elements of low degree have more entries per row, and 512 rows take two chunks: 256 rows from 2.75 entries per row on the
+// average on (hexahedra of degree 1, 7.8 entries, 2 million elements 66 -> 46 us; degree 2, 3.4 entries, 592 620 elements
+// 69 -> 62 us; degree 3, 2.4 entries, 49 -> 52 us, not taken), and where 512 rows per workgroup leave the device with few
+// workgroups (27 x 30 x 29 elements of degree 2 5.3 -> 3.6 us, 21 x 24 x 23 of degree 3 4.2 -> 3.7 us).
+// Rows of many entries share elements with the rows of the next layer of the mesh, a plane of nodes away, which a run of
+// kXcdRun workgroups leaves to another XCD (degree 1: every value fetched 2.8 times): longer runs there (degree 1 50 -> 46
+// us, degree 2 63 -> 62 us; degrees 3 and 4, 512 rows: the same).
 constexpr int kGatherPerLane = 8;
 constexpr int kGatherChunk = kGatherPerLane * kLanes;
-constexpr int kGatherRows = 2;  // rows per lane
 
+template <int ROWS, unsigned RUN>  // rows per lane, workgroups per XCD and run
 __global__ __launch_bounds__(kLanes) void sumGatherKernel(double *__restrict__ Aout, const double *__restrict__ Ain,
                                                           const int *__restrict__ InvM,
                                                           const int *__restrict__ InvMOff, int domain_size)
 {
     __shared__ double vals[kGatherChunk];
-    const int d0 = xcdContiguousBlock() * (kLanes * kGatherRows);  // first row of this workgroup
+    const int d0 = xcdContiguousBlock<RUN>() * (kLanes * ROWS);  // first row of this workgroup
     if (d0 >= domain_size) return;
-    const int dEnd = d0 + kLanes * kGatherRows < domain_size ? d0 + kLanes * kGatherRows : domain_size;
+    const int dEnd = d0 + kLanes * ROWS < domain_size ? d0 + kLanes * ROWS : domain_size;
     const int first = InvMOff[d0], last = InvMOff[dEnd];
-    int rowBegin[kGatherRows], rowEnd[kGatherRows];
-    double sum[kGatherRows];
+    int rowBegin[ROWS], rowEnd[ROWS];
+    double sum[ROWS];
 #pragma unroll
-    for (int r = 0; r < kGatherRows; ++r)
+    for (int r = 0; r < ROWS; ++r)
     {
         const int d = d0 + r * kLanes + threadIdx.x;
         rowBegin[r] = d < domain_size ? InvMOff[d] : 0;
@@ -351,7 +359,7 @@ __global__ __launch_bounds__(kLanes) void sumGatherKernel(double *__restrict__ A
         for (int u = 0; u < kGatherPerLane; ++u) vals[threadIdx.x + u * kLanes] = a[u];
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kGatherRows; ++r)
+        for (int r = 0; r < ROWS; ++r)
         {
             const int lo = rowBegin[r] > c ? rowBegin[r] : c;
             const int hi = rowEnd[r] < c + n ? rowEnd[r] : c + n;
@@ -360,7 +368,7 @@ __global__ __launch_bounds__(kLanes) void sumGatherKernel(double *__restrict__ A
         __syncthreads();
     }
 #pragma unroll
-    for (int r = 0; r < kGatherRows; ++r)
+    for (int r = 0; r < ROWS; ++r)
     {
         const int d = d0 + r * kLanes + threadIdx.x;
         if (d < domain_size) __builtin_nontemporal_store(sum[r], &Aout[d]);
@@ -477,8 +485,18 @@ void HipGPUOps::FlatIndexedScatter(Tensor &Aout, Tensor &Ain, IndexMapping &M)
 void HipGPUOps::FlatIndexedSumGather(Tensor &Aout, Tensor &Ain, IndexMapping &M)
 {
     const int n = M.GetDomainSize();
-    hipLaunchKernelGGL(sumGatherKernel, dim3(gridFor((static_cast<size_t>(n) + kGatherRows - 1) / kGatherRows)), dim3(kLanes), 0, stream(), Aout.GetDeviceData(),
-                       Ain.GetDeviceData(), M.GetInvMap().GetDeviceData(), M.GetInvMapOffsets().GetDeviceData(), n);
+    const size_t entries = static_cast<size_t>(M.GetRangeSize());
+    auto launch = [&](auto kernel, int rows) {
+        hipLaunchKernelGGL(kernel, dim3(gridFor((static_cast<size_t>(n) + rows - 1) / rows)), dim3(kLanes), 0, stream(),
+                           Aout.GetDeviceData(), Ain.GetDeviceData(), M.GetInvMap().GetDeviceData(),
+                           M.GetInvMapOffsets().GetDeviceData(), n);
+    };
+    if (4 * entries > 11 * static_cast<size_t>(n))
+        launch(sumGatherKernel<1, 128>, 1);
+    else if (n <= 2 * kLanes * 1024)
+        launch(sumGatherKernel<1, kXcdRun>, 1);
+    else
+        launch(sumGatherKernel<2, kXcdRun>, 2);
     ACRO_HIP_CHECK(hipGetLastError());
 }
 

@@ -613,6 +613,22 @@ def test_sum_gather_large_random_map_bit_exact(at, engine, checker):
     assert np.array_equal(out.data, checker.scatter(src, M.map))
 
 
+@pytest.mark.parametrize("domain,entries", [
+    (2 * 256 * 1024, 2.75), (2 * 256 * 1024 + 1, 2.75),      # the line between 256 and 512 rows per workgroup, by rows
+    (2 * 256 * 1024 + 1, 2.7500001), (270001, 7.8)])         # and by entries per row; runs of 128 workgroups and a remainder
+def test_sum_gather_forms_bit_exact(at, engine, checker, domain, entries):
+    rng = np.random.default_rng(domain)
+    rsize = int(np.ceil(domain * entries)) if entries > 2.75 else int(domain * entries)
+    M = at.IndexMapping(domain, rsize)
+    M.map[:] = np.minimum(domain - 1, np.sort(rng.integers(0, domain, rsize)) ^ rng.integers(0, 64, rsize))   # ragged, nearly in order
+    vals = rng.uniform(-1, 1, rsize)
+    acc = at.Tensor(domain)
+    acc.Set(99.0)
+    engine.FlatIndexedSumGather(acc, to_tensor(at, vals), M)
+    acc.MoveFromGPU()
+    assert np.array_equal(acc.data, checker.sum_gather(vals, M.map, domain))
+
+
 @pytest.mark.parametrize("domain,rsize,skew", [(1, 9001, 0), (1030, 3, 0), (2500, 70001, 3), (4099, 4099, 0)])
 def test_scatter_and_sum_gather_ragged_maps_bit_exact(at, engine, checker, domain, rsize, skew):
     # rows of the inverse map from empty to tens of thousands of entries (longer than one staging chunk), domain and
