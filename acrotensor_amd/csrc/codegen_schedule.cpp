@@ -991,9 +991,27 @@ auto Generator::PlaceLdsFromBothEnds(int nb) -> int
     return ceiling;
 }
 
+// A group that writes one tensor, 4 KB and more per batch entry, and reads at most a third of that.
+auto Generator::OneLargeResult() const -> bool
+{
+    std::set<int> written, counted;
+    double stored = 0.0, loaded = 0.0;
+    for (const auto &s : subs)
+    {
+        if (!stores[uvars[s.out.uvar].storage].transient && !uvars[s.out.uvar].isVirtual && written.insert(uvars[s.out.uvar].storage).second)
+            stored += static_cast<double>(s.out.size) / static_cast<double>(E);
+        for (const auto &v : s.in)
+        {
+            if (IsPureInput(v.uvar) && has(v.idx, batch) && counted.insert(v.uvar).second) loaded += static_cast<double>(v.size) / static_cast<double>(E);
+        }
+    }
+    return written.size() == 1 && stored >= 512.0 && stored >= 3.0 * loaded;
+}
+
 auto Generator::ChooseBatching() -> void
 {
     ComputeLdsWishes();
+    bool packed = false;
     long maxLane = 1;
     for (const auto &s : subs) maxLane = std::max(maxLane, s.laneCount);
 
@@ -1165,8 +1183,12 @@ auto Generator::ChooseBatching() -> void
         const bool threeWide = mostWaves == 3 || (mostWaves == 6 && leastWaves >= 2 && chainFill < 0.68 && ldsOfOneEntry() <= 160 * 1024 / 8 / 4);
         if (chains && NB == 1 && NT == 256 && threeWide && 5 * endWidth <= 6 * chainWidth && chainFill >= 0.54 && chainFill < 0.85) NT = bestNT = 192;
         const bool wanted = envInt("ACRO_HIP_PACK") > 0 || (envInt("ACRO_HIP_PACK") == 0 && NT != 192 && (NB > 1 || idle < 0.5 || (chainFill < 0.54 && E >= 1024)));
-        if (wanted && best >= 1.1 * base)
+        // (not one large result per entry and little else to move: its workgroups stream out best with few entries, whatever
+        // their lanes do.  p = 2 mass assembly with 3^3 points, 46 028 elements, us: 3 entries in 256 lanes 62.6, one, which
+        // the rule for such streams below makes two in 512, 46.5)
+        if (wanted && best >= 1.1 * base && !OneLargeResult())
         {
+            packed = NT == 128 && bestNT == 256;
             NB = bestNB;
             NT = bestNT;
         }
@@ -1354,14 +1376,18 @@ auto Generator::ChooseBatching() -> void
     // the upper half idle, which halves the residency.  Measured: p=2 mass assembly 37.2 -> 34.3 us, p=3 mass
     // apply with all intermediates stored 355 -> 335 us; the same change costs the read-dominated p=3 mass
     // apply with transient intermediates 8 % (86.4 -> 93.6 us), hence the condition.
-    if (NT == 128 && !lightWorkgroups && opt.force_nt <= 0 && envInt("ACRO_HIP_NT") <= 0 && batch >= 0)
+    if ((NT == 128 || packed) && !lightWorkgroups && opt.force_nt <= 0 && envInt("ACRO_HIP_NT") <= 0 && batch >= 0)
     {
         double stored = 0.0, loaded = 0.0;
-        std::set<int> counted;
+        std::set<int> counted, results;
         for (int k = 0; k < K; ++k)
         {
             const Sub &s = subs[k];
-            if (StoresToGlobal(k)) stored += static_cast<double>(s.out.size) / static_cast<double>(E);
+            if (StoresToGlobal(k))
+            {
+                stored += static_cast<double>(s.out.size) / static_cast<double>(E);
+                results.insert(uvars[s.out.uvar].storage);
+            }
             for (size_t v = 0; v < s.in.size(); ++v)
             {
                 const Source src = SourceOf(k, static_cast<int>(v));
@@ -1372,25 +1398,59 @@ auto Generator::ChooseBatching() -> void
         }
         if (stored >= 3.0 * loaded && stored > 0.0)
         {
-            NT = 256;
-            // Results that leave through their LDS tiles are written as one contiguous range per tensor and
-            // workgroup.  Twice the batch entries in workgroups of twice the lanes keep as many entries in flight
-            // per CU and make those ranges twice as long (p=3 mass apply with all intermediates stored, 4 entries
-            // in 256 lanes -> 8 in 512: 336 -> 311 us; 8 in 256 lanes 332 us, 16 in 1 024 lanes 331 us).
             bool throughLds = false;
             for (int k = 0; k < K; ++k) throughLds = throughLds || CopiesOutFromLds(k);
-            if (throughLds && NB >= envInt("ACRO_HIP_WRITE_BATCH_FROM", 1) && opt.force_nb <= 0 && envInt("ACRO_HIP_NB") <= 0 && 2L * NB <= E && envInt("ACRO_HIP_WRITE_BATCH") >= 0)
+            // Results that leave through their LDS tiles are written as one contiguous range per tensor and workgroup.
+            // Several of them: powers of two of batch entries, whose ranges start and end on (parts of) lines, up to 16
+            // (whole lines), as far as one pass of 512 lanes and 36 KB of LDS go; few work items take 256 or 128 lanes.  Mass
+            // apply with every intermediate stored on 2^22 degrees of freedom, us, the packing of lanes it replaces ->
+            // this: p = 1, 2^3 points 64 entries in 512 lanes 46.3 -> 42.8 (16 in 128), p = 2, 3^3 28 in 512 48.4 -> 43.4
+            // (16 in 256), 4^3 16 in 256 92.3 -> 88.4 (in 512), p = 4, 5^3 10 in 512 49.0 -> 45.4 (16), 6^3 5 in 256 84.9
+            // -> 75.9 (8 in 512), p = 5, 6^3 7 in 256 46.6 -> 45.5 (8 in 512), 7^3 3 in 256 81.6 -> 74.3 (4 in 512).
+            // Batches that would leave fewer than four workgroups per compute unit keep theirs (p = 5, 6^3 and 4 854 elements
+            // 14.9 / 17.2).
+            long maxLane = 1;
+            for (const auto &s : subs) maxLane = std::max(maxLane, s.laneCount);
+            long entries = 16;
+            std::vector<int> placedBefore;
+            for (const auto &st : stores) placedBefore.push_back(st.ldsOffset);
+            while (entries > 1 && (entries * maxLane > 512 || PlaceLds(static_cast<int>(entries)) > 36 * 1024 / 8)) entries /= 2;
+            for (size_t si = 0; si < stores.size(); ++si) stores[si].ldsOffset = placedBefore[si];
+            if (throughLds && results.size() >= 3 && E >= 1024 * entries && opt.force_nb <= 0 && envInt("ACRO_HIP_NB") <= 0 && envInt("ACRO_HIP_WRITE_BATCH") >= 0)
             {
-                const int wider = PlaceLds(2 * NB);
-                if (wider <= budgetDoubles / 2)
+                NB = static_cast<int>(entries);
+                NT = entries * maxLane >= 160 ? 512 : (entries * maxLane > 64 ? 256 : 128);
+                ldsDoubles = PlaceLds(NB);
+            }
+            // A kernel on its own of many factors that keeps nothing in LDS has its lanes go round instead: powers of two of
+            // batch entries until a workgroup moves 12 KB, in 128 lanes (p = 1 mass assembly with 2^3 points, 524 288
+            // elements, us: 8 entries, half of the lanes idle 58.4, 16 in 128 lanes 47.5, 32 43.3; of two factors, the same
+            // or slower: outer products of 6 x 6 87.4 / 90.3, 10 x 10 matrices scaled per entry 41.5 / 47.5).
+            else if (NT == 128 && !throughLds && ldsDoubles == 0 && subs.size() == 1 && subs[0].in.size() >= 4 && E >= 16384)
+            {
+                entries = 1;
+                while (8.0 * (stored + loaded) * static_cast<double>(entries) < 12288.0 && entries < 64) entries *= 2;
+                if (entries > NB && opt.force_nb <= 0 && envInt("ACRO_HIP_NB") <= 0) NB = static_cast<int>(entries);
+            }
+            // One or two: twice the batch entries in workgroups of twice the lanes keep as many entries in flight per CU
+            // and make the ranges twice as long (p=3 mass apply with all intermediates stored, 4 entries in 256 lanes ->
+            // 8 in 512: 336 -> 311 us; 8 in 256 lanes 332 us, 16 in 1 024 lanes 331 us).
+            else if (NT == 128)
+            {
+                NT = 256;
+                if (throughLds && NB >= envInt("ACRO_HIP_WRITE_BATCH_FROM", 1) && opt.force_nb <= 0 && envInt("ACRO_HIP_NB") <= 0 && 2L * NB <= E && envInt("ACRO_HIP_WRITE_BATCH") >= 0)
                 {
-                    NB *= 2;
-                    NT = 512;
-                    ldsDoubles = wider;
-                }
-                else
-                {
-                    ldsDoubles = PlaceLds(NB);
+                    const int wider = PlaceLds(2 * NB);
+                    if (wider <= budgetDoubles / 2)
+                    {
+                        NB *= 2;
+                        NT = 512;
+                        ldsDoubles = wider;
+                    }
+                    else
+                    {
+                        ldsDoubles = PlaceLds(NB);
+                    }
                 }
             }
         }

@@ -283,6 +283,7 @@ class Generator
     int LdsNeed(const Storage &st, int nb) const { return st.tileSize * (st.staged ? 1 : nb); }
     int PlaceLds(int nb);
     int PlaceLdsFromBothEnds(int nb);
+    bool OneLargeResult() const;
     void ChooseBatching();
     bool EntriesAreFastest() const;
     void ChooseEntriesFastest();

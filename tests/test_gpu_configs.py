@@ -303,3 +303,36 @@ def test_node_vector_to_element_vector_and_back_full_size(at, engine):
     multiplicity = np.bincount(dofs.ravel(), minlength=nodes)
     assert multiplicity.min() == 1 and multiplicity.max() == 8
     assert np.array_equal(back.data, multiplicity * Lv)
+
+
+# workgroups of streams that mostly write: every tensor of a chain stored (powers of two of entries, from 1 024 workgroups
+# on), with a remainder of entries, at the line and below it; one large result; a kernel of many factors without LDS
+@pytest.mark.parametrize("p,q,elements,entries,lanes", [
+    (1, 2, 16384, 16, 128), (1, 2, 16383, 64, 512), (2, 3, 16387, 16, 256), (2, 4, 16397, 16, 512), (4, 5, 16391, 16, 512),
+    (4, 6, 8193, 8, 512), (4, 6, 8191, 5, 256), (5, 7, 4097, 4, 512)])
+def test_stored_chains_in_powers_of_two_of_elements(at, engine, checker, p, q, elements, entries, lanes):
+    wl = workloads.config4(E=elements, Q=q, P=p + 1)
+    tensors = workloads.bind_to_engine(wl, at, transient=False)
+    workloads.launch(wl, engine, tensors)
+    assert "%d per workgroup of %d lanes" % (entries, lanes) in engine.GetLastImplementation()
+    arrays = {n: a.copy() for n, a in wl.arrays.items()}
+    for kernel, out, ins in wl.kernels:                      # contractions of the interface's order, numpy's sums
+        lhs, rhs = kernel.split("=")
+        terms = ["".join(t.split("_")[1:]) for t in rhs.split()]
+        arrays[out] = np.einsum(",".join(terms) + "->" + "".join(lhs.strip().split("_")[1:]), *[arrays[n] for n in ins], optimize=True)
+    for name in ("T1", "T2", "T3", "U", "V1", "V2", "Y"):
+        tensors[name].MoveFromGPU()
+        assert np.abs(tensors[name].data - arrays[name]).max() <= TOL * np.abs(arrays[name]).max(), name
+
+
+@pytest.mark.parametrize("p,q,elements,entries,lanes", [(2, 3, 1001, 2, 512), (1, 2, 16389, 32, 128), (1, 2, 16383, 8, 256)])
+def test_assembly_workgroups(at, engine, p, q, elements, entries, lanes):
+    B = workloads.counter_uniform(3, 0, (q, p + 1), -1.0, 1.0)
+    W = workloads.counter_uniform(3, 1, (elements, q, q, q), 0.5, 1.5)
+    M, tB, tW = at.Tensor(elements, *[p + 1] * 6), at.Tensor(q, p + 1), at.Tensor(*W.shape)
+    tB.data[...], tW.data[...] = B, W
+    engine("M_e_i_j_k_l_m_n = B_q_i B_q_l B_r_j B_r_m B_s_k B_s_n W_e_q_r_s", M, *[tB] * 6, tW)
+    assert "%d per workgroup of %d lanes" % (entries, lanes) in engine.GetLastImplementation()
+    M.MoveFromGPU()
+    expected = np.einsum("qi,ql,rj,rm,sk,sn,eqrs->eijklmn", B, B, B, B, B, B, W, optimize=True)
+    assert np.abs(M.data - expected).max() <= TOL * np.abs(expected).max()
