@@ -1,5 +1,6 @@
 // Kernel code generator, emission of the fused chain kernel: phases, prefetch, item loops, LDS copy-out.
 #include "hip_codegen_impl.hpp"
+#include "hip_kernel.hpp"
 
 namespace acro
 {
@@ -236,6 +237,20 @@ auto Generator::Emit(HipKernelPlan &plan) -> void
     // issued, the first phase starts as soon as its own operands are there instead of after everything that was
     // prefetched (p=7 diffusion apply: 960 -> 943 us).  Only when some later phase prefetches at all.
     const bool firstToo = pipelined || envInt("ACRO_HIP_PREFETCH_FIRST") >= 0;
+    // Several chains in the first phase that fill their wavefronts in part: their loads stand behind two branches each, and
+    // run-time compilers before ROCm 7.2 then hold all that is prefetched through the phases in between (diffusion apply at
+    // p = 4, 6^3 points 97 registers instead of 44, and so on), which costs more wavefronts than the order of the loads
+    // gains: from five values per lane on they stay in their phase.  Inputs changing, 2^22 points, us, prefetched -> in the
+    // phase: p = 4, 6^3 65.9 -> 59.0, p = 5, 6^3 / 7^3 81.2 -> 67.1 / 73.8 -> 61.0, p = 6, 7^3 / 8^3 78.3 -> 67.3 / 86.0 -> 63.3,
+    // p = 8, 9^3 / 10^3 83.5 -> 75.2 / 114.7 -> 73.9; four values, p = 3, 4^3 / 5^3 62.3 / 63.6 and 59.2 / 60.6; whole
+    // wavefronts, p = 7, 8^3 to 10^3, 1 to 3 % slower in the phase.  With 7.2: p = 4, 6^3 59.5 / 59.2, p = 6, 8^3 63.4 / 63.2,
+    // p = 8, 9^3 / 10^3 74.0 / 75.0 and 71.7 / 73.2.
+    bool firstInPart = phases[0].chains.size() > 1 && !pipelined && RunTimeCompilerVersion() < 702;
+    {
+        bool whole = true;
+        for (const Chain &c : phases[0].chains) whole = whole && 10 * c.W >= 9 * ((c.W + 63) / 64 * 64);
+        firstInPart = firstInPart && !whole;
+    }
     // Later phases first (they have the latency to hide), the first phase last, with what is left of the budget.
     std::vector<size_t> phaseOrder;
     for (size_t pi = 1; pi < phases.size(); ++pi) phaseOrder.push_back(pi);
@@ -273,7 +288,7 @@ auto Generator::Emit(HipKernelPlan &plan) -> void
             }
             perLane = std::max(perLane, perPass);
         }
-        if (!ok || perLane == 0 || perLane * ph.passes > prefetchBudget) continue;
+        if (!ok || perLane == 0 || perLane * ph.passes > prefetchBudget || (pi == 0 && firstInPart && perLane >= 5)) continue;
         prefetchBudget -= perLane * ph.passes;
         (pi == 0 ? firstPrefetchDoubles : laterPrefetchDoubles) += perLane * ph.passes;
         ph.prefetched = true;

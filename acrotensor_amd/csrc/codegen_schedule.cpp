@@ -1,6 +1,5 @@
 // Kernel code generator, the schedule: register tiles and lane order, kernels applied in the registers of their producers, phases, LDS tiles and their placement, batch and workgroup size.
 #include "hip_codegen_impl.hpp"
-#include "hip_kernel.hpp"
 
 namespace acro
 {
@@ -1131,24 +1130,13 @@ auto Generator::ChooseBatching() -> void
         // wavefronts (p=2 mass assembly).  Groups that batch anyway take the better packing (p=1 mass apply:
         // 8 -> 14 entries per workgroup, 62.9 -> 74.9 % of the HBM peak; p=4: 2 -> 5 entries in 256 lanes,
         // 67.5 -> 72.0 %), and so do groups whose wavefronts would be mostly idle.
-        // Groups of parallel chains (phases of several kernels, "chains") with a compiler before ROCm 7.2.  Those need twice
-        // the registers for one entry per workgroup (diffusion apply at p = 4, 6^3 points: 97 with ROCm 7.0, which PyTorch
-        // 2.10 brings along, 44 with 7.2), so few wavefronts share a SIMD, and other shapes of workgroup are faster; from 7.2
-        // on, one entry in 256 lanes is (all on 2^22 points, us: two entries at p = 4, 6^3 59 -> 66, three wavefronts at
-        // p = 5, 6^3 / 7^3 65 -> 67 / 61 -> 62, p = 8, 9^3 72 -> 80).  The rest is measured with 7.0:
-        // Kernels that fill about half of their wavefronts, whatever the pointwise kernels between them do, take the better
-        // packing from four entries per compute unit on (below, the device has too few workgroups as it is): p = 4, 6^3
-        // 83 -> 64 with 19 418 elements, 13.3 -> 12.1 with 2 000, 8.3 -> 8.6 with 1 000, 3.8 -> 4.9 with 256.  Chains that
-        // fill more keep one entry, and where a phase is then three wavefronts, the workgroup is three wavefronts too (the
-        // fourth had nothing but its share of the pointwise kernel, and kept its registers): p = 5, 6^3 / 7^3 90 -> 81 /
-        // 91 -> 73, p = 6, 7^3 83 -> 78, p = 4, 7^3 / 8^3 74 -> 65 / 76 -> 68.  Wavefronts that are nearly full keep four (fill
-        // 0.875: p = 5, 8^3 73.6 against 75.7, p = 8, 7^3 and 3 000 elements 36.5 against 39.9), and so do groups whose
-        // first or last kernel is wider than the chains between them, fewer points than coefficients (p = 8, 6^3 and 3 000
-        // elements 31.2 against 34.3; p = 9, 7^3 42.3 against 48.1; up to a fifth wider is none the worse: p = 6, 6^3
-        // 110 -> 99).  Phases of six wavefronts run in two passes of three where no phase is narrower than two, their fill
-        // makes the second pass short and LDS lets four workgroups live on a compute unit (p = 8, 9^3 112 -> 83; fill 0.71,
-        // 8^3: 117 against 123; a single wavefront in the first and last phase, p = 7, 9^3: 66.9 against 69.1; three
-        // workgroups, p = 7 and 10^3: 940 against 1 110).
+        // Groups of parallel chains (phases of several kernels, "chains") can take other shapes as well: two entries where the
+        // chains fill about half of their wavefronts (from four workgroups per compute unit on), and workgroups of three
+        // wavefronts where a phase is three (or six of which the second pass is short and none is narrower than two), none
+        // is nearly full and the first and last kernel are no wider than the chains between them.  Only on request
+        // (ACRO_HIP_PACK_CHAINS=1): one entry in 256 lanes is as fast or faster since the first phase's loads no longer
+        // cost registers throughout (see the prefetch; diffusion apply on 2^22 points, us, these shapes / one entry in 256:
+        // p = 4, 6^3 64.2 / 60.3, p = 5, 6^3 / 7^3 66.1 / 67.9 and 62.8 / 61.3, p = 6, 7^3 69.0 / 67.9, p = 8, 9^3 84.0 / 76.1).
         double chainItems = 0.0, chainLanes = 0.0;
         long mostWaves = 0, leastWaves = 64, chainWidth = 1, endWidth = 1;   // (widths: lanes of the widest kernel)
         for (int ph = 0; ph <= subs.back().phase; ++ph)
@@ -1173,8 +1161,7 @@ auto Generator::ChooseBatching() -> void
             mostWaves = std::max(mostWaves, waves);
             chainWidth = std::max(chainWidth, widest);
         }
-        const int packChains = envInt("ACRO_HIP_PACK_CHAINS");
-        const bool chains = chainLanes > 0.0 && (packChains > 0 || (packChains == 0 && RunTimeCompilerVersion() < 702));
+        const bool chains = chainLanes > 0.0 && envInt("ACRO_HIP_PACK_CHAINS") > 0;
         const double chainFill = chains ? chainItems / chainLanes : 1.0;
         auto ldsOfOneEntry = [&] {
             const int firstFit = PlaceLds(1), bothEnds = PlaceLdsFromBothEnds(1);

@@ -336,3 +336,18 @@ def test_assembly_workgroups(at, engine, p, q, elements, entries, lanes):
     M.MoveFromGPU()
     expected = np.einsum("qi,ql,rj,rm,sk,sn,eqrs->eijklmn", B, B, B, B, B, B, W, optimize=True)
     assert np.abs(M.data - expected).max() <= TOL * np.abs(expected).max()
+
+
+@pytest.mark.parametrize("p,q,elements", [(4, 6, 37), (5, 7, 21), (6, 8, 10), (8, 9, 9), (8, 10, 5), (3, 5, 33)])
+def test_diffusion_with_the_first_phases_loads_in_their_phase(at, checker, monkeypatch, p, q, elements):
+    """The form that run-time compilers before ROCm 7.2 are given for parallel chains in partly filled wavefronts, whichever
+    compiler runs here: only the later phases' inputs are requested ahead."""
+    monkeypatch.setenv("ACRO_HIP_PREFETCH_FIRST", "-1")
+    engine = at.TensorEngine("HIP")
+    wl = workloads.config5(E=elements, Q=q, P=p + 1)
+    tensors = workloads.bind_to_engine(wl, at, transient=True)
+    workloads.launch(wl, engine, tensors)
+    src = engine.GetLastImplementation()
+    assert "streaming inputs of phase 3, requested before" in src and "streaming inputs of phase 0" not in src
+    expected = workloads.run_on_checker(wl, checker)["Y"]
+    assert rel_err(fetch(tensors, "Y"), expected) <= TOL
