@@ -95,21 +95,33 @@ def _contract_through_ctypes(engine, kernel, out, inputs):
     return load().acro_engine_contract(engine, kernel.encode(), out._address, arr, len(inputs))
 
 
+def _call_module():
+    """csrc/python_call.cpp, or None where the library was built without this interpreter's headers at hand."""
+    load()
+    if not os.path.exists(CALL_PATH):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("_acro_call", CALL_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_acro_call", loader))
+    loader.exec_module(module)
+    return module
+
+
 def contract_function():
     """``contract(engine address, kernel string, output, tuple of inputs) -> status``: acro_engine_contract for tensors
-    of acrotensor_amd.api, without ctypes between (csrc/python_call.cpp) where the library was built with this
-    interpreter's headers at hand."""
+    of acrotensor_amd.api, without ctypes between where that is built."""
     global _contract
     if _contract is None:
-        load()
-        if not os.path.exists(CALL_PATH):
-            _contract = _contract_through_ctypes
-            return _contract
-        loader = importlib.machinery.ExtensionFileLoader("_acro_call", CALL_PATH)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_acro_call", loader))
-        loader.exec_module(module)
-        _contract = module.contract
+        module = _call_module()
+        _contract = module.contract if module else _contract_through_ctypes
     return _contract
+
+
+def capture_functions():
+    """``begin(engine address) -> status`` and ``end(engine address) -> status``: the entry points around a multi-kernel
+    launch, likewise."""
+    module = _call_module()
+    lib = load()
+    return (module.begin, module.end) if module else (lib.acro_engine_begin_multi_kernel_launch, lib.acro_engine_end_multi_kernel_launch)
 
 
 def load():

@@ -204,6 +204,7 @@ class TensorEngine:
         self._lib = _capi.load()
         self._h = ctypes.c_void_p()
         self._contract = _capi.contract_function()
+        self._begin, self._end = _capi.capture_functions()
         _check(self._lib.acro_engine_create(exec_type.encode(), ctypes.byref(self._h)))
         self._address = self._h.value
 
@@ -241,10 +242,12 @@ class TensorEngine:
             self._h, buf, size, needed))
 
     def BeginMultiKernelLaunch(self):
-        _check(self._lib.acro_engine_begin_multi_kernel_launch(self._h))
+        if self._begin(self._address):
+            _check(1)
 
     def EndMultiKernelLaunch(self):
-        _check(self._lib.acro_engine_end_multi_kernel_launch(self._h))
+        if self._end(self._address):
+            _check(1)
 
     def EndMultiKernelLaunchGetImplementation(self):
         """End the capture without executing it; returns the fused kernel's source (needs no device)."""

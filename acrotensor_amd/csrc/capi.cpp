@@ -399,8 +399,23 @@ int acro_engine_contract(acro_engine *e, const char *kernel, acro_tensor *out, a
 {
     return guarded([&] {
         require(e != nullptr && kernel != nullptr && out != nullptr, "null argument");
-        std::vector<Tensor *> in = unwrap(inputs, num_inputs);
-        e->te(std::string(kernel), out->t, in);
+        Tensor *few[8];
+        std::vector<Tensor *> many;
+        Tensor **in = few;
+        if (num_inputs < 0 || num_inputs > 8 || inputs == nullptr)
+        {
+            many = unwrap(inputs, num_inputs);
+            in = many.data();
+        }
+        else
+        {
+            for (int i = 0; i < num_inputs; ++i)
+            {
+                require(inputs[i] != nullptr, "null tensor handle");
+                few[i] = inputs[i]->t;
+            }
+        }
+        e->te.Contract(kernel, out->t, in, static_cast<size_t>(num_inputs));
         // The call that must not allocate requires this one to have run first on the device; the address of its
         // scratch array is looked up here, where loading code and allocating is allowed.
         if (!e->te.InMultiKernelLaunch()) resolveNoAllocScratch();

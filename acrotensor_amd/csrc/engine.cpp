@@ -141,8 +141,61 @@ void TensorEngine::ResetCapture()
 {
     MKLKernels.clear();
     MKLOutputT.clear();
+    for (auto &list : MKLInputT)
+    {
+        if (SpareInputs.size() >= 64) break;
+        list.clear();
+        SpareInputs.push_back(std::move(list));
+    }
     MKLInputT.clear();
     MKLMatrixOps.clear();
+}
+
+void TensorEngine::Contract(const char *kernel_str, Tensor *output, Tensor *const *inputs, size_t num_inputs)
+{
+    DimensionedKernel *kernel = IsMultiKernelLaunch ? RecordedBefore(kernel_str, output, inputs, num_inputs) : nullptr;
+    if (kernel == nullptr)
+    {
+        std::vector<Tensor *> list(inputs, inputs + num_inputs);
+        (*this)(std::string(kernel_str), output, list);
+        return;
+    }
+    MKLKernels.push_back(kernel);
+    MKLOutputT.push_back(output);
+    if (SpareInputs.empty())
+        MKLInputT.emplace_back();
+    else
+    {
+        MKLInputT.push_back(std::move(SpareInputs.back()));
+        SpareInputs.pop_back();
+    }
+    MKLInputT.back().assign(inputs, inputs + num_inputs);
+}
+
+// The dimensioned kernel of a call at this position of an earlier capture that had this kernel string and tensors of
+// these ranks and extents (they passed the checks of GetAddDimensionedKernel then).
+DimensionedKernel *TensorEngine::RecordedBefore(const char *kernel_str, Tensor *output, Tensor *const *inputs, size_t num_inputs)
+{
+    const size_t position = MKLKernels.size();
+    if (position >= LastRecorded.size()) return nullptr;
+    const RecordedCalls &calls = LastRecorded[position];
+    for (int way = 0; way < 4; ++way)
+    {
+        if (calls.resolved[way].kernel == nullptr || calls.kernel_str[way] != kernel_str) continue;
+        const std::vector<int> &dims = calls.resolved[way].dims;
+        size_t i = 0;
+        auto same = [&](const Tensor *t) {
+            const std::vector<int> &d = t->GetDims();
+            if (!t->IsInitialized() || i + 1 + d.size() > dims.size() || dims[i] != static_cast<int>(d.size())) return false;
+            if (!std::equal(d.begin(), d.end(), dims.begin() + i + 1)) return false;
+            i += 1 + d.size();
+            return true;
+        };
+        bool all = same(output);
+        for (size_t v = 0; v < num_inputs && all; ++v) all = same(inputs[v]);
+        if (all && i == dims.size()) return calls.resolved[way].kernel;
+    }
+    return nullptr;
 }
 
 void TensorEngine::operator()(const std::string &kernel_str, Tensor *output, std::vector<Tensor *> &inputs)
@@ -160,7 +213,19 @@ void TensorEngine::operator()(const std::string &kernel_str, Tensor *output, std
     MKLOutputT.push_back(output);
     MKLInputT.push_back(inputs);
 
-    if (!IsMultiKernelLaunch)
+    if (IsMultiKernelLaunch)
+    {
+        const size_t position = MKLKernels.size() - 1;
+        if (position < 256)
+        {
+            if (LastRecorded.size() <= position) LastRecorded.resize(position + 1);
+            RecordedCalls &calls = LastRecorded[position];
+            calls.kernel_str[calls.next] = kernel_str;
+            calls.resolved[calls.next] = LastDimensioned[kernel];
+            calls.next = (calls.next + 1) % 4;
+        }
+    }
+    else
     {
         LastExecutor = GetAddKernelExecutor();
         LastExecutor->ExecuteSingle(output, inputs);
@@ -330,6 +395,15 @@ class NotTransient
 
 void TensorEngine::FinishCapture(std::string *implementation)
 {
+    // Kernels and nothing else: one group, as recorded.
+    if (implementation == nullptr && MKLMatrixOps.empty() && !MKLKernels.empty())
+    {
+        LastExecutor = GetAddKernelExecutor();
+        LastExecutor->SetGatheredInputs({});
+        LastExecutor->ExecuteMulti(MKLOutputT, MKLInputT);
+        ResetCapture();
+        return;
+    }
     std::vector<DimensionedKernel *> kernels;
     std::vector<Tensor *> outputs;
     std::vector<std::vector<Tensor *>> inputs;
@@ -722,6 +796,7 @@ void TensorEngine::Clear()
     Ops = nullptr;
     LastExecutor = nullptr;
     LastDimensioned.clear();
+    LastRecorded.clear();
     LastCapture.clear();
     LastCaptureExecutor = nullptr;
     ResetCapture();

@@ -276,7 +276,16 @@ class HipExecutor : public KernelExecutor
         gathered.swap(Gathered);  // this call only
         // a gathered operand is the result of a scatter: nothing to copy to the device for it
         for (const auto &g : gathered) g.operand->SwitchToGPU();
-        for (int ki = 0; ki < K; ++ki) MoveTensorsToGPU(outputs[ki], inputs[ki]);
+        // One tensor per variable (the usual case): what follows looks at each of them once, not at every occurrence.
+        const bool plain = CollectOperands(outputs, inputs);
+        if (plain)
+        {
+            for (Tensor *t : Operands) t->MoveToGPU();
+        }
+        else
+        {
+            for (int ki = 0; ki < K; ++ki) MoveTensorsToGPU(outputs[ki], inputs[ki]);
+        }
 
         // The same tensors in the same places as in the previous call, with the same buffers and marks: the same
         // binding, and the variant it led to (the usual case inside a solver's loop; the analysis below costs several
@@ -305,12 +314,27 @@ class HipExecutor : public KernelExecutor
             for (int d = 0; d < root->GetRank(); ++d) s.root_shape = (s.root_shape ^ static_cast<unsigned>(root->GetDim(d))) * 1099511628211ull;
             ThisCall.push_back(s);
         };
-        for (int ki = 0; ki < K; ++ki)
+        if (plain)
         {
-            note(outputs[ki]);
-            for (const Tensor *t : inputs[ki]) note(t);
+            for (const Tensor *t : Operands) note(t);
         }
-        const bool repeated = gathered.empty() && LastCallVariant != nullptr && (ThisCall == LastCall || SameBinding());
+        else
+        {
+            for (int ki = 0; ki < K; ++ki)
+            {
+                note(outputs[ki]);
+                for (const Tensor *t : inputs[ki]) note(t);
+            }
+        }
+        // (which variable each gathered operand is: what of it the analysis depends on)
+        GatheredVars.clear();
+        for (const auto &g : gathered)
+        {
+            const auto at = std::find(Operands.begin(), Operands.end(), g.operand);
+            GatheredVars.push_back(at != Operands.end() ? static_cast<int>(at - Operands.begin()) : -1);
+        }
+        const bool repeated = LastCallVariant != nullptr && plain == LastPlain && (plain || gathered.empty()) &&
+                              GatheredVars == LastGatheredVars && (ThisCall == LastCall || SameBinding());
         HipCodegenOptions options;
         if (!repeated)
         {
@@ -333,33 +357,41 @@ class HipExecutor : public KernelExecutor
             KernelExecutor::ExecuteMulti(outputs, inputs);
             return;
         }
-        if (gathered.empty())
+        if (plain || gathered.empty())
         {
             LastCall.swap(ThisCall);
             LastCallVariant = &v;
-            if (!repeated) NoteBinding(options);
+            LastPlain = plain;
+            LastGatheredVars.swap(GatheredVars);
+            if (repeated)
+                options.gathered = LastGathered;
+            else
+            {
+                LastGathered = options.gathered;
+                NoteBinding(options);
+            }
         }
         MaterialiseGathered(gathered, v.plan.gathers_applied ? &options.gathered : nullptr);
-        std::vector<const int *> gatherMap(gathered.size(), nullptr);
-        std::vector<const double *> gatherSource(gathered.size(), nullptr);
+        GatherMap.assign(gathered.size(), nullptr);
+        GatherSource.assign(gathered.size(), nullptr);
         if (v.plan.gathers_applied)
         {
             for (size_t g = 0; g < gathered.size(); ++g)
             {
                 gathered[g].source->MoveToGPU();
                 gathered[g].map->MoveToGPU();
-                gatherMap[g] = gathered[g].map->GetMap().GetDeviceData();
-                gatherSource[g] = gathered[g].source->GetDeviceData();
+                GatherMap[g] = gathered[g].map->GetMap().GetDeviceData();
+                GatherSource[g] = gathered[g].source->GetDeviceData();
             }
         }
         const size_t nparam = v.plan.param_occurrence.size();
-        std::vector<double *> ptr(nparam);
+        Pointers.resize(nparam);
         for (size_t i = 0; i < nparam; ++i)
         {
             const auto &occ = v.plan.param_occurrence[i];
-            ptr[i] = (occ.second < 0 ? outputs[occ.first] : inputs[occ.first][occ.second])->GetDeviceData();
-            ACROBATIC_ASSERT(ptr[i] != nullptr, "Tensor has no device memory.");
-            ptr[i] -= v.plan.param_offset[i];
+            Pointers[i] = (occ.second < 0 ? outputs[occ.first] : inputs[occ.first][occ.second])->GetDeviceData();
+            ACROBATIC_ASSERT(Pointers[i] != nullptr, "Tensor has no device memory.");
+            Pointers[i] -= v.plan.param_offset[i];
         }
         double *scratch = nullptr;
         if (v.plan.scratch_doubles > 0 && hip::NoAllocation::Active())
@@ -380,30 +412,68 @@ class HipExecutor : public KernelExecutor
         }
         for (const auto &z : v.plan.zero_fills)
         {
-            hip::FillDouble(ptr[z.param] + z.offset, 0.0, static_cast<size_t>(z.count));
+            hip::FillDouble(Pointers[z.param] + z.offset, 0.0, static_cast<size_t>(z.count));
         }
         for (const HipLaunch &launch : v.plan.launches)
         {
-            std::vector<void *> args(launch.params.size());
-            for (size_t i = 0; i < args.size(); ++i)
+            Arguments.resize(launch.params.size());
+            for (size_t i = 0; i < Arguments.size(); ++i)
             {
                 const int code = launch.params[i];
                 if (code >= 0)
-                    args[i] = static_cast<void *>(&ptr[code]);
+                    Arguments[i] = static_cast<void *>(&Pointers[code]);
                 else if (code == -1)
-                    args[i] = static_cast<void *>(&scratch);
+                    Arguments[i] = static_cast<void *>(&scratch);
                 else if ((-code - 2) % 2 == 0)
-                    args[i] = static_cast<void *>(&gatherMap[(-code - 2) / 2]);
+                    Arguments[i] = static_cast<void *>(&GatherMap[(-code - 2) / 2]);
                 else
-                    args[i] = static_cast<void *>(&gatherSource[(-code - 2) / 2]);
+                    Arguments[i] = static_cast<void *>(&GatherSource[(-code - 2) / 2]);
             }
-            v.kernel->Launch(launch.function_name, launch.grid, launch.grid_y, launch.block, args.data());
+            v.kernel->Launch(launch.function_name, launch.grid, launch.grid_y, launch.block, Arguments.data());
         }
+    }
+
+    // Fills Operands with the tensor of every variable; false where occurrences of one variable are different tensors.
+    bool CollectOperands(const std::vector<Tensor *> &outputs, const std::vector<std::vector<Tensor *>> &inputs)
+    {
+        const int K = MultiKernel->GetNumKernels();
+        if (OccurrenceVars.empty())
+        {
+            for (int ki = 0; ki < K; ++ki)
+            {
+                for (int vari = -1; vari < MultiKernel->Kernels[ki]->GetNumInputVars(); ++vari) OccurrenceVars.push_back(MultiKernel->GetUVari(ki, vari));
+            }
+        }
+        Operands.assign(MultiKernel->GetNumUVars(), nullptr);
+        size_t i = 0;
+        auto take = [&](Tensor *t) {
+            Tensor *&operand = Operands[OccurrenceVars[i++]];
+            if (operand == nullptr) operand = t;
+            return operand == t;
+        };
+        for (int ki = 0; ki < K; ++ki)
+        {
+            if (i + 1 + inputs[ki].size() > OccurrenceVars.size() || !take(outputs[ki])) return false;
+            for (Tensor *t : inputs[ki])
+            {
+                if (!take(t)) return false;
+            }
+        }
+        return i == OccurrenceVars.size();
     }
 
     std::map<std::string, std::unique_ptr<Variant>> Variants;
     Variant *LastVariant = nullptr;
-    // one entry per tensor of a call, in call order
+    std::vector<int> OccurrenceVars;   // the variable of every occurrence, in call order
+    std::vector<Tensor *> Operands;    // this call's tensor of every variable
+    bool LastPlain = false;            // the previous call's entries below are one per variable, not per occurrence
+    std::vector<int> GatheredVars, LastGatheredVars;
+    std::vector<int> LastGathered;     // HipCodegenOptions::gathered of the previous call
+    std::vector<double *> Pointers;    // arguments of the launches
+    std::vector<void *> Arguments;
+    std::vector<const int *> GatherMap;
+    std::vector<const double *> GatherSource;
+    // one entry per variable of a call, or per tensor in call order where a variable's occurrences differ
     struct Seen
     {
         const Tensor *tensor, *root;
@@ -458,12 +528,20 @@ class HipExecutor : public KernelExecutor
             if (LastRelations.back().root == static_cast<int>(i)) LastRoots.push_back(static_cast<int>(i));
         }
         WrittenRoots.assign(LastRoots.size(), 0);
-        size_t i = 0;
-        for (int ki = 0; ki < MultiKernel->GetNumKernels(); i += 1 + MultiKernel->Kernels[ki]->GetNumInputVars(), ++ki)
-        {
-            const int root = LastRelations[i].root;   // occurrence i is the output of kernel ki
+        auto written = [&](size_t entry) {
+            const int root = LastRelations[entry].root;
             WrittenRoots[std::find(LastRoots.begin(), LastRoots.end(), root) - LastRoots.begin()] = 1;
+        };
+        if (LastPlain)
+        {
+            for (size_t u = 0; u < LastCall.size(); ++u)
+            {
+                if (MultiKernel->IsOutputUVar(static_cast<int>(u))) written(u);
+            }
+            return;
         }
+        size_t i = 0;
+        for (int ki = 0; ki < MultiKernel->GetNumKernels(); i += 1 + MultiKernel->Kernels[ki]->GetNumInputVars(), ++ki) written(i);
     }
 
     // Whether this call's tensors lead to the previous call's variant without the analysis.

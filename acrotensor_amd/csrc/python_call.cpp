@@ -1,7 +1,8 @@
-// The engine call of the Python mirror (acrotensor_amd/api.py) as a CPython function over the C ABI.  A program that goes
+// The engine call of the Python mirror (acrotensor_amd/api.py), and the two that open and close a multi-kernel launch, as
+// CPython functions over the C ABI.  A program that goes
 // through ctypes pays for every argument's conversion; a solver on a small batch issues its kernels faster than that (a
-// mass apply of seven recorded kernels takes 2 us on the device).  Per recorded kernel, the C ABI's own 0.4 us included:
-// 2.2 us through ctypes, 0.55 us here (both measured on one host).
+// mass apply of seven recorded kernels takes 2 us on the device).  Per recorded kernel of a capture that is repeated, the C
+// ABI's own 0.1 us included: 0.3 us, and 1.9 us through ctypes (both measured on one host).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -56,7 +57,22 @@ PyObject *contract(PyObject *, PyObject *const *args, Py_ssize_t count)
     return PyLong_FromLong(status);
 }
 
+// begin(engine address), end(engine address) -> status of acro_engine_begin_ / _end_multi_kernel_launch
+template <int (*ENTRY)(acro_engine *)>
+PyObject *capture(PyObject *, PyObject *address)
+{
+    acro_engine *engine = static_cast<acro_engine *>(PyLong_AsVoidPtr(address));
+    if (engine == nullptr && PyErr_Occurred() != nullptr) return nullptr;
+    int status = 0;
+    Py_BEGIN_ALLOW_THREADS
+    status = ENTRY(engine);
+    Py_END_ALLOW_THREADS
+    return PyLong_FromLong(status);
+}
+
 PyMethodDef methods[] = {
+    {"begin", capture<acro_engine_begin_multi_kernel_launch>, METH_O, nullptr},
+    {"end", capture<acro_engine_end_multi_kernel_launch>, METH_O, nullptr},
     {"contract", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(contract)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -41,6 +41,8 @@ class TensorEngine
         (*this)(kernel_str, &out, inputs);
     }
     void operator()(const std::string &kernel_str, Tensor *out, std::vector<Tensor *> &inputs);
+    // The same for callers that hold the string and the tensors as plain arrays (the C ABI).
+    void Contract(const char *kernel_str, Tensor *output, Tensor *const *inputs, size_t num_inputs);
 
     template <typename... In>
     std::string GetImplementation(const std::string &kernel_str, Tensor &out, Tensor &in1, In &...more)
@@ -117,6 +119,17 @@ class TensorEngine
         DimensionedKernel *kernel = nullptr;
     };
     std::unordered_map<const TensorKernel *, DimensionedMemo> LastDimensioned;
+    // What was recorded last at each position of a capture (up to four different calls): captures that are repeated, with
+    // the same kernel strings and extents, find their dimensioned kernels there without looking the strings up.
+    struct RecordedCalls
+    {
+        std::string kernel_str[4];
+        DimensionedMemo resolved[4];
+        int next = 0;  // the one to give way
+    };
+    std::vector<RecordedCalls> LastRecorded;
+    DimensionedKernel *RecordedBefore(const char *kernel_str, Tensor *output, Tensor *const *inputs, size_t num_inputs);
+    std::vector<std::vector<Tensor *>> SpareInputs;  // emptied lists of inputs, kept for their memory
     std::vector<int> DimsOfThisCall;
     std::vector<DimensionedKernel *> LastCapture;
     KernelExecutor *LastCaptureExecutor = nullptr;

@@ -232,3 +232,70 @@ def test_mesh_operator_in_one_capture_with_the_sum_gather(at, engine, checker, a
     if after:
         out.MoveFromGPU()
         assert rel_err(out.data, expected[after]) <= TOL
+
+
+def test_repeated_captures_bind_what_each_of_them_was_given(at, engine, checker):
+    """Captures with a scatter over and over: other vectors, maps, marks and operands, none of which may be the last one's."""
+    rng = np.random.default_rng(9)
+    nodes, E, n = 300, 41, 8
+    vectors = [rng.uniform(-1, 1, nodes) for _ in range(2)]
+    maps = []
+    for k in range(2):
+        M = at.IndexMapping(nodes, E * n)
+        M.map[:] = rng.integers(0, nodes, E * n)
+        maps.append(M)
+    W = rng.uniform(-1, 1, (E, n))
+    L, tW, X, A, R = [to_tensor(at, v) for v in vectors], to_tensor(at, W), at.Tensor(E, n), at.Tensor(E), at.Tensor(E, n)
+    resident = rng.uniform(-1, 1, (E, n))
+    steps = [(0, 0, True), (0, 0, True), (1, 0, True), (1, 1, True), (0, 1, False), (0, 1, True), (None, None, True), (1, 0, True), ("R", 1, True), (0, 0, True)]
+    for v, m, transient in steps:
+        X.SetTransient(transient)
+        if v is None:                                # no scatter: the operand's own values
+            X.data[...] = resident
+            X.SwitchFromGPU()
+            X.MoveToGPU()
+        engine.BeginMultiKernelLaunch()
+        if v == "R":                                 # the kernel reads a tensor that no scatter of the capture writes
+            engine.FlatIndexedScatter(X, L[0], maps[m])
+            R.data[...] = resident
+            R.SwitchFromGPU()
+        elif v is not None:
+            engine.FlatIndexedScatter(X, L[v], maps[m])
+        operand = R if v == "R" else X
+        engine("A_e = X_e_n W_e_n", A, operand, tW)
+        engine.EndMultiKernelLaunch()
+        read = resident if v in (None, "R") else vectors[v][maps[m].map].reshape(E, n)
+        A.MoveFromGPU()
+        assert rel_err(A.data, (read * W).sum(axis=1)) <= TOL, (v, m, transient)
+        assert ("X<-gathered" in engine.GetLastImplementation()) == (transient and v not in (None, "R"))
+        if v not in (None, "R") and not transient:
+            X.MoveFromGPU()
+            assert np.array_equal(X.data, read)
+
+
+def test_captures_that_alternate_at_the_same_positions(at, engine, checker):
+    """More kernel strings and extents per position of a capture than are remembered, in turn, and a capture that is cut short
+    by an error."""
+    rng = np.random.default_rng(10)
+    kernels = ["S_e_i = A_e_i B_e", "S_e_i = A_e_i", "S_e_i = B_e A_e_i", "S_e_i += A_e_i B_e", "S_e_i = A_e_i B_e B_e"]
+    for turn in range(3):
+        for e, i in ((5, 4), (6, 4), (5, 3)):
+            for kernel in kernels:
+                A, B, S0 = rng.uniform(-1, 1, (e, i)), rng.uniform(-1, 1, e), rng.uniform(-1, 1, (e, i))
+                S, T, t = to_tensor(at, S0), at.Tensor(e, i), {"A": to_tensor(at, A), "B": to_tensor(at, B)}
+                engine.BeginMultiKernelLaunch()
+                engine(kernel, S, *[t[x[0]] for x in kernel.split("= ")[1].split()])
+                engine("T_e_i = S_e_i B_e", T, S, t["B"])
+                engine.EndMultiKernelLaunch()
+                scale = B[:, None] ** kernel.count("B_")
+                expected = A * scale + (S0 if "+=" in kernel else 0.0)
+                S.MoveFromGPU()
+                T.MoveFromGPU()
+                assert rel_err(S.data, expected) <= TOL and rel_err(T.data, expected * B[:, None]) <= TOL
+        broken = at.TensorEngine("HIP")
+        broken.BeginMultiKernelLaunch()
+        broken("S_e_i = A_e_i B_e", S, t["A"], t["B"])
+        with pytest.raises(at.AcroError):
+            broken("S_e_i = A_e_i B_e", S, t["A"])
+        with pytest.raises(at.AcroError):
+            broken("T_e_i = S_e_i B_e", T, S, at.Tensor(17))
