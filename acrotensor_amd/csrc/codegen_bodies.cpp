@@ -484,7 +484,7 @@ auto Generator::GlobalStore(int k, const std::string &gaddr, const std::string &
 auto Generator::NeedsLdsCopy(int k) const -> bool
 {
     const Storage &st = StoreOf(subs[k].out.uvar);
-    return st.inLds && (st.liveTo > k || st.copyOutOnly);
+    return st.inLds && (st.liveTo > k || (st.copyOutOnly && StoresToGlobal(k)));
 }
 
 // A result that must reach device memory AND stays in LDS for a later kernel is written to device memory from
@@ -505,7 +505,8 @@ auto Generator::CopiesOutFromLds(int k) const -> bool
     if (st.members.size() != 1 || st.batchDim != 0 || !u.fixed.empty() || u.viewOffset != 0) return false;
     for (size_t j = 0; j < subs.size(); ++j)
     {
-        if (static_cast<int>(j) != k && uvars[subs[j].out.uvar].storage == u.storage) return false;
+        if (static_cast<int>(j) == k || uvars[subs[j].out.uvar].storage != u.storage) continue;
+        if (!st.copyOutOnly || StoresToGlobal(static_cast<int>(j))) return false;
     }
     return true;
 }

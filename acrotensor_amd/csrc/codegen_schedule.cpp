@@ -770,21 +770,34 @@ auto Generator::ComputeLdsWishes() -> void
 auto Generator::ChooseCopyOutTile() -> void
 {
     if (envInt("ACRO_HIP_COPY_OUT_TILE") < 0 || envInt("ACRO_HIP_LDS_COPY_OUT") < 0 || envInt("ACRO_HIP_PERSIST") > 0) return;
-    // the kernel that writes the group's last result (for a kernel evaluated in steps: its last step)
-    const int k = static_cast<int>(subs.size()) - 1;
+    // the kernel that writes the group's last result (for a kernel evaluated in steps: its last step), and the others
+    // whose results no kernel of the group reads
+    for (int k = static_cast<int>(subs.size()) - 1; k >= 0; --k) LeaveThroughTile(k);
+}
+
+auto Generator::LeaveThroughTile(int k) -> void
+{
     const Sub &s = subs[k];
-    if (s.loopMode || s.matrixOp != 0 || s.op != '=' || s.out.repeated || s.splitLanes != 0 || s.tile.empty()) return;
+    const bool group = subs.size() > 1;
+    // (of an accumulation whose terms are summed in registers, "Y = ...", "Y += ...", the last kernel)
+    int first = k;
+    while (first > 0 && subs[first].forwardedOld) --first;
+    if (s.loopMode || s.matrixOp != 0 || subs[first].op != '=' || s.out.repeated || s.splitLanes != 0 || s.tile.empty()) return;
     const UVarInfo &u = uvars[s.out.uvar];
     Storage &st = stores[u.storage];
     if (!st.elementLocal || st.anyRepeated || st.members.size() != 1 || st.batchDim != 0 || !u.fixed.empty() || u.viewOffset != 0 || st.transient) return;
-    for (int j = 0; j <= k; ++j)
+    for (int j = 0; j < static_cast<int>(subs.size()); ++j)
     {
-        if (j != k && uvars[subs[j].out.uvar].storage == u.storage) return;
+        if ((j < first || j > k) && uvars[subs[j].out.uvar].storage == u.storage) return;
         for (const auto &r : subs[j].in)
         {
             if (uvars[r.uvar].storage == u.storage) return;
         }
     }
+    // Launches of less than 1 MB of this result keep what the rules for a few workgroups give them: the barrier and the
+    // second pass are in the open there.
+    const bool large = group && E * st.tileSize >= (1L << 17);
+    if (!large && (k + 1 != static_cast<int>(subs.size()) || first != k)) return;
     // Results in planes ("D_e_m_n_k1_k2_k3" with the lanes along k and the tile (m, n)) whose length is no multiple of 64
     // bytes: a wavefront's stores start anywhere in a line, and a streaming store of part of a 64-byte piece costs as much as
     // two.  An entry's planes are one contiguous range, so they leave through a tile too, of up to 64 KB.  Geometric factors
@@ -813,13 +826,24 @@ auto Generator::ChooseCopyOutTile() -> void
     // memory-side cache.  Rotated tensors, by the lanes / through the tile: 7 x 9 operator 59 -> 72 %, 7 x 7 59 -> 75 %,
     // 5 x 5 64 -> 75 %, 4 x 4 69 -> 75 %, outer product of two 8-vectors 78 -> 91 %.)
     const long longRun = envInt("ACRO_HIP_COPY_OUT_RUN", 4);
-    // (the check for scattered stores covers runs of up to seven, also inside a group, where the rule for long runs does
-    // not apply: the p = 6 mass apply ends in runs of seven, 66 against 73 % of the HBM peak)
-    if (run < std::max<long>(longRun, 8) && envInt("ACRO_HIP_COPY_OUT_TILE") < 2)
+    // (the check for scattered stores covers runs of up to seven, also inside a small group, where the rule for long runs
+    // does not apply)
+    // Large launches of a group: whatever the run, and from 60 % of the lines on (30 % for entries below 24 doubles: 2D mass
+    // apply at p = 3, 16 per entry, 66.8 against 68.0 us; and for accumulated results, whose workgroups have more LDS:
+    // diffusion apply on 2^22 points p = 3, 5^3 points 59.9 against 62.0, p = 4, 6^3 59.8 against 62.3).  Every stage of a
+    // chain ends with the tile along the fastest index, so its last result leaves in runs of P doubles per lane.  Us by the
+    // lanes -> through the tile, run-time compiler 7.0: mass apply on 2^24 degrees of freedom p = 7, 8^3 points 78.7 -> 66.2
+    // (floor 63), p = 8, 9^3 92.9 -> 78.5 and 10^3 99.5 -> 89.3, p = 4, 5^3 77.4 -> 71.1; 1000 elements at p = 8 8.6 -> 7.5;
+    // with the element map and the sum-gather p = 3, 5^3 136 -> 132; 2D mass apply, 400 MB, run of 8 76 -> 68, 10 87 -> 72, 15
+    // 96 -> 84; interpolation as a chain to 8^3 points 102 -> 57, 10^3 99 -> 65, 11^3 117 -> 70; diffusion apply on 2^25
+    // points, accumulated in registers, p = 7, 8^3 530 -> 505.  The three components of a gradient, of which two are not the
+    // last kernel's result, 3^3 points 121 -> 61, 7^3 132 -> 72, 9^3 142 -> 80, 10^3 134 -> 87.
+    const bool lowCoverage = !large || st.tileSize < 24 || first != k;
+    if ((large || run < std::max<long>(longRun, 8)) && envInt("ACRO_HIP_COPY_OUT_TILE") < 2)
     {
         const int entries = static_cast<int>(std::max<long>(1, 64 / std::max<long>(1, s.laneCount)));
         const double coverage = WaveStoreLineCoverage(k, entries);
-        scattered = oddPlanes || (s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", 30) ||
+        scattered = oddPlanes || (s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", lowCoverage ? 30 : 60) ||
                                          (coverage < 0.95 && envInt("ACRO_HIP_COPY_OUT_WRITERS") >= 0 && WritesDominate())));
     }
     if (subs.size() != 1 && !scattered) return;
@@ -827,7 +851,8 @@ auto Generator::ChooseCopyOutTile() -> void
     st.copyOutOnly = true;
     st.wantLds = true;
     st.liveTo = k;
-    st.phaseFrom = st.phaseTo = PhaseOf(k);
+    st.phaseFrom = PhaseOf(k);
+    st.phaseTo = st.phaseFrom + 1;   // (copied out after the barrier that ends the phase, while the next one may have begun)
 }
 
 auto Generator::ChooseStagedInputs() -> void
@@ -1462,6 +1487,18 @@ auto Generator::ChooseBatching() -> void
             ldsDoubles = tighter;
         else
             for (size_t si = 0; si < stores.size(); ++si) stores[si].ldsOffset = before[si];
+    }
+
+    // A result accumulated in registers leaves from there after all where few workgroups are resident: nothing hides the
+    // second pass.  Diffusion apply on 2^25 points by the lanes / through the tile: p = 7, 10^3 points (53 KB of LDS, three
+    // workgroups) 480 / 515 us, p = 6, 10^3 (49 KB) 466 / 473, p = 8, 10^3 (48 KB) 538 / 535, 11^3 848 / 873, but 9^3 (35 KB)
+    // p = 7 502 / 478, p = 8 562 / 548.
+    for (const auto &s : subs)
+    {
+        Storage &st = stores[uvars[s.out.uvar].storage];
+        if (!s.forwardedOld || !st.copyOutOnly || static_cast<long>(ldsDoubles) * 8 <= 40 * 1024) continue;
+        st.copyOutOnly = st.wantLds = st.inLds = false;
+        st.liveTo = -1;
     }
 }
 

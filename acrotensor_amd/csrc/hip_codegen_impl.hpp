@@ -269,6 +269,7 @@ class Generator
     int PhaseOf(int k) const { return subs[k].phase; }
     void ComputeLdsWishes();
     void ChooseCopyOutTile();
+    void LeaveThroughTile(int k);
 
     // A small operand that does not depend on the batch entry but whose address depends on the lane
     // ("A_e_i = B_i_j X_e_j" with one lane per i: lane i walks along row i of B, 512 bytes from its neighbour's) cannot

@@ -351,3 +351,55 @@ def test_diffusion_with_the_first_phases_loads_in_their_phase(at, checker, monke
     assert "streaming inputs of phase 3, requested before" in src and "streaming inputs of phase 0" not in src
     expected = workloads.run_on_checker(wl, checker)["Y"]
     assert rel_err(fetch(tensors, "Y"), expected) <= TOL
+
+
+GRADIENT = ["A_e_q_j_k = B_q_i X_e_i_j_k", "G_e_q_j_k = H_q_i X_e_i_j_k", "A2_e_q_r_k = B_r_j A_e_q_j_k", "A3_e_q_r_k = H_r_j A_e_q_j_k",
+            "G2_e_q_r_k = B_r_j G_e_q_j_k", "Y0_e_q_r_s = B_s_k G2_e_q_r_k", "Y1_e_q_r_s = B_s_k A3_e_q_r_k", "Y2_e_q_r_s = H_s_k A2_e_q_r_k"]
+MASS = ["T1_e_q_j_k = B_q_i X_e_i_j_k", "T2_e_q_r_k = B_r_j T1_e_q_j_k", "T3_e_q_r_s = B_s_k T2_e_q_r_k", "U_e_q_r_s = D_e_q_r_s T3_e_q_r_s",
+        "V1_e_i_r_s = B_q_i U_e_q_r_s", "V2_e_i_j_s = B_r_j V1_e_i_r_s", "Y_e_i_j_k = B_s_k V2_e_i_j_s"]
+DIFFERENCE = MASS[:5] + ["V1b_e_i_r_s = H_q_i U_e_q_r_s", MASS[5], "V2b_e_i_j_s = H_r_j V1b_e_i_r_s", MASS[6], "Y_e_i_j_k -= H_s_k V2b_e_i_j_s"]
+
+
+@pytest.mark.parametrize("kernels,p,q,elements,copied", [
+    (MASS, 7, 8, 389, "Y"), (MASS, 8, 9, 257, "Y"), (MASS, 3, 4, 4857, "Y"), (MASS, 3, 4, 4854, ""), (MASS, 6, 6, 607, "Y"),
+    (GRADIENT, 3, 4, 2051, "Y0 Y1 Y2"), (GRADIENT, 7, 9, 191, "Y0 Y1 Y2"), (GRADIENT, 2, 3, 4901, "Y0 Y1 Y2"), (GRADIENT, 4, 6, 501, "Y2"),
+    (DIFFERENCE, 7, 8, 389, "Y"), (DIFFERENCE, 8, 9, 257, "Y"), (DIFFERENCE, 7, 8, 380, "")])
+def test_results_of_a_chain_in_whole_lines(at, monkeypatch, kernels, p, q, elements, copied):
+    """Results of 1 MB and more leave through LDS tiles also in long runs per lane, when their terms were summed in registers
+    and when they are not the last: the same bits as the lanes' own stores give, within a tolerance of the sums."""
+    shapes, rng = {}, np.random.RandomState(elements)
+    for k in kernels:
+        for v in k.replace("-=", "=").replace("=", " ").split():
+            name, *idx = v.split("_")
+            shapes[name] = [elements if i == "e" else q if i in "qrs" else p for i in idx]
+    arrays = {n: rng.uniform(-1.0, 1.0, s) for n, s in shapes.items()}
+    results = [n for n in shapes if n.startswith("Y")]
+    scratch = [n for n in shapes if n not in results and n not in "XDBH"]
+
+    def run(engine):
+        t = {}
+        for n in shapes:
+            t[n] = at.Tensor(*shapes[n]) if n in scratch else to_tensor(at, arrays[n])
+            t[n].SetTransient(n in scratch)
+        engine.BeginMultiKernelLaunch()
+        for k in kernels:
+            engine(k, *[t[v.split("_")[0]] for v in k.replace("-=", "=").replace("=", " ").split()])
+        engine.EndMultiKernelLaunch()
+        for n in results:
+            t[n].MoveFromGPU()
+        return {n: t[n].data.copy() for n in results}
+
+    engine = at.TensorEngine("HIP")
+    got = run(engine)
+    src = engine.GetLastImplementation()
+    assert [n for n in results if "// %s: LDS tiles -> device memory" % n in src] == copied.split()
+    monkeypatch.setenv("ACRO_HIP_COPY_OUT_TILE", "-1")
+    plain = run(at.TensorEngine("HIP"))
+    for k in kernels:
+        names = [v.split("_") for v in k.replace("-=", "=").replace("=", " ").split()]
+        letters = ["".join(v[1:]) for v in names]
+        value = np.einsum("%s->%s" % (",".join(letters[1:]), letters[0]), *[arrays[v[0]] for v in names[1:]], optimize=True)
+        arrays[names[0][0]] = arrays[names[0][0]] - value if "-=" in k else value
+    for n in results:
+        assert np.array_equal(got[n], plain[n])
+        assert np.abs(got[n] - arrays[n]).max() <= TOL * np.abs(arrays[n]).max()
