@@ -546,6 +546,21 @@ auto Generator::EmitOperator(HipKernelPlan &plan) -> void
     plan.launches.push_back(launch);
 }
 
+// Rows that are no whole 64-byte pieces, results of 26 to 144 MiB: ordinary stores, whose lines the memory-side cache
+// still holds when the next operation reads them.  The product itself takes a little longer, the two together less:
+// us, streaming stores -> ordinary ones, inputs and outputs changing, with the transposed product behind it | alone:
+//   110 x 60, 131 072 entries 103.6 -> 96.6 | 50.6 -> 53.8     65 x 64 69.8 -> 65.2 | 36.7 -> 37.0
+//   90 x 64 84.4 -> 79.8 | 42.7 -> 44.3     125 x 64, 90 000 82.1 -> 77.3 | 40.1 -> 43.0 (one set of tensors:
+//   75.5 -> 71.0 | 36.2 -> 36.8), 131 072 102.9 -> 101.5 | 51.2 -> 52.8 (94.0 -> 86.5 | 44.8 -> 45.4),
+//   30 000 38.0 -> 35.4 | 20.8 -> 22.8
+// Smaller results stay in the cache either way and larger ones do not: 90 x 64, 30 000 33.3 -> 35.5 | 17.0 -> 18.8;
+// 65 x 64, 500 000 213.5 -> 219.0 | 115.4 -> 117.5 (one set 94 -> 116); 100 x 50, 300 000 185.3 -> 191.3 | 89.4 -> 92.9.
+static constexpr long kCachedResultFrom = 13L << 18, kCachedResultTo = 18L << 20;   // doubles
+static auto ReadAgainFromCache(long resultDoubles, long rows) -> bool
+{
+    return rows % 8 != 0 && resultDoubles >= kCachedResultFrom && resultDoubles <= kCachedResultTo;
+}
+
 // The same on the FP64 matrix cores: a wavefront takes 16 entries at a time and forms their nI outputs with
 // v_mfma_f64_16x16x4 (16 entries x 16 outputs x 4 terms per instruction).  The entries' vectors are the
 // instruction's first operand, read with ordinary 16-byte vector loads (lane = entry + 16 * term group); the
@@ -583,11 +598,25 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
     // out as one contiguous range.
     // (all 16 entries at once where LDS allows, else 8 or 4 at a time)
     int stageRounds = 0;
-    if (!next && shape.allRows == 0 && shape.comp == 1 && nI % 16 != 0 && envInt("ACRO_HIP_OPERATOR_STAGE_OUT") >= 0)
+    // Operators that fill most of LDS run one wavefront per SIMD, whose matrix instructions wait for each trip's vectors:
+    // those of the next trip are requested before this trip's arithmetic (behind the last trip its own again, so that the
+    // request is unconditional).  Us, before -> after: 125 x 64 on 30 000 entries with the transposed product behind it
+    // 35.4 -> 34.3, on 131 072 101.0 -> 99.0; 128 x 64 34.2 -> 32.7 and 98.1 -> 95.8, alone on 262 143 83.5 -> 79; 100 x 64
+    // on 30 000 31.2 -> 29.7.  Smaller operators keep more wavefronts: 72 x 64 35.5 -> 37.7; odd rows of a result too large
+    // for the memory-side cache wait for its streaming stores: 110 x 60 on 262 143 75.2 -> 82, 90 x 80 89 -> 94.5.
+    const bool ahead = !next && pairs && shape.comp == 1 && s.op == '=' && nIp * nJp >= 7168 &&
+                       (nI % 8 == 0 || E * nAll <= kCachedResultTo) && shape.perElement.empty() && shape.perColumn.empty() &&
+                       envInt("ACRO_HIP_OPERATOR_AHEAD") >= 0;
+    const long mostLds = ahead ? 104 * 1024 : 64 * 1024;
+    // (An operator of more than 4096 entries in one block of rows: the results of 8 entries at a time beside the 64 KB of the
+    // operator, in 16-byte pieces, where they are streamed out and small: 125 x 64 on 25 003 entries 19.2 -> 18.1 us, the
+    // lanes' own stores 19.1; 110 x 60 19.9 -> 19.0, 20.3; on 262 143 85.6 -> 88.9.)
+    const bool whole = ahead && shape.allRows == nI && E * nI < kCachedResultFrom;
+    if (!next && (shape.allRows == 0 || whole) && shape.comp == 1 && nI % 16 != 0 && envInt("ACRO_HIP_OPERATOR_STAGE_OUT") >= 0)
     {
         for (int rounds : {1, 2, 4})
         {
-            if (stageRounds == 0 && (nIp * nJp + 64 / rounds * nI) * 8 <= 64 * 1024) stageRounds = rounds;
+            if (stageRounds == 0 && (nIp * nJp + 64 / rounds * nI) * 8 <= mostLds) stageRounds = rounds;
         }
     }
     const bool viaStage = stageRounds > 0;
@@ -681,15 +710,35 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
     out << "    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;\n";
     // (A contiguous range of trips per workgroup instead of this stride: the same or up to 8 % slower.)
     out << "    const long waves = (long)gridDim.x * 4;\n";
+    const std::string vectors = "[&] { const acro_pair t = *reinterpret_cast<const acro_pair *>(x + 8 * q); return double2{t.x, t.y}; }();\n";
+    const std::string pastEnd = nJp != nJ ? "8 * q + 2 * g >= " + str(nJ) + " ? double2{0.0, 0.0} : " : std::string();
+    auto requestAhead = [&](const std::string &which) {
+        out << "            const long ex = " << which << " * 16 + c" << (ragged ? " < " + str(E) + " ? " + which + " * 16 + c : " + str(E - 1) : std::string()) << ";\n";
+        out << "            const double *x = " << X << " + " << Lit(uvars[x.uvar].viewOffset) << " + ex * " << nJ << " + 2 * g;\n";
+        out << "#pragma unroll\n            for (int q = 0; q < " << nJp / 8 << "; ++q) ahead[q] = " << pastEnd << vectors;
+    };
+    if (ahead)
+    {
+        out << "    double2 ahead[" << nJp / 8 << "];\n    {\n        const long trip = (long)blockIdx.x * 4 + (threadIdx.x >> 6), here = trip < " << tiles << " ? trip : " << tiles - 1 << ";\n";
+        requestAhead("here");
+        out << "    }\n";
+    }
     out << "    for (long tile = (long)blockIdx.x * 4 + (threadIdx.x >> 6); tile < " << tiles << "; tile += waves)\n    {\n";
     // (a kernel that the compiler can only fit into the registers with spills is compiled again with this macro:
     // the operator's values are then read from LDS on every trip instead of being kept in registers across trips)
     out << "#ifdef ACRO_KEEP_OPERATOR_IN_LDS\n        __asm__ volatile(\"\" ::: \"memory\");\n#endif\n";
-    if (ragged)
+    if (ahead)
+    {
+        out << "        double2 xv[" << nJp / 8 << "];\n#pragma unroll\n        for (int q = 0; q < " << nJp / 8 << "; ++q) xv[q] = ahead[q];\n";
+        out << "        {   // the next trip's vectors (behind the last one its own again)\n            const long trip = tile + waves < " << tiles << " ? tile + waves : tile;\n";
+        requestAhead("trip");
+        out << "        }\n";
+    }
+    else if (ragged)
         out << "        const long ex = tile * 16 + c < " << E << " ? tile * 16 + c : " << E - 1 << ";  // past the end: any valid entry, never stored\n";
     else
         out << "        const long ex = tile * 16 + c;\n";
-    if (pairs)
+    if (pairs && !ahead)
     {
         out << "        const double *x = " << X << " + " << Lit(uvars[x.uvar].viewOffset) << " + ex * " << nJ << " + 2 * g;\n";
         out << "        double2 xv[" << nJp / 8 << "];\n";
@@ -714,7 +763,7 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
                 << " + 2 * g + 8 * q;\n            xv[q].x *= f[0];\n            xv[q].y *= f[1];\n        }\n";
         }
     }
-    else
+    else if (!ahead)
     {
         const long C = shape.comp;
         if (C > 1)
@@ -762,17 +811,7 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
         const long C = sh.comp;
         // (a block of rows: the entries' results lie `stride` apart and start at row `off`)
         const long stride = sh.allRows > 0 ? sh.allRows : rows, off = sh.rowOffset;
-        // Rows that are no whole 64-byte pieces, results of 26 to 144 MiB: ordinary stores, whose lines the memory-side cache
-        // still holds when the next operation reads them.  The product itself takes a little longer, the two together less:
-        // us, streaming stores -> ordinary ones, inputs and outputs changing, with the transposed product behind it | alone:
-        //   110 x 60, 131 072 entries 103.6 -> 96.6 | 50.6 -> 53.8     65 x 64 69.8 -> 65.2 | 36.7 -> 37.0
-        //   90 x 64 84.4 -> 79.8 | 42.7 -> 44.3     125 x 64, 90 000 82.1 -> 77.3 | 40.1 -> 43.0 (one set of tensors:
-        //   75.5 -> 71.0 | 36.2 -> 36.8), 131 072 102.9 -> 101.5 | 51.2 -> 52.8 (94.0 -> 86.5 | 44.8 -> 45.4),
-        //   30 000 38.0 -> 35.4 | 20.8 -> 22.8
-        // Smaller results stay in the cache either way and larger ones do not: 90 x 64, 30 000 33.3 -> 35.5 | 17.0 -> 18.8;
-        // 65 x 64, 500 000 213.5 -> 219.0 | 115.4 -> 117.5 (one set 94 -> 116); 100 x 50, 300 000 185.3 -> 191.3 | 89.4 -> 92.9.
-        const long resultDoubles = E * stride;
-        const bool readAgain = stride % 8 != 0 && resultDoubles >= (13L << 18) && resultDoubles <= (18L << 20);
+        const bool readAgain = ReadAgainFromCache(E * stride, stride);
         const bool streamsHere = streams && (!readAgain || envInt("ACRO_HIP_OPERATOR_ODD_ROWS") < 0);
         if (viaStage)
         {
@@ -811,6 +850,20 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
                         << "            const int count = (int)(left < 0 ? 0 : (left < " << entries << " ? left : " << entries << ")) * " << rows << ";\n";
                 else
                     out << "            const int count = " << entries * rows << ";\n";
+                if (ahead)
+                {
+                    // (16-byte pieces; the last entries of an odd number may end in a single double)
+                    out << "            for (int i = 2 * lane; i < count; i += 128)\n            {\n";
+                    if (ragged) out << "                if (i + 1 == count) { a[i] = mid[i]; break; }\n";
+                    if (streamsHere)
+                        out << "                __builtin_nontemporal_store(*reinterpret_cast<const acro_pair *>(mid + i), reinterpret_cast<acro_pair *>(a + i));\n";
+                    else
+                        out << "                *reinterpret_cast<acro_pair *>(a + i) = *reinterpret_cast<const acro_pair *>(mid + i);\n";
+                    out << "            }\n";
+                    out << "        }\n";
+                    out << "        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, \"wavefront\");\n        __builtin_amdgcn_wave_barrier();\n";
+                    continue;
+                }
                 out << "            for (int i = lane; i < count; i += 64)\n";
                 if (streams)
                     out << "                __builtin_nontemporal_store(mid[i], a + i);\n";

@@ -403,3 +403,26 @@ def test_results_of_a_chain_in_whole_lines(at, monkeypatch, kernels, p, q, eleme
     for n in results:
         assert np.array_equal(got[n], plain[n])
         assert np.abs(got[n] - arrays[n]).max() <= TOL * np.abs(arrays[n]).max()
+
+
+@pytest.mark.parametrize("rows,cols,entries,whole", [(125, 64, 2049, True), (125, 64, 16 * 4096 + 23, False), (125, 64, 4103, True), (126, 62, 16391, True),
+                                                     (113, 64, 2057, True), (128, 56, 4099, False), (125, 64, 27263, False), (110, 60, 30983, False)])
+def test_operators_that_fill_lds_request_the_next_vectors_ahead(at, engine, monkeypatch, rows, cols, entries, whole):
+    """The same bits as without the request, and nothing behind the result is written (an odd count of doubles at its end)."""
+    rng = np.random.RandomState(rows + entries)
+    B, X = rng.uniform(-1.0, 1.0, (rows, cols)), rng.uniform(-1.0, 1.0, (entries, cols))
+
+    def run(eng):
+        parent = to_tensor(at, np.full((3, entries, rows), 7.0))       # (the result may start at an odd double)
+        eng("A_e_i = B_i_j X_e_j", at.SliceTensor(parent, 1), to_tensor(at, B), to_tensor(at, X))
+        parent.MoveFromGPU()
+        assert np.all(parent.data[0] == 7.0) and np.all(parent.data[2] == 7.0)
+        return parent.data[1].copy()
+
+    got = run(engine)
+    src = engine.GetLastImplementation()
+    assert "ahead[" in src and ("results written out through LDS" in src) == whole
+    monkeypatch.setenv("ACRO_HIP_OPERATOR_AHEAD", "-1")
+    assert np.array_equal(got, run(at.TensorEngine("HIP")))
+    expected = X @ B.T
+    assert np.abs(got - expected).max() <= TOL * np.abs(expected).max()
