@@ -838,12 +838,18 @@ auto Generator::LeaveThroughTile(int k) -> void
     // 96 -> 84; interpolation as a chain to 8^3 points 102 -> 57, 10^3 99 -> 65, 11^3 117 -> 70; diffusion apply on 2^25
     // points, accumulated in registers, p = 7, 8^3 530 -> 505.  The three components of a gradient, of which two are not the
     // last kernel's result, 3^3 points 121 -> 61, 7^3 132 -> 72, 9^3 142 -> 80, 10^3 134 -> 87.
+    // (45 % where intermediates are stored as well, which leave through their own tiles: p = 3, 5^3 points 80.4 against 81.1)
     const bool lowCoverage = !large || st.tileSize < 24 || first != k;
+    bool storedBetween = false;
+    for (const auto &q : subs)
+    {
+        for (const auto &r : q.in) storedBetween = storedBetween || (stores[uvars[r.uvar].storage].written && !stores[uvars[r.uvar].storage].transient && !uvars[r.uvar].isVirtual);
+    }
     if ((large || run < std::max<long>(longRun, 8)) && envInt("ACRO_HIP_COPY_OUT_TILE") < 2)
     {
         const int entries = static_cast<int>(std::max<long>(1, 64 / std::max<long>(1, s.laneCount)));
         const double coverage = WaveStoreLineCoverage(k, entries);
-        scattered = oddPlanes || (s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", lowCoverage ? 30 : 60) ||
+        scattered = oddPlanes || (s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", lowCoverage ? 30 : (storedBetween ? 45 : 60)) ||
                                          (coverage < 0.95 && envInt("ACRO_HIP_COPY_OUT_WRITERS") >= 0 && WritesDominate())));
     }
     if (subs.size() != 1 && !scattered) return;
