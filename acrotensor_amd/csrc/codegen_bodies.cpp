@@ -866,6 +866,71 @@ auto Generator::EmitSplitLanesBody(int k, std::vector<std::string> &lines) -> vo
     lines.push_back("}");
 }
 
+// The terms of a sum in batches: all loads of a batch, then its products and sums, in the order of the terms.  With few lanes
+// a lane's loads are all that is in flight, and the barrier keeps the compiler from moving them between the sums: asked for as
+// many by "#pragma unroll" it interleaves loads and waits, with five operands per lane unrolled by 8, with two by 32.  Us,
+// unrolled by four | by 8, 16 or 32 | in batches: 3 x 3 sums over 1 024 slices 39 | 18 | 17, 2 047 slices 113 | 41 | 33;
+// "S_i_j = A_n_i B_n_j", 1 000 terms, 4 x 4 outputs 42 | 75 | 18; five and eight operands per lane, 1 000 terms and outputs
+// 178 | 492 | 113 and 429 | 1 190 | 181, six, 9 outputs 124 | 268 | 80; four per lane and four shared ones, 16 384 outputs
+// 180 | 279 | 111.  Slower than unrolled, of what was tried: 200 x 5 terms with a transposed factor 70 | 13.8 | 16.5, 80 x 12
+// terms of two operands per lane (10 x 10 outputs) 26.9 | 30.9.
+auto Generator::SumInBatches(int k, const std::vector<int> &order, const std::function<std::string(size_t)> &operand, std::vector<std::string> &lines) -> void
+{
+    const Sub &s = subs[k];
+    long scalars = 0;
+    for (size_t v = 0; v < s.in.size(); ++v) scalars += SourceOf(k, static_cast<int>(v)) == kFromConstant ? 1 : 0;
+    const long vectors = static_cast<long>(s.in.size()) - scalars;
+    // (per lane, us with 8 / 16 / 24 / 32 / 48 terms: two operands 29 / 22 / 19 / 19 / 19, four 55 / 48 / 50 / 48 / 51, eight
+    // 114 / 99 / 93 / 127 / 723; shared ones, with 8 / 12 / 16 / 24: two 28 / 24 / 23 / 22, three 31 / 27 / 28 / 51, four 34 /
+    // 33 / 62 / 43, seven 51 / 131 / 111 / 109; one operand, or one and a shared one, 2 047 terms with 16 / 24 / 32 / 40 / 48:
+    // 39 / 36 / 34 / 33 / 32)
+    const long byVectors = vectors <= 2 ? 32 : (vectors == 3 ? 24 : std::max<long>(2, std::min<long>(16, 128 / vectors)));
+    const long byScalars = scalars <= 1 ? 32 : (scalars == 2 ? 24 : (scalars <= 4 ? 12 : std::max<long>(2, std::min<long>(8, 56 / scalars))));
+    const long most = s.in.size() <= 2 && scalars <= 1 ? 40 : std::min(byVectors, byScalars);
+    // A batch is a range of the innermost index, or, where that is short, of the next one with all of the innermost.
+    const int inner = order.back();
+    const bool both = order.size() > 1 && 2L * extent[inner] <= most;
+    const int ranged = both ? order[order.size() - 2] : inner;
+    const long each = both ? extent[inner] : 1, step = std::min<long>(most / each, extent[ranged]);
+    std::string indent;
+    for (size_t j = 0; j + (both ? 2 : 1) < order.size(); ++j)
+    {
+        const std::string c = IdxVar(order[j]);
+        lines.push_back(indent + "for (int " + c + " = 0; " + c + " < " + str(extent[order[j]]) + "; ++" + c + ")");
+        lines.push_back(indent + "{");
+        indent += "    ";
+    }
+    auto batchOf = [&](const std::string &from, long n) {
+        const std::string terms = str(n * each);
+        std::string values, prod;
+        for (size_t v = 0; v < s.in.size(); ++v)
+        {
+            const std::string name = "x" + str(static_cast<long>(v));
+            values += (values.empty() ? "double " : ", ") + name + "[" + terms + "]";
+            prod = prod.empty() ? name + "[t]" : "(" + prod + " * " + name + "[t])";
+        }
+        lines.push_back(indent + "{");
+        lines.push_back(indent + "    " + values + ";");
+        lines.push_back("#pragma unroll");
+        lines.push_back(indent + "    for (int t = 0; t < " + terms + "; ++t)");
+        lines.push_back(indent + "    {");
+        lines.push_back(indent + "        const int " + IdxVar(ranged) + " = " + from + (both ? " + t / " + str(each) : std::string(" + t")) + ";");
+        if (both) lines.push_back(indent + "        const int " + IdxVar(inner) + " = t % " + str(each) + ";");
+        for (size_t v = 0; v < s.in.size(); ++v) lines.push_back(indent + "        x" + str(static_cast<long>(v)) + "[t] = " + operand(v) + ";");
+        lines.push_back(indent + "    }");
+        lines.push_back(indent + "    __builtin_amdgcn_sched_barrier(0);");
+        lines.push_back("#pragma unroll");
+        lines.push_back(indent + "    for (int t = 0; t < " + terms + "; ++t) sum += " + prod + ";");
+        lines.push_back(indent + "}");
+    };
+    const long whole = extent[ranged] / step * step;
+    lines.push_back("#pragma unroll 1");
+    lines.push_back(indent + "for (int first = 0; first < " + str(whole) + "; first += " + str(step) + ")");
+    batchOf("first", step);
+    if (whole < extent[ranged]) batchOf(str(whole), extent[ranged] - whole);
+    for (; !indent.empty(); indent.resize(indent.size() - 4)) lines.push_back(indent.substr(4) + "}");
+}
+
 auto Generator::EmitLoopBody(int k, std::vector<std::string> &lines) -> void
 {
     const Sub &s = subs[k];
@@ -896,25 +961,6 @@ auto Generator::EmitLoopBody(int k, std::vector<std::string> &lines) -> void
         (carried || s.tile.empty() ? order : inner).push_back(c);
     }
     order.insert(order.end(), inner.begin(), inner.end());
-    // One output per lane and fewer lanes than the device holds wavefronts to hide a load behind: bound by the latency of the
-    // loads, so more of them are in flight (3 x 3 sums of a stream, us with 4 / 8 / 16 / 32 / 64: 1 024 terms 39 / 26 / 20 / 18 /
-    // 19, 2 047 terms 112 / 68 / 45 / 41 / 38).  As many as the registers hold with several operands.
-    const bool fewLanes = tc == 1 && E * s.laneCount <= 16384;
-    const std::string unroll = "#pragma unroll " + std::string(!fewLanes ? "4" : (s.in.size() <= 2 ? "32" : (s.in.size() <= 4 ? "16" : "8")));
-    std::string indent;
-    for (size_t j = 0; j < order.size(); ++j)
-    {
-        const std::string c = IdxVar(order[j]);
-        // Around a register tile only the innermost loop is unrolled: with every loop unrolled the compiler requests
-        // all scalar operands of all terms at once and spills them.
-        if (j + 1 == order.size())
-            lines.push_back(indent + (tc > 1 && extent[order[j]] <= 8 ? "#pragma unroll" : unroll));
-        else if (tc > 1)
-            lines.push_back(indent + "#pragma unroll 1");
-        lines.push_back(indent + "for (int " + c + " = 0; " + c + " < " + str(extent[order[j]]) + "; ++" + c + ")");
-        lines.push_back(indent + "{");
-        indent += "    ";
-    }
     std::vector<int> value(nidx, 0);
     auto operand = [&](size_t v) {
         const VarRef &r = s.in[v];
@@ -934,8 +980,25 @@ auto Generator::EmitLoopBody(int k, std::vector<std::string> &lines) -> void
         if (lds) return "lds[o_k" + str(k) + "v" + str(v) + " + " + off + "]";
         return GlobalRead(r.uvar, "o_k" + str(k) + "v" + str(v) + " + " + off, StreamedOnce(k, static_cast<int>(v)));
     };
+    // One output per lane and at most a wavefront per compute unit: bound by the latency of the loads.
+    const bool fewLanes = s.tile.empty() && E * s.laneCount <= 16384;
+    std::string indent;
+    for (size_t j = 0; j < order.size() && !fewLanes; ++j)
+    {
+        const std::string c = IdxVar(order[j]);
+        // Around a register tile only the innermost loop is unrolled: with every loop unrolled the compiler requests
+        // all scalar operands of all terms at once and spills them.
+        if (j + 1 == order.size())
+            lines.push_back(indent + (tc > 1 && extent[order[j]] <= 8 ? "#pragma unroll" : "#pragma unroll 4"));
+        else if (tc > 1)
+            lines.push_back(indent + "#pragma unroll 1");
+        lines.push_back(indent + "for (int " + c + " = 0; " + c + " < " + str(extent[order[j]]) + "; ++" + c + ")");
+        lines.push_back(indent + "{");
+        indent += "    ";
+    }
+    if (fewLanes) SumInBatches(k, order, operand, lines);
     std::string common;
-    for (size_t v = 0; v < s.in.size(); ++v)
+    for (size_t v = 0; v < s.in.size() && !fewLanes; ++v)
     {
         if (onTile[v]) continue;
         const std::string opnd = operand(v);
@@ -946,7 +1009,7 @@ auto Generator::EmitLoopBody(int k, std::vector<std::string> &lines) -> void
         lines.push_back(indent + "const double common = " + common + ";");
         common = "common";
     }
-    for (long t = 0; t < tc; ++t)
+    for (long t = 0; t < tc && !fewLanes; ++t)
     {
         long rem = t;
         for (int j = static_cast<int>(s.tile.size()) - 1; j >= 0; --j)
@@ -963,7 +1026,7 @@ auto Generator::EmitLoopBody(int k, std::vector<std::string> &lines) -> void
         }
         lines.push_back(indent + sumName(t) + " += " + prod + ";");
     }
-    for (size_t j = 0; j < order.size(); ++j)
+    for (size_t j = 0; j < order.size() && !fewLanes; ++j)
     {
         indent.resize(indent.size() - 4);
         lines.push_back(indent + "}");

@@ -359,6 +359,7 @@ class Generator
     void EmitUnrolledBody(int k, ForwardMap &forwarded, std::vector<std::string> &lines, const std::map<std::string, std::string> *preloaded = nullptr, std::vector<std::pair<std::string, std::string>> *globalLoads = nullptr);
     void EmitMatrixBody(int k, Body &body, ForwardMap &forwarded);
     void EmitSplitLanesBody(int k, std::vector<std::string> &lines);
+    void SumInBatches(int k, const std::vector<int> &order, const std::function<std::string(size_t)> &operand, std::vector<std::string> &lines);
     void EmitLoopBody(int k, std::vector<std::string> &lines);
 
     // ------------------------------------------------------------------------------ reduction schedule

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import acrotensor_amd as at
-from acrotensor_amd import workloads
+from acrotensor_amd import _capi, workloads
 
 
 @pytest.fixture(scope="module")
@@ -986,3 +986,19 @@ print(version.value // 100000)
     releases = {subprocess.run([sys.executable, "-c", program, first], cwd=root, env=env, check=True, capture_output=True, text=True).stdout.split()[-1]
                 for first in ("", "torch", "")}
     assert len(list(tmp_path.glob("*.hsaco"))) == len(releases)
+
+
+@pytest.mark.parametrize("factors,terms", [("B_n", 40), ("B_n_i", 40), ("B_n_i C_n", 32), ("B_n_i C_n_i", 24), ("B_n C_n", 24), ("B_n C_n D_n", 12), ("B_n_i C_n_i D_n_i F_n_i", 16),
+                                           ("B_n C_n_i D_n F_n_i G_n H_n_i K_n", 12), ("B_n_i C_n_i D_n_i F_n_i G_n_i H_n_i K_n_i L_n_i P_n_i Q_n_i", 11),
+                                           ("B_n C_n D_n F_n G_n H_n K_n", 8)])
+def test_sums_of_few_lanes_request_as_many_terms_as_the_registers_hold(TE, factors, terms):
+    """All loads of a batch before its sums, whatever the number of operands, and nothing in private memory."""
+    names = factors.split()
+    tensors = [at.Tensor(*[1000, 100][:v.count("_")]) for v in names]
+    src = TE.GetImplementation("S_i = A_n_i " + factors, at.Tensor(100), at.Tensor(1000, 100), *tensors)
+    assert "first += %d)" % terms in src and src.count("sched_barrier") == (2 if 1000 % terms else 1)
+    function, private = re.search(r"void (acro_\w+)\(", src).group(1), ctypes.c_int(-1)
+    assert _capi.load().acro_hip_compile_private_bytes(b"unit_batches", src.encode(), function.encode(), ctypes.byref(private)) == 0
+    assert private.value == 0
+    wide = TE.GetImplementation("S_i = A_n_i " + factors, at.Tensor(16385), at.Tensor(1000, 16385), *[at.Tensor(1000) if v.count("_") == 1 else at.Tensor(1000, 16385) for v in names])
+    assert "sched_barrier" not in wide

@@ -2,6 +2,8 @@
 through the C ABI.  Expected values come from the checker (the restated CPU interpreter) and, as in the reference's
 tests, from closed forms.  Integer-valued inputs make results exact in fp64 whatever the summation order, so those
 comparisons are bit-exact (index mapping); random inputs are held to 1e-12 relative to the largest entry."""
+import re
+
 import numpy as np
 import pytest
 
@@ -1656,7 +1658,7 @@ def test_other_tensors_that_relate_differently_never_take_the_previous_binding(a
     ("S_i = A_n_m_i B_m_n", [(33, 37, 4), (37, 33)]),
 ])
 def test_sums_as_counted_loops_of_few_lanes(at, engine, checker, kernel, shapes):
-    """Some hundred terms per lane and few lanes: unrolled by 32, 16 and 8, with remainders of the loop.  Integer values: exact."""
+    """Some hundred terms per lane and few lanes, in batches, with remainders.  Integer values: exact."""
     rng = np.random.default_rng(shapes[0][0])
     ins = [rng.integers(-4, 5, s).astype(np.float64) for s in shapes]
     out0 = rng.integers(-4, 5, output_shape(kernel, shapes)).astype(np.float64)
@@ -1669,3 +1671,31 @@ def test_sums_as_counted_loops_of_few_lanes(at, engine, checker, kernel, shapes)
     S.MoveFromGPU()
     assert "as counted loops" in engine.GetLastImplementation()
     assert np.array_equal(S.data, expected)
+
+
+@pytest.mark.parametrize("kernel,sizes", [
+    ("S_i = A_n_i B_n", dict(n=1024, i=9)), ("S_i = A_n_i B_n", dict(n=1023, i=1000)), ("S_i = A_n_i", dict(n=545, i=16384)),
+    ("S_i_j = A_n_i B_n_j", dict(n=1000, i=4, j=4)), ("S_i = A_n_i B_n_i C_n_i", dict(n=601, i=33)), ("S_i = A_n_i B_n C_n", dict(n=799, i=7)),
+    ("S_i = A_n_i B_n C_n D_n F_n", dict(n=997, i=70)), ("S_i = A_n_i B_n_i C_n_i D_n_i F_n_i G_n_i H_n_i K_n_i", dict(n=1001, i=130)),
+    ("S_i = A_n_i B_n C_n D_n F_n G_n H_n K_n", dict(n=1001, i=3)), ("S_i += A_n_i B_n C_n_i D_n F_n_i G_n H_n_i K_n", dict(n=650, i=257)),
+    ("S_i = A_n_m_i B_m_n", dict(n=200, m=5, i=30)), ("S_i = A_n_m_i B_m_n", dict(n=5, m=131, i=30)), ("S_i -= A_n_m_i B_m_n", dict(n=40, m=17, i=2)),
+    ("S_i = A_n_m_l_i B_l", dict(n=7, m=23, l=6, i=11)), ("S_i = A_n_m_l_i B_l_m", dict(n=11, m=3, l=33, i=11))])
+def test_sums_of_few_lanes_in_batches_keep_the_order_of_their_terms(at, engine, kernel, sizes):
+    """Products that are exact (all factors but one are powers of two), added one after the other: the same bits."""
+    rng = np.random.default_rng(sizes["n"])
+    out, *ins = [(v[0], v.split("_")[1:]) for v in re.sub(r"[+-]?=", " ", kernel).split()]
+    shape = lambda idx: tuple(sizes[x] for x in idx)
+    values = {name: rng.standard_normal(shape(idx)) if k == 0 else 2.0 ** rng.integers(-2, 3, shape(idx)) for k, (name, idx) in enumerate(ins)}
+    terms = [x for x in ins[0][1] if x not in out[1]]
+    order = terms + out[1]                                # the sum's indices, outermost first, then the result's
+    product = 1.0
+    for name, idx in ins:
+        aligned = np.transpose(values[name], [idx.index(x) for x in order if x in idx])
+        product = product * aligned.reshape([sizes[x] if x in idx else 1 for x in order])
+    total = np.cumsum(product.reshape((-1,) + shape(out[1])), axis=0)[-1]
+    start = rng.standard_normal(shape(out[1]))
+    S = to_tensor(at, start)
+    engine(kernel, S, *[to_tensor(at, values[name]) for name, _ in ins])
+    S.MoveFromGPU()
+    assert "sched_barrier" in engine.GetLastImplementation()
+    assert np.array_equal(S.data, total if " = " in kernel else (start + total if "+=" in kernel else start - total))
