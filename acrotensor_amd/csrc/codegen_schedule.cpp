@@ -786,6 +786,7 @@ auto Generator::LeaveThroughTile(int k) -> void
     const UVarInfo &u = uvars[s.out.uvar];
     Storage &st = stores[u.storage];
     if (!st.elementLocal || st.anyRepeated || st.members.size() != 1 || st.batchDim != 0 || !u.fixed.empty() || u.viewOffset != 0 || st.transient) return;
+    if (leftToLanes.count(u.storage) != 0) return;
     for (int j = 0; j < static_cast<int>(subs.size()); ++j)
     {
         if ((j < first || j > k) && uvars[subs[j].out.uvar].storage == u.storage) return;
@@ -1038,7 +1039,22 @@ auto Generator::OneLargeResult() const -> bool
     return written.size() == 1 && stored >= 512.0 && stored >= 3.0 * loaded;
 }
 
+// Batch entries and lanes of a workgroup, and what it keeps in LDS.  Tiles that only serve to write a group's results out in
+// whole lines are part of that choice; one that proves to cost more than it gives is given up, and the choice is made again
+// without it.
 auto Generator::ChooseBatching() -> void
+{
+    leftToLanes.clear();
+    const std::vector<Storage> before = stores;
+    for (int givenUp = ChooseBatchingAndTiles(); givenUp >= 0; givenUp = ChooseBatchingAndTiles())
+    {
+        leftToLanes.insert(givenUp);
+        stores = before;
+    }
+}
+
+// Returns the storage whose tile is to be given up, or -1.
+auto Generator::ChooseBatchingAndTiles() -> int
 {
     ComputeLdsWishes();
     bool packed = false;
@@ -1330,6 +1346,25 @@ auto Generator::ChooseBatching() -> void
     {
         ldsDoubles = PlaceLds(NB);
         if (ldsDoubles <= budgetDoubles) break;
+        // Where it is the tiles that only serve to write a group's results out that do not fit, the largest of them goes before
+        // anything that is read from LDS does.  Gradient of 12 coefficients at 11 and 12 points, 300 MB: tiles for all three
+        // results and three or four intermediates in device memory 175 and 180 us, no tiles and none or one there 141 and 144,
+        // two tiles or one and the same intermediates 120 and 135.  (Fewer entries per workgroup are the lesser evil: mass
+        // apply, 5 coefficients and 3 points, 4 entries with the tile 52, 10 without 62.)
+        int leaves = -1;
+        bool anyStaged = false;
+        for (size_t si = 0; si < stores.size() && subs.size() > 1; ++si)
+        {
+            anyStaged = anyStaged || (stores[si].staged && stores[si].inLds);
+            if (stores[si].copyOutOnly && stores[si].inLds && (leaves < 0 || stores[si].tileSize > stores[leaves].tileSize)) leaves = static_cast<int>(si);
+        }
+        if (leaves >= 0 && (anyStaged || NB == 1 || opt.force_nb > 0))
+        {
+            for (auto &st : stores) st.inLds = st.inLds && !st.copyOutOnly;
+            const bool fits = PlaceLds(NB) <= budgetDoubles;
+            if (fits) return leaves;
+            for (auto &st : stores) st.inLds = st.inLds || st.copyOutOnly;
+        }
         bool dropped = false;  // staged operands are the first to go back to device memory
         for (auto &st : stores)
         {
@@ -1348,7 +1383,7 @@ auto Generator::ChooseBatching() -> void
         int biggest = -1;
         for (size_t si = 0; si < stores.size(); ++si)
         {
-            if (stores[si].inLds && (biggest < 0 || stores[si].tileSize > stores[biggest].tileSize))
+            if (stores[si].inLds && (leaves < 0 || !stores[si].copyOutOnly) && (biggest < 0 || stores[si].tileSize > stores[biggest].tileSize))
                 biggest = static_cast<int>(si);
         }
         if (biggest < 0) break;
@@ -1506,6 +1541,7 @@ auto Generator::ChooseBatching() -> void
         st.copyOutOnly = st.wantLds = st.inLds = false;
         st.liveTo = -1;
     }
+    return -1;
 }
 
 // A kernel on its own whose tensors all have the batch index as their fastest dimension ("A_i_e = B_i_e C_i_e",

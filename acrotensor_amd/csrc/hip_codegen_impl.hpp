@@ -285,7 +285,9 @@ class Generator
     int PlaceLds(int nb);
     int PlaceLdsFromBothEnds(int nb);
     bool OneLargeResult() const;
+    std::set<int> leftToLanes;   // storages of results whose tiles ChooseBatching has given up
     void ChooseBatching();
+    int ChooseBatchingAndTiles();
     bool EntriesAreFastest() const;
     void ChooseEntriesFastest();
     static long ConflictCycles(const std::vector<long> &addr);

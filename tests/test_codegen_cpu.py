@@ -1002,3 +1002,31 @@ def test_sums_of_few_lanes_request_as_many_terms_as_the_registers_hold(TE, facto
     assert private.value == 0
     wide = TE.GetImplementation("S_i = A_n_i " + factors, at.Tensor(16385), at.Tensor(1000, 16385), *[at.Tensor(1000) if v.count("_") == 1 else at.Tensor(1000, 16385) for v in names])
     assert "sched_barrier" not in wide
+
+
+GRADIENT = ["A_e_q_j_k = B_q_i X_e_i_j_k", "G_e_q_j_k = H_q_i X_e_i_j_k", "A2_e_q_r_k = B_r_j A_e_q_j_k", "A3_e_q_r_k = H_r_j A_e_q_j_k",
+            "G2_e_q_r_k = B_r_j G_e_q_j_k", "Y0_e_q_r_s = B_s_k G2_e_q_r_k", "Y1_e_q_r_s = B_s_k A3_e_q_r_k", "Y2_e_q_r_s = H_s_k A2_e_q_r_k"]
+
+
+def gradient_source(TE, p, q, elements, transient=True):
+    calls = [[v.split("_") for v in k.replace("=", " ").split()] for k in GRADIENT]
+    shapes = {v[0]: [elements if i == "e" else q if i in "qrs" else p for i in v[1:]] for c in calls for v in c}
+    t = {n: at.Tensor(*s) for n, s in shapes.items()}
+    for n in ("A", "G", "A2", "A3", "G2"):
+        t[n].SetTransient(transient)
+    TE.BeginMultiKernelLaunch()
+    for k, c in zip(GRADIENT, calls):
+        TE(k, *[t[v[0]] for v in c])
+    return TE.EndMultiKernelLaunchGetImplementation()
+
+
+@pytest.mark.parametrize("p,q,tiles", [(12, 11, 2), (12, 12, 1), (13, 11, 2), (14, 12, 1), (9, 9, 3)])
+def test_tiles_for_results_never_push_an_intermediate_out_of_lds(monkeypatch, p, q, tiles):
+    """A group that exceeds 64 KB of LDS keeps there what it keeps without the tiles that its results leave through."""
+    def stored_intermediates():
+        src = gradient_source(at.TensorEngine("HIP"), p, q, 4000)
+        return re.findall(r"; (A|G|A2|A3|G2)->(?:lds\+)?global", src), src.count(": LDS tiles -> device memory")
+
+    chosen, copied = stored_intermediates()
+    monkeypatch.setenv("ACRO_HIP_COPY_OUT_TILE", "-1")
+    assert (chosen, copied) == (stored_intermediates()[0], tiles)

@@ -362,7 +362,7 @@ DIFFERENCE = MASS[:5] + ["V1b_e_i_r_s = H_q_i U_e_q_r_s", MASS[5], "V2b_e_i_j_s 
 
 @pytest.mark.parametrize("kernels,p,q,elements,copied", [
     (MASS, 7, 8, 389, "Y"), (MASS, 8, 9, 257, "Y"), (MASS, 3, 4, 4857, "Y"), (MASS, 3, 4, 4854, ""), (MASS, 6, 6, 607, "Y"),
-    (GRADIENT, 3, 4, 2051, "Y0 Y1 Y2"), (GRADIENT, 7, 9, 191, "Y0 Y1 Y2"), (GRADIENT, 2, 3, 4901, "Y0 Y1 Y2"), (GRADIENT, 4, 6, 501, "Y2"),
+    (GRADIENT, 3, 4, 2051, "Y0 Y1 Y2"), (GRADIENT, 7, 9, 191, "Y0 Y1 Y2"), (GRADIENT, 2, 3, 4901, "Y0 Y1 Y2"), (GRADIENT, 4, 6, 501, "Y2"), (GRADIENT, 12, 11, 101, "Y1 Y2"),
     (DIFFERENCE, 7, 8, 389, "Y"), (DIFFERENCE, 8, 9, 257, "Y"), (DIFFERENCE, 7, 8, 380, "")])
 def test_results_of_a_chain_in_whole_lines(at, monkeypatch, kernels, p, q, elements, copied):
     """Results of 1 MB and more leave through LDS tiles also in long runs per lane, when their terms were summed in registers
