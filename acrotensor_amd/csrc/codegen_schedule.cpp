@@ -1530,16 +1530,14 @@ auto Generator::ChooseBatchingAndTiles() -> int
             for (size_t si = 0; si < stores.size(); ++si) stores[si].ldsOffset = before[si];
     }
 
-    // A result accumulated in registers leaves from there after all where few workgroups are resident: nothing hides the
-    // second pass.  Diffusion apply on 2^25 points by the lanes / through the tile: p = 7, 10^3 points (53 KB of LDS, three
+    // A result accumulated in registers leaves from there where few workgroups are resident: nothing hides the second pass.
+    // Diffusion apply on 2^25 points by the lanes / through the tile: p = 7, 10^3 points (53 KB of LDS with it, three
     // workgroups) 480 / 515 us, p = 6, 10^3 (49 KB) 466 / 473, p = 8, 10^3 (48 KB) 538 / 535, 11^3 848 / 873, but 9^3 (35 KB)
     // p = 7 502 / 478, p = 8 562 / 548.
     for (const auto &s : subs)
     {
-        Storage &st = stores[uvars[s.out.uvar].storage];
-        if (!s.forwardedOld || !st.copyOutOnly || static_cast<long>(ldsDoubles) * 8 <= 40 * 1024) continue;
-        st.copyOutOnly = st.wantLds = st.inLds = false;
-        st.liveTo = -1;
+        const int result = uvars[s.out.uvar].storage;
+        if (s.forwardedOld && stores[result].copyOutOnly && static_cast<long>(ldsDoubles) * 8 > 40 * 1024) return result;
     }
     return -1;
 }

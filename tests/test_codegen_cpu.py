@@ -1030,3 +1030,12 @@ def test_tiles_for_results_never_push_an_intermediate_out_of_lds(monkeypatch, p,
     chosen, copied = stored_intermediates()
     monkeypatch.setenv("ACRO_HIP_COPY_OUT_TILE", "-1")
     assert (chosen, copied) == (stored_intermediates()[0], tiles)
+
+
+@pytest.mark.parametrize("p,q", [(11, 14), (11, 13), (7, 10), (10, 9)])
+def test_a_tile_given_up_for_an_accumulated_result_leaves_nothing_behind(monkeypatch, p, q):
+    """Above 40 KB of LDS the result leaves by the lanes, from the workgroup that a group without the tile has."""
+    wl = workloads.config5(E=2 ** 17 // (p + 1) ** 3 + 1, Q=q, P=p + 1)      # (1 MB of results: from there on the tile is considered)
+    chosen = chain_source(at.TensorEngine("HIP"), wl, transient=True)
+    monkeypatch.setenv("ACRO_HIP_COPY_OUT_TILE", "-1")
+    assert chosen == chain_source(at.TensorEngine("HIP"), wl, transient=True)
