@@ -798,6 +798,17 @@ auto Generator::LeaveThroughTile(int k) -> void
     // Launches of less than 1 MB of this result keep what the rules for a few workgroups give them: the barrier and the
     // second pass are in the open there.
     const bool large = group && E * st.tileSize >= (1L << 17);
+    bool storedBetween = false;
+    for (const auto &q : subs)
+    {
+        for (const auto &r : q.in) storedBetween = storedBetween || (stores[uvars[r.uvar].storage].written && !stores[uvars[r.uvar].storage].transient && !uvars[r.uvar].isVirtual);
+    }
+    // Nor do results before the last where intermediates are stored through tiles of their own and a workgroup's few entries
+    // of this result are no whole 64-byte pieces: with the LDS of the additional tiles there are fewer still, and every
+    // range's ends cost a piece.  Three gradient components with every intermediate stored, 200 MB, us, one tile / three:
+    // 3 coefficients, 5 points 40.3 / 48.4, 5, 7 39.0 / 49.2, 6, 7 40.0 / 43.9, 7, 9 41.9 / 49.0, 9, 11 42.7 / 45.4; whole
+    // pieces, 4, 6 42.3 / 34.6, 6, 8 46.3 / 33.6, 7, 8 48.0 / 33.9 (without any tile); 16 entries of 27: 38.3 / 34.2.
+    if (storedBetween && k + 1 != static_cast<int>(subs.size()) && st.tileSize % 8 != 0 && st.tileSize >= 64) return;
     if (!large && (k + 1 != static_cast<int>(subs.size()) || first != k)) return;
     // Results in planes ("D_e_m_n_k1_k2_k3" with the lanes along k and the tile (m, n)) whose length is no multiple of 64
     // bytes: a wavefront's stores start anywhere in a line, and a streaming store of part of a 64-byte piece costs as much as
@@ -841,11 +852,6 @@ auto Generator::LeaveThroughTile(int k) -> void
     // last kernel's result, 3^3 points 121 -> 61, 7^3 132 -> 72, 9^3 142 -> 80, 10^3 134 -> 87.
     // (45 % where intermediates are stored as well, which leave through their own tiles: p = 3, 5^3 points 80.4 against 81.1)
     const bool lowCoverage = !large || st.tileSize < 24 || first != k;
-    bool storedBetween = false;
-    for (const auto &q : subs)
-    {
-        for (const auto &r : q.in) storedBetween = storedBetween || (stores[uvars[r.uvar].storage].written && !stores[uvars[r.uvar].storage].transient && !uvars[r.uvar].isVirtual);
-    }
     if ((large || run < std::max<long>(longRun, 8)) && envInt("ACRO_HIP_COPY_OUT_TILE") < 2)
     {
         const int entries = static_cast<int>(std::max<long>(1, 64 / std::max<long>(1, s.laneCount)));

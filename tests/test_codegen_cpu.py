@@ -1039,3 +1039,13 @@ def test_a_tile_given_up_for_an_accumulated_result_leaves_nothing_behind(monkeyp
     chosen = chain_source(at.TensorEngine("HIP"), wl, transient=True)
     monkeypatch.setenv("ACRO_HIP_COPY_OUT_TILE", "-1")
     assert chosen == chain_source(at.TensorEngine("HIP"), wl, transient=True)
+
+
+@pytest.mark.parametrize("p,q,results", [(2, 3, 3), (3, 4, 3), (3, 5, 1), (5, 7, 1), (4, 6, 3), (8, 9, 1), (7, 8, 3)])
+def test_results_before_the_last_share_tiles_with_stored_intermediates_in_whole_pieces_only(TE, p, q, results):
+    """Intermediates that are stored leave through tiles of their own; without them every result has one."""
+    def copied(transient):
+        src = gradient_source(TE, p, q, 30000, transient)
+        return sum("// Y%d: LDS tiles -> device memory" % n in src for n in range(3))
+
+    assert copied(False) == results and copied(True) == 3
