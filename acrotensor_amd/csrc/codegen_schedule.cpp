@@ -799,6 +799,11 @@ auto Generator::LeaveThroughTile(int k) -> void
     // second pass are in the open there.
     const bool large = group && E * st.tileSize >= (1L << 17);
     bool storedBetween = false;
+    double results = 0.0;   // doubles that the launch writes
+    for (const auto &other : stores)
+    {
+        if (other.written && !other.transient && !uvars[other.members[0]].isVirtual) results += static_cast<double>(E) * other.tileSize;
+    }
     for (const auto &q : subs)
     {
         for (const auto &r : q.in) storedBetween = storedBetween || (stores[uvars[r.uvar].storage].written && !stores[uvars[r.uvar].storage].transient && !uvars[r.uvar].isVirtual);
@@ -850,13 +855,16 @@ auto Generator::LeaveThroughTile(int k) -> void
     // 96 -> 84; interpolation as a chain to 8^3 points 102 -> 57, 10^3 99 -> 65, 11^3 117 -> 70; diffusion apply on 2^25
     // points, accumulated in registers, p = 7, 8^3 530 -> 505.  The three components of a gradient, of which two are not the
     // last kernel's result, 3^3 points 121 -> 61, 7^3 132 -> 72, 9^3 142 -> 80, 10^3 134 -> 87.
-    // (45 % where intermediates are stored as well, which leave through their own tiles: p = 3, 5^3 points 80.4 against 81.1)
+    // Where intermediates are stored as well, through tiles of their own, the same up to 320 MB of results, and from 45 % on
+    // beyond: mass apply with every intermediate stored, runs of three and four, 60 % against 45 %, tensors changing, 3^3 to
+    // 6^3 points: 0.84 to 0.98 of the time at 90 MB in all, 0.90 to 0.98 at 200 MB, 0.98 to 1.00 at 330 to 390 MB, but 0.95 to
+    // 1.02 at 450 MB and 0.98 to 1.04 at 1 GB (p = 3, 5^3 points, 65 537 elements 81.1 against 80.4).
     const bool lowCoverage = !large || st.tileSize < 24 || first != k;
     if ((large || run < std::max<long>(longRun, 8)) && envInt("ACRO_HIP_COPY_OUT_TILE") < 2)
     {
         const int entries = static_cast<int>(std::max<long>(1, 64 / std::max<long>(1, s.laneCount)));
         const double coverage = WaveStoreLineCoverage(k, entries);
-        scattered = oddPlanes || (s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", lowCoverage ? 30 : (storedBetween ? 45 : 60)) ||
+        scattered = oddPlanes || (s.laneCount >= 2 && (coverage < 0.01 * envInt("ACRO_HIP_COPY_OUT_COVERAGE", lowCoverage ? 30 : (storedBetween && results > 40.0 * 1024 * 1024 ? 45 : 60)) ||
                                          (coverage < 0.95 && envInt("ACRO_HIP_COPY_OUT_WRITERS") >= 0 && WritesDominate())));
     }
     if (subs.size() != 1 && !scattered) return;

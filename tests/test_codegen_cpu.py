@@ -1049,3 +1049,18 @@ def test_results_before_the_last_share_tiles_with_stored_intermediates_in_whole_
         return sum("// Y%d: LDS tiles -> device memory" % n in src for n in range(3))
 
     assert copied(False) == results and copied(True) == 3
+
+
+@pytest.mark.parametrize("transient", [False, True])
+def test_last_result_of_a_stored_chain_leaves_through_a_tile_up_to_320_mb(TE, transient):
+    """p = 3, 5^3 points: runs of four doubles; 674 doubles per element with every intermediate stored."""
+    line = 40 * 2 ** 20 // 674
+    for elements in (2049, line, line + 1):
+        wl = workloads.config4(E=1, Q=5, P=4)
+        t = {n: at.Tensor(*(a.shape if n == "B" else (elements,) + a.shape[1:])) for n, a in wl.arrays.items()}
+        for n in wl.transient:
+            t[n].SetTransient(transient)
+        TE.BeginMultiKernelLaunch()
+        for k, out, ins in wl.kernels:
+            TE(k, t[out], *[t[n] for n in ins])
+        assert ("// Y: LDS tiles -> device memory" in TE.EndMultiKernelLaunchGetImplementation()) == (transient or elements <= line)
