@@ -4,6 +4,7 @@ The library is built in-tree by ``acrotensor_amd.build.build_library`` (hipcc, g
 it is missing: there is no host fallback for any operation.
 """
 import ctypes
+import functools
 import importlib.machinery
 import importlib.util
 import os
@@ -95,12 +96,14 @@ def _contract_through_ctypes(engine, kernel, out, inputs):
     return load().acro_engine_contract(engine, kernel.encode(), out._address, arr, len(inputs))
 
 
-def _call_module():
-    """csrc/python_call.cpp, or None where the library was built without this interpreter's headers at hand."""
+@functools.lru_cache(maxsize=None)
+def _call_module(path):
+    """csrc/python_call.cpp, or None where the library was built without this interpreter's headers at hand.  Loaded once, not
+    for every engine (12 us each)."""
     load()
-    if not os.path.exists(CALL_PATH):
+    if not os.path.exists(path):
         return None
-    loader = importlib.machinery.ExtensionFileLoader("_acro_call", CALL_PATH)
+    loader = importlib.machinery.ExtensionFileLoader("_acro_call", path)
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_acro_call", loader))
     loader.exec_module(module)
     return module
@@ -111,7 +114,7 @@ def contract_function():
     of acrotensor_amd.api, without ctypes between where that is built."""
     global _contract
     if _contract is None:
-        module = _call_module()
+        module = _call_module(CALL_PATH)
         _contract = module.contract if module else _contract_through_ctypes
     return _contract
 
@@ -119,7 +122,7 @@ def contract_function():
 def capture_functions():
     """``begin(engine address) -> status`` and ``end(engine address) -> status``: the entry points around a multi-kernel
     launch, likewise."""
-    module = _call_module()
+    module = _call_module(CALL_PATH)
     lib = load()
     return (module.begin, module.end) if module else (lib.acro_engine_begin_multi_kernel_launch, lib.acro_engine_end_multi_kernel_launch)
 

@@ -130,6 +130,13 @@ def test_engine_calls_do_without_the_extension_module(monkeypatch):
         te("S_i = A_i B_i", S, A, B)
 
 
+def test_engines_look_their_call_functions_up_once(monkeypatch):
+    at.TensorEngine("HIP")
+    monkeypatch.setattr(importlib.machinery, "ExtensionFileLoader", None)      # (a second look-up would fail)
+    first, second = at.TensorEngine("HIP"), at.TensorEngine("HIP")
+    assert (first._contract, first._begin, first._end) == (second._contract, second._begin, second._end)
+
+
 def test_the_library_builds_without_a_python_installation():
     csrc = os.path.join(os.path.dirname(_capi.__file__), "csrc")
 
