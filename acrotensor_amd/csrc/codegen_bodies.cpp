@@ -484,7 +484,8 @@ auto Generator::GlobalStore(int k, const std::string &gaddr, const std::string &
 auto Generator::NeedsLdsCopy(int k) const -> bool
 {
     const Storage &st = StoreOf(subs[k].out.uvar);
-    return st.inLds && (st.liveTo > k || (st.copyOutOnly && StoresToGlobal(k)));
+    // (of a result whose terms are summed in registers only the last kernel's values leave through the tile)
+    return st.inLds && (st.copyOutOnly ? StoresToGlobal(k) : st.liveTo > k);
 }
 
 // A result that must reach device memory AND stays in LDS for a later kernel is written to device memory from

@@ -1064,3 +1064,10 @@ def test_last_result_of_a_stored_chain_leaves_through_a_tile_up_to_320_mb(TE, tr
         for k, out, ins in wl.kernels:
             TE(k, t[out], *[t[n] for n in ins])
         assert ("// Y: LDS tiles -> device memory" in TE.EndMultiKernelLaunchGetImplementation()) == (transient or elements <= line)
+
+
+def test_partial_sums_of_an_accumulated_result_stay_in_registers(TE):
+    """Its last kernel alone writes the tile that the result leaves through."""
+    src = chain_source(TE, workloads.config5(E=190, Q=9, P=9), transient=True)
+    assert "// Y: LDS tiles -> device memory" in src
+    assert re.findall(r"\] Y_e_i_j_k .*; Y->(\S*)", src) == ["", "", "lds+global"]
