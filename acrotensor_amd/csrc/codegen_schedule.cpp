@@ -1191,46 +1191,7 @@ auto Generator::ChooseBatchingAndTiles() -> int
         // wavefronts (p=2 mass assembly).  Groups that batch anyway take the better packing (p=1 mass apply:
         // 8 -> 14 entries per workgroup, 62.9 -> 74.9 % of the HBM peak; p=4: 2 -> 5 entries in 256 lanes,
         // 67.5 -> 72.0 %), and so do groups whose wavefronts would be mostly idle.
-        // Groups of parallel chains (phases of several kernels, "chains") can take other shapes as well: two entries where the
-        // chains fill about half of their wavefronts (from four workgroups per compute unit on), and workgroups of three
-        // wavefronts where a phase is three (or six of which the second pass is short and none is narrower than two), none
-        // is nearly full and the first and last kernel are no wider than the chains between them.  Only on request
-        // (ACRO_HIP_PACK_CHAINS=1): one entry in 256 lanes is as fast or faster since the first phase's loads no longer
-        // cost registers throughout (see the prefetch; diffusion apply on 2^22 points, us, these shapes / one entry in 256:
-        // p = 4, 6^3 64.2 / 60.3, p = 5, 6^3 / 7^3 66.1 / 67.9 and 62.8 / 61.3, p = 6, 7^3 69.0 / 67.9, p = 8, 9^3 84.0 / 76.1).
-        double chainItems = 0.0, chainLanes = 0.0;
-        long mostWaves = 0, leastWaves = 64, chainWidth = 1, endWidth = 1;   // (widths: lanes of the widest kernel)
-        for (int ph = 0; ph <= subs.back().phase; ++ph)
-        {
-            long kernelsHere = 0, waves = 0, widest = 0;
-            double items = 0.0, lanes = 0.0;
-            for (const auto &s : subs)
-            {
-                if (s.phase != ph || s.fusedWithPrev) continue;
-                const double weight = static_cast<double>(std::max<long>(1, s.tileCount * s.contrCount));
-                if (ph == 0 || ph == subs.back().phase) endWidth = std::max<long>(endWidth, s.laneCount);
-                widest = std::max<long>(widest, s.laneCount);
-                ++kernelsHere;
-                waves += (s.laneCount + 63) / 64;
-                items += weight * s.laneCount;
-                lanes += weight * 64.0 * ((s.laneCount + 63) / 64);
-            }
-            if (kernelsHere > 0) leastWaves = std::min(leastWaves, waves);
-            if (kernelsHere < 3) continue;
-            chainItems += items;
-            chainLanes += lanes;
-            mostWaves = std::max(mostWaves, waves);
-            chainWidth = std::max(chainWidth, widest);
-        }
-        const bool chains = chainLanes > 0.0 && envInt("ACRO_HIP_PACK_CHAINS") > 0;
-        const double chainFill = chains ? chainItems / chainLanes : 1.0;
-        auto ldsOfOneEntry = [&] {
-            const int firstFit = PlaceLds(1), bothEnds = PlaceLdsFromBothEnds(1);
-            return bothEnds > 0 ? std::min(firstFit, bothEnds) : firstFit;
-        };
-        const bool threeWide = mostWaves == 3 || (mostWaves == 6 && leastWaves >= 2 && chainFill < 0.68 && ldsOfOneEntry() <= 160 * 1024 / 8 / 4);
-        if (chains && NB == 1 && NT == 256 && threeWide && 5 * endWidth <= 6 * chainWidth && chainFill >= 0.54 && chainFill < 0.85) NT = bestNT = 192;
-        const bool wanted = envInt("ACRO_HIP_PACK") > 0 || (envInt("ACRO_HIP_PACK") == 0 && NT != 192 && (NB > 1 || idle < 0.5 || (chainFill < 0.54 && E >= 1024)));
+        const bool wanted = envInt("ACRO_HIP_PACK") > 0 || (envInt("ACRO_HIP_PACK") == 0 && (NB > 1 || idle < 0.5));
         // (not one large result per entry and little else to move: its workgroups stream out best with few entries, whatever
         // their lanes do.  p = 2 mass assembly with 3^3 points, 46 028 elements, us: 3 entries in 256 lanes 62.6, one, which
         // the rule for such streams below makes two in 512, 46.5)

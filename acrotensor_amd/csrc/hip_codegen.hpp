@@ -55,8 +55,6 @@
 //   ACRO_HIP_LDS_PAD=1|2        pad LDS tile strides against bank conflicts (2: even if a resident workgroup is lost)
 //   ACRO_HIP_PACK=1|-1          1: pick batch / workgroup size for wavefront utilisation also when one batch entry per
 //                               workgroup would do; -1: never (default: only for groups that batch several entries)
-//   ACRO_HIP_PACK_CHAINS=1|-1   groups of parallel chains: batch and workgroup size of their own / chosen as for other groups
-//                               (default: their own with run-time compilers before ROCm 7.2)
 //   ACRO_HIP_INTERLEAVE_TILE=-1|<n>  transposed stages sum the outputs of a tile one after the other / term by term from operators
 //                               of n entries on (default 64, from 9 outputs in the tile on, 10 for a kernel on its own)
 //   ACRO_HIP_PERSIST=<n>        persistent grid of n workgroups per CU looping over the batch

@@ -99,11 +99,9 @@ def test_config5_diffusion_apply(at, engine, checker, E, Q, P, transient):
 
 @pytest.mark.parametrize("E,Q,P", [(3, 6, 5), (1025, 6, 5), (2, 7, 6), (5, 6, 6), (3, 7, 7), (3, 9, 9), (2, 10, 9), (7, 9, 9)])
 @pytest.mark.parametrize("transient", [False, True])
-def test_diffusion_apply_with_three_wavefronts_or_two_entries_per_workgroup(at, checker, monkeypatch, E, Q, P, transient):
-    # chains that fill about half of their wavefronts (two entries from 1 024 on), three wavefronts per phase, phases of six wavefronts in
-    # two passes, operators of more than 64 entries applied transposed a row at a time
-    monkeypatch.setenv("ACRO_HIP_PACK_CHAINS", "1")        # (the default with run-time compilers before ROCm 7.2)
-    test_config5_diffusion_apply(at, at.TensorEngine("HIP"), checker, E, Q, P, transient)
+def test_diffusion_apply_in_partly_filled_wavefronts(at, engine, checker, E, Q, P, transient):
+    # chains of half a wavefront, of three and of six, and operators of more than 64 entries applied transposed a row at a time
+    test_config5_diffusion_apply(at, engine, checker, E, Q, P, transient)
 
 
 @pytest.mark.parametrize("E,Q,P,transient", [(11, 9, 9, True), (10, 10, 9, False), (9, 8, 8, True)])
