@@ -571,7 +571,7 @@ static auto ReadAgainFromCache(long resultDoubles, long rows) -> bool
 // doubles of a 16-byte load the operands of two successive steps.  MI355X's vector and matrix FP64 peaks are the
 // same; what the matrix cores save is operand delivery: no scalar loads and 1/16 of the LDS reads.
 // 64 x 64 on 2^18 entries: 47 - 51 us against 79 us with scalar loads (512 workgroups; 58 us with 1 024, 76 us
-// with 2 048; loading the next 16 entries ahead of the arithmetic made no difference).
+// with 2 048; with the next 16 entries requested ahead, below, 51.5 -> 59).
 // With `next` (and its kernel `nextSub`) the result of this operator never leaves the chip: it is scaled, written
 // to a per-wavefront piece of LDS in the result layout (entry 4r + lane / 16, output lane % 16), read back in the
 // operand layout (entry lane % 16, term group lane / 16) and multiplied by the second operator.
@@ -598,12 +598,18 @@ auto Generator::EmitOperatorMatrixCores(HipKernelPlan &plan, const OperatorShape
     // out as one contiguous range.
     // (all 16 entries at once where LDS allows, else 8 or 4 at a time)
     int stageRounds = 0;
-    // Operators that fill most of LDS run one wavefront per SIMD, whose matrix instructions wait for each trip's vectors:
-    // those of the next trip are requested before this trip's arithmetic (behind the last trip its own again, so that the
-    // request is unconditional).  Us, before -> after: 125 x 64 on 30 000 entries with the transposed product behind it
-    // 35.4 -> 34.3, on 131 072 101.0 -> 99.0; 128 x 64 34.2 -> 32.7 and 98.1 -> 95.8, alone on 262 143 83.5 -> 79; 100 x 64
-    // on 30 000 31.2 -> 29.7.  Smaller operators keep more wavefronts: 72 x 64 35.5 -> 37.7; odd rows of a result too large
-    // for the memory-side cache wait for its streaming stores: 110 x 60 on 262 143 75.2 -> 82, 90 x 80 89 -> 94.5.
+    // Operators of more than 4096 entries run one wavefront per SIMD, whose matrix instructions wait for each trip's
+    // vectors: those of the next trip are requested before this trip's arithmetic (behind the last trip its own again, so
+    // that the request is unconditional).  Us, before -> after: 125 x 64 on 30 000 entries with the transposed product
+    // behind it 35.4 -> 34.3, on 131 072 101.0 -> 99.0; 128 x 64 34.2 -> 32.7 and 98.1 -> 95.8, alone on 262 143 83.5 -> 79;
+    // 100 x 64 on 30 000 31.2 -> 29.7.  The line is an empirical one: from it on the request pays or costs nothing to speak
+    // of, below it small batches gain and large ones lose, on as many wavefronts: with the transposed product on 30 000 |
+    // 131 072 entries 72 x 64 25.0 -> 23.3 | 64.3 -> 66.8, 96 x 64 27.1 -> 25.6 | 72.8 -> 76.7; alone on 131 072 64 x 64
+    // 28.7 -> 30.0, 72 x 64 35.8 -> 37.6, 80 x 80 38.0 -> 39.6 (112 x 64, above it, 42.1 -> 42.4, with the transposed
+    // product 85.1 -> 84.3).  Odd rows of a result beyond the memory-side cache lose where 16 does not divide the entries as
+    // well, and gain or lose where it does: 110 x 60 on 262 143 75.1 -> 81.9, 90 x 80 88.6 -> 93.6, 125 x 64 85.9 -> 86.6;
+    // 125 x 64 on 262 144 84.5 -> 81.8, on 500 000 165 -> 171, 110 x 60 on 200 000 68.5 -> 65.1.  (The compiled loop waits
+    // at the head of a trip for everything in flight, the stores that the trip before issued behind the request included.)
     const bool ahead = !next && pairs && shape.comp == 1 && s.op == '=' && nIp * nJp >= 7168 &&
                        (nI % 8 == 0 || E * nAll <= kCachedResultTo) && shape.perElement.empty() && shape.perColumn.empty() &&
                        envInt("ACRO_HIP_OPERATOR_AHEAD") >= 0;

@@ -855,6 +855,10 @@ auto Generator::LeaveThroughTile(int k) -> void
     // 96 -> 84; interpolation as a chain to 8^3 points 102 -> 57, 10^3 99 -> 65, 11^3 117 -> 70; diffusion apply on 2^25
     // points, accumulated in registers, p = 7, 8^3 530 -> 505.  The three components of a gradient, of which two are not the
     // last kernel's result, 3^3 points 121 -> 61, 7^3 132 -> 72, 9^3 142 -> 80, 10^3 134 -> 87.
+    // Fewer points than coefficients, where the tile is LDS that the chain would not hold: coefficients, points, 300 MB, mass
+    // apply 5, 3 61.8 -> 52.5, 7, 5 64.5 -> 52.9, 8, 5 64.8 -> 48.2, 9, 6 78.6 -> 52.7, 12, 9 71.0 -> 59.3 (4, 3 47.8 -> 47.4 the
+    // least of 19); back from 6, 8, 9 points to 8, 10, 12 80 -> 48, 78 -> 52, 87 -> 54; diffusion apply 7, 4 62.5 -> 59.3, 9, 6
+    // 63.4 -> 58.3, 8, 7 56.5 -> 52.6, 7, 5 and 9, 7 the same, 10, 7 63.6 -> 64.9, and one shape that loses, 8, 6 56.3 -> 60.1.
     // Where intermediates are stored as well, through tiles of their own, the same up to 320 MB of results, and from 45 % on
     // beyond: mass apply with every intermediate stored, runs of three and four, 60 % against 45 %, tensors changing, 3^3 to
     // 6^3 points: 0.84 to 0.98 of the time at 90 MB in all, 0.90 to 0.98 at 200 MB, 0.98 to 1.00 at 330 to 390 MB, but 0.95 to

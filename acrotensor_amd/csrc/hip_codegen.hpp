@@ -72,13 +72,15 @@
 //   ACRO_HIP_COLLAPSE=-1        offsets are sums over every lane index (runs of lane indices that an operand lays out in
 //                               the lanes' own order are not collapsed into one multiple of the item number)
 //   ACRO_HIP_WRITE_BATCH=-1     write-heavy launches whose results leave through LDS tiles keep their batch size
-//                               (default: twice the batch entries in workgroups of 512 lanes)
+//                               (default: twice the batch entries in workgroups of 512 lanes; three results and more: a power
+//                               of two up to 16)
 //   ACRO_HIP_OPERATOR_COMPONENTS=-1  operators applied to vectors with trailing component indices ("A_e_i_k = B_i_j X_e_j_k")
 //                               run through the generic schedule, not on the matrix cores
 //   ACRO_HIP_COPY_OUT_TILE=-1|2 -1: results are always stored by the lanes that computed them; 2: an LDS tile that the workgroup
 //                               writes out in whole lines only for a kernel on its own whose lanes each hold a long run of outputs
-//                               (default: also for the last kernel of any group whose store instructions would fill less than
-//                               30 % of the lines they touch).  ACRO_HIP_COPY_OUT_MAX=<doubles per batch entry> (default 2048)
+//                               (default: also for results of groups whose store instructions would fill less than 30 % of the
+//                               lines they touch, 60 % from 1 MB of the result on; ACRO_HIP_COPY_OUT_COVERAGE=<percent>).
+//                               ACRO_HIP_COPY_OUT_MAX=<doubles per batch entry> (default 2048)
 //   ACRO_HIP_OPERATOR_ODD_ROWS=-1  operators in blocks of rows: results of 26 to 144 MiB in rows that are no multiple of 64 bytes
 //                               keep the streaming hint on their stores, too
 //   ACRO_HIP_COPY_OUT_PLANES=-1 results in planes whose length is no multiple of 64 bytes are stored by the lanes that computed them
@@ -115,6 +117,7 @@
 //   ACRO_HIP_OPERATOR_COMPONENTS=2  vectors with components: always entries (entry, component), never the components of an entry together
 //   ACRO_HIP_OPERATOR_BLOCKS=-1 operators of more than 4 096 entries are not applied in blocks of rows (generic schedule instead)
 //   ACRO_HIP_OPERATOR_STAGE_OUT=-1  results of operators whose rows 16 does not divide are stored by the lanes that hold them
+//   ACRO_HIP_OPERATOR_AHEAD=-1  operators that fill LDS never request the next trip's vectors ahead
 //   ACRO_HIP_OPERATOR_FOLD=-1   a pointwise kernel that rescales an operator kernel's transient result is not folded into it
 //   ACRO_HIP_OPERATOR_PAIR=-1   two operator-shaped kernels with a transient intermediate are not joined into one matrix-core kernel
 //   ACRO_HIP_OPERATOR_SEQUENCE=-1  groups of several large operator-shaped kernels run as one fused chain kernel instead of one
